@@ -30,9 +30,9 @@ _libs: dict[str, ctypes.CDLL] = {}
 
 
 def build(ref: bool = False) -> None:
-    """Compile liboracle.so (and _ref/ when ``ref`` and the reference exists)."""
+    """Compile liboracle.so (and _ref/ when ``ref`` and the reference's sources exist)."""
     subprocess.run(["make", "-s", "-C", _HERE], check=True)
-    if ref and os.path.isdir("/root/reference"):
+    if ref and os.path.isfile("/root/reference/src/backend/backend_naive.cc"):
         subprocess.run(["make", "-s", "-C", _HERE, "ref"], check=True)
 
 
