@@ -1,0 +1,448 @@
+// Causal attention of several queries (the prompt, or a piece of it against
+// the cache; backend_naive.cc:344-378) on the matrix cores.  The one-query
+// decode forms and the general kernel are in model_kernels.hip.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <cmath>
+#include <type_traits>
+
+#include "common.h"
+#include "device.h"
+
+namespace vvh {
+
+namespace {
+
+typedef _Float16 h4v __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ h4v lds_read_tr16(const f16* p)
+{
+    typedef short s4v __attribute__((ext_vector_type(4)));
+    const s4v v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s4v*)(p));
+    return __builtin_bit_cast(h4v, v);
+}
+
+// LDS slot of 16-byte chunk c of row r in a tile of D-wide fp16 rows.  Two
+// kinds of reads meet no bank twice: 16 consecutive rows of one chunk (the K
+// operand), and 4 consecutive rows of 4 consecutive chunks (the transposed V
+// operand, whose rows must fall in different 64-byte groups).
+template <int D>
+__device__ __forceinline__ int attn_swz(int r)
+{
+    return D == 128 ? ((r & 3) << 2) | ((r >> 2) & 3) : (((r >> 1) & 1) << 2) | ((r >> 2) & 3);
+}
+
+// One row of the general kernel's arithmetic in one wave: scores, maximum,
+// exponentials and sum over the `len` visible keys only.  For rows whose
+// result from the tiles is not finite: a key past a row's last visible one
+// has weight 0 in the tiles, and 0 times an infinity or NaN of its V row
+// would reach the sums.
+template <int D>
+__device__ void attn_row_general(const f16* __restrict__ qr, const f16* __restrict__ kh, const f16* __restrict__ vh,
+                                 int64_t kvs, int len, float scale, f16* __restrict__ orow, int lane)
+{
+    constexpr int E = D / 64;
+    float qv[E], o[E];
+#pragma unroll
+    for (int e = 0; e < E; e++) {
+        qv[e] = (float)qr[lane * E + e];
+        o[e] = 0.0f;
+    }
+    auto score = [&](int t) {
+        float d = 0.0f;
+#pragma unroll
+        for (int e = 0; e < E; e++) d += qv[e] * (float)kh[t * kvs + lane * E + e];
+        return wave_sum_xor(d) * scale;
+    };
+    float mx = -INFINITY, sum = 0.0f;
+    for (int t = 0; t < len; t++) mx = fmaxf(mx, score(t));
+    for (int t = 0; t < len; t++) sum += expf(score(t) - mx);
+    for (int t = 0; t < len; t++) {
+        const float p = expf(score(t) - mx) / sum;
+#pragma unroll
+        for (int e = 0; e < E; e++) o[e] += p * (float)vh[t * kvs + lane * E + e];
+    }
+#pragma unroll
+    for (int e = 0; e < E; e++) orow[lane * E + e] = (f16)o[e];
+}
+
+}  // namespace
+
+// ---------------------------------------------------------------------------
+// fp16 q, K and V, head_dim 64 or 128.  The G = H / KVH query heads of a kv
+// head read the same keys, so the rows of a kv head's problem are the pairs
+// (query s, head h of the group), row r = s G + h: a tile of consecutive rows
+// covers few queries, which keeps its causal edge short, and a call of a few
+// queries still fills tiles.
+//
+// A block of 4 RG waves takes 32 RG rows; wave (rg, kg) takes rows 32 rg .. + 31
+// and, of every stage of 128 keys, the 32 keys of group kg.  K and V stages go
+// straight from memory to LDS, two stages deep, one barrier per stage.  Per
+// stage a wave:
+//   S^T = K q^T    v_mfma_f32_32x32x16_f16, A = K rows, B = the 32 query rows
+//                  (kept in registers): lane l gets row l % 32's scores of 16
+//                  keys, 8 (i / 4) + 4 (l / 32) + i % 4 for i < 16;
+//   softmax        p = exp2(score scale log2 e - m), m the row's running
+//                  maximum in log2 units, moved (and O, l rescaled) only when
+//                  a score exceeds it by more than 8: p stays below 2^8;
+//   O^T += V^T p   A = V^T by LDS transpose reads, B = the lane's own p: the
+//                  order of keys inside an MFMA is free as long as A and B
+//                  share it, so p needs no shuffles.  p goes in as fp16 high
+//                  and low parts (two products), about 22 bits.
+// The groups' (m, l, O) are merged through LDS at the end; blocks that share a
+// row block's keys (gridDim.y of them) leave theirs to k_attention_prefill_merge.
+//
+// A stage costs about 3400 clocks with one wave per SIMD or two (8 waves): the
+// chain of a wave's products, softmax and products (24 MFMAs of 32 clocks and
+// about 190 vector operations at head_dim 128), not the loads (the same with
+// them left out).  Measured against one block per (head, query) with the dot
+// products on the vector unit (k_attention): 512 queries, 14 heads on 2 of 64,
+// 78 -> 7.7 us; 2048, 12 on 2 of 128, 1740 -> 34; 500 after 3500 positions, 1840
+// -> 34.  Two 32-key tiles per wave and stage (half as many stages of twice the
+// length), 128 rows per block, and the next stage's scores computed during
+// this one's softmax all measured the same or slower.
+// ---------------------------------------------------------------------------
+template <int D, int RG>
+__global__ __launch_bounds__(256 * RG) void k_attention_prefill(
+    const f16* __restrict__ q, const f16* __restrict__ k, const f16* __restrict__ v, int32_t n_q, int32_t len0,
+    int32_t KVH, int32_t G, float scale, float scale_log2, f16* __restrict__ out, float* __restrict__ ws)
+{
+    constexpr int KG = 4;  // key groups
+    constexpr int NW = RG * KG, NT = 64 * NW, ROWS = 32 * RG;
+    constexpr int KS = 32 * KG;           // keys per stage
+    constexpr int CPR = D / 8;            // 16-byte chunks per row
+    constexpr int RPP = 64 / CPR;         // rows per 1 KB load
+    constexpr int LP = KS / RPP / NW;     // loads of K (and of V) per wave and stage
+    constexpr int DT = D / 16, DE = D / 32;
+    static_assert(KS / RPP % NW == 0, "whole loads per wave");
+    constexpr int kStage = 2 * KS * D;    // halves: K rows, then V rows
+    static_assert(kStage * 2 >= NW / 2 * 32 * D * 4, "half of the waves' O in each stage");
+    __shared__ __align__(1024) f16 sm0[kStage], sm1[kStage];
+    __shared__ float wm[NW][32], wl[NW][32];
+    __shared__ int32_t bad[ROWS];
+
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int rg = wave % RG, kg = wave / RG;
+    const int ln = lane & 31, hb = lane >> 5, gl = lane & 15;
+    const int H = G * KVH;
+    const int R = n_q * G, nrb = (R + ROWS - 1) / ROWS;
+    // longest rows first, so the last blocks to start are the short ones
+    const int kvh = blockIdx.x % KVH, rb = nrb - 1 - (int)(blockIdx.x / KVH);
+    const int r0 = rb * ROWS, wr0 = r0 + rg * 32;
+    const int total = len0 + n_q - 1;
+    const int blk_last = (r0 + ROWS < R ? r0 + ROWS : R) - 1;
+    const int all_stages = (len0 + blk_last / G + KS - 1) / KS;
+    // split z of the block's keys: stages [st0, st1)
+    const int ns = (int)gridDim.y, per = (all_stages + ns - 1) / ns;
+    const int st0 = (int)blockIdx.y * per, st1 = st0 + per < all_stages ? st0 + per : all_stages;
+    const bool active = wr0 < R;
+    const int wlast = wr0 + 31 < R ? wr0 + 31 : R - 1;
+    const int row = wr0 + ln < R ? wr0 + ln : R - 1;
+    const int qs = row / G;
+    const int lim = len0 + qs;                                     // keys the lane's row sees
+    const int wmin = active ? len0 + wr0 / G : 0, wmax = active ? len0 + wlast / G : 0;
+    const int64_t kvs = (int64_t)KVH * D;
+    const f16* kh = k + (int64_t)kvh * D;
+    const f16* vh = v + (int64_t)kvh * D;
+    const int64_t q_off = ((int64_t)qs * H + (int64_t)kvh * G + (row - qs * G)) * D;
+
+    const uint32_t kv_bytes = (uint32_t)(((int64_t)total * kvs - (int64_t)kvh * D) * 2);
+    const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(const_cast<f16*>(kh), 0, (int)kv_bytes, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(const_cast<f16*>(vh), 0, (int)kv_bytes, 0x00020000);
+    const uint32_t stride = (uint32_t)(kvs * 2);
+    // a lane's 16 bytes of a load: row r of the stage, the chunk that belongs in its slot
+    auto stage = [&](auto P) -> f16* {
+        if constexpr (decltype(P)::value == 0) return sm0;
+        else return sm1;
+    };
+    auto issue = [&](auto P, int st) {
+        f16* sk = stage(P);
+        f16* sv = sk + KS * D;
+#pragma unroll
+        for (int i = 0; i < LP; i++) {
+            const int p = wave * LP + i, r = p * RPP + lane / CPR;
+            const int c = (lane % CPR) ^ attn_swz<D>(r);
+            const int key = st * KS + r < total ? st * KS + r : total - 1;
+            const uint32_t off = (uint32_t)key * stride + (uint32_t)c * 16;
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, sk + p * 512, 16, off, 0, 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rv, sv + p * 512, 16, off, 0, 0, 0);
+        }
+    };
+
+    constexpr auto P0 = std::integral_constant<int, 0>{};
+    constexpr auto P1 = std::integral_constant<int, 1>{};
+    if (st0 < st1) issue(P0, st0);
+    h8 qf[DT];
+#pragma unroll
+    for (int d = 0; d < DT; d++) qf[d] = *reinterpret_cast<const h8*>(q + q_off + 16 * d + 8 * hb);
+    float m = -1e30f, l = 0.0f;
+    f16v o[DE];
+#pragma unroll
+    for (int e = 0; e < DE; e++) o[e] = f16v{};
+
+    auto step = [&](auto P, auto PN, int st) {
+        wait_vmcnt<0>();
+        lds_barrier();  // stage st in LDS for every wave; every wave is done with stage st - 1
+        if (st + 1 < st1) issue(PN, st + 1);
+        const int k0 = st * KS + kg * 32;  // the wave's first key of the stage
+        if (k0 >= wmax) return;
+        const f16* sk = stage(P) + kg * 32 * D;
+        const f16* sv = sk + KS * D;
+        f16v s = f16v{};
+#pragma unroll
+        for (int d = 0; d < DT; d++) {
+            const h8 kf = *reinterpret_cast<const h8*>(sk + ln * D + (((2 * d + hb) ^ attn_swz<D>(ln)) * 8));
+            s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf, qf[d], s, 0, 0, 0);
+        }
+        if (k0 + 32 > wmin) {  // keys past some row's last visible one
+#pragma unroll
+            for (int i = 0; i < 16; i++)
+                if (k0 + 8 * (i / 4) + 4 * hb + i % 4 >= lim) s[i] = -INFINITY;
+        }
+        float mx = s[0];
+#pragma unroll
+        for (int i = 1; i < 16; i++) mx = fmaxf(mx, s[i]);
+        mx = max_x32(mx) * scale_log2;
+        const bool up = mx > m + 8.0f;
+        if (__any(up)) {
+            const float mn = up ? mx : m, corr = __builtin_amdgcn_exp2f(m - mn);
+            m = mn;
+            l *= corr;
+#pragma unroll
+            for (int e = 0; e < DE; e++) o[e] *= corr;
+        }
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            h8 ph, pl;
+#pragma unroll
+            for (int j = 0; j < 8; j += 2) {
+                float p[2];
+#pragma unroll
+                for (int w = 0; w < 2; w++) {
+                    p[w] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[8 * u + j + w], scale_log2, -m));
+                    l += p[w];
+                }
+                const h2 hi = __builtin_convertvector(f2{p[0], p[1]}, h2);
+                // the remainders, exact, by one mixed-precision FMA each
+                const h2 lo = __builtin_convertvector(
+                    f2{__builtin_fmaf((float)hi[0], -1.0f, p[0]), __builtin_fmaf((float)hi[1], -1.0f, p[1])}, h2);
+                ph[j] = hi[0];
+                ph[j + 1] = hi[1];
+                pl[j] = lo[0];
+                pl[j + 1] = lo[1];
+            }
+            // V^T: lane (dim 32 e + ln) of keys 16 u + 8 jj + 4 hb + 0..3, jj = 0, 1,
+            // one transpose read each (16 lanes: 4 keys x 16 dims)
+            h8 va[DE];
+#pragma unroll
+            for (int e = 0; e < DE; e++) {
+                h4v a[2];
+#pragma unroll
+                for (int jj = 0; jj < 2; jj++) {
+                    const int r = 16 * u + 8 * jj + 4 * hb + (gl >> 2);
+                    const int c = 4 * e + 2 * ((lane >> 4) & 1) + ((gl & 3) >> 1);
+                    a[jj] = lds_read_tr16(sv + r * D + (c ^ attn_swz<D>(r)) * 8 + 4 * (gl & 1));
+                }
+                va[e] = h8{a[0][0], a[0][1], a[0][2], a[0][3], a[1][0], a[1][1], a[1][2], a[1][3]};
+            }
+            // every dim tile's high product before the low ones: no product waits on the one before it
+#pragma unroll
+            for (int e = 0; e < DE; e++) o[e] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va[e], ph, o[e], 0, 0, 0);
+#pragma unroll
+            for (int e = 0; e < DE; e++) o[e] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va[e], pl, o[e], 0, 0, 0);
+        }
+    };
+    for (int st = st0; st < st1; st += 2) {
+        step(P0, P1, st);
+        if (st + 1 < st1) step(P1, P0, st + 1);
+    }
+    l = sum_x32(l);
+
+    lds_barrier();  // every wave is done with the stages
+    // wave w's O rows of D floats (half of the waves per stage), 16-byte chunk c of row r at slot c ^ r
+    auto os = [&](int w, int r, int c) {
+        return reinterpret_cast<f4*>((w < NW / 2 ? sm0 : sm1) + w % (NW / 2) * 64 * D) + r * (D / 4) + (c ^ (r & 15));
+    };
+    if (hb == 0) {
+        wm[wave][ln] = m;
+        wl[wave][ln] = l;
+    }
+    if (tid < ROWS) bad[tid] = 0;
+#pragma unroll
+    for (int e = 0; e < DE; e++)
+#pragma unroll
+        for (int g = 0; g < 4; g++)
+            *os(wave, ln, 8 * e + 2 * g + hb) =
+                f4{o[e][4 * g], o[e][4 * g + 1], o[e][4 * g + 2], o[e][4 * g + 3]};
+    __syncthreads();
+    auto row_off = [&](int r) {
+        const int s_ = r / G;
+        return ((int64_t)s_ * H + (int64_t)kvh * G + (r - s_ * G)) * D;
+    };
+    auto finish = [&](int rr, int d, f4 num, float den) {
+        h4v w;
+        bool nf = false;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const float y = num[j] / den;
+            nf = nf || !(__builtin_fabsf(y) <= 3.0e38f);
+            w[j] = (f16)y;
+        }
+        if (nf) bad[rr] = 1;
+        *reinterpret_cast<h4v*>(out + row_off(r0 + rr) + d) = w;
+    };
+    // partials of split z of row r: D floats at row z KVH R + kvh R + r, and (m, l) after all rows
+    const int64_t pr0 = ((int64_t)blockIdx.y * KVH + kvh) * R + r0;
+    f4* wo = reinterpret_cast<f4*>(ws);
+    float2* wml = reinterpret_cast<float2*>(ws + (int64_t)ns * KVH * R * D);
+    for (int idx = tid; idx < ROWS * (D / 4); idx += NT) {
+        const int rr = idx / (D / 4), c = idx % (D / 4);
+        if (r0 + rr >= R) break;
+        const int w0 = rr / 32, ri = rr & 31;  // wave of key group g: w0 + g RG
+        float M = wm[w0][ri];
+#pragma unroll
+        for (int g = 1; g < KG; g++) M = fmaxf(M, wm[w0 + g * RG][ri]);
+        f4 num = f4{0.0f, 0.0f, 0.0f, 0.0f};
+        float den = 0.0f;
+#pragma unroll
+        for (int g = 0; g < KG; g++) {
+            const float f = __builtin_amdgcn_exp2f(wm[w0 + g * RG][ri] - M);
+            num += f * *os(w0 + g * RG, ri, c);
+            den += f * wl[w0 + g * RG][ri];
+        }
+        if (ns == 1) {
+            finish(rr, 4 * c, num, den);
+        } else {
+            wo[(pr0 + rr) * (D / 4) + c] = num;
+            if (c == 0) wml[pr0 + rr] = make_float2(M, den);
+        }
+    }
+    if (ns > 1) return;  // k_attention_prefill_merge finishes the rows
+    __syncthreads();
+    for (int rr = wave; rr < ROWS; rr += NW) {
+        if (r0 + rr >= R) break;
+        if (!__builtin_amdgcn_readfirstlane(bad[rr])) continue;  // always, with finite inputs
+        const int64_t off = row_off(r0 + rr);
+        attn_row_general<D>(q + off, kh, vh, kvs, len0 + (r0 + rr) / G, scale, out + off, lane);
+    }
+}
+
+// The rows of a call whose keys were split over ns blocks: a wave per row sums
+// the splits' numerators and denominators under their common maximum, in order.
+template <int D>
+__global__ __launch_bounds__(256) void k_attention_prefill_merge(const f16* __restrict__ q, const f16* __restrict__ k,
+                                                                 const f16* __restrict__ v, int32_t n_q, int32_t len0,
+                                                                 int32_t KVH, int32_t G, float scale, int32_t ns,
+                                                                 f16* __restrict__ out, const float* __restrict__ ws)
+{
+    constexpr int E = D / 64;
+    const int lane = threadIdx.x & 63, R = n_q * G;
+    const int row = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + (threadIdx.x >> 6)));
+    if (row >= R * KVH) return;
+    const int kvh = row / R, r = row - kvh * R, s = r / G;
+    const int64_t rows = (int64_t)KVH * R;
+    const float2* wml = reinterpret_cast<const float2*>(ws + rows * ns * D);
+    float M = -1e30f, den = 0.0f;
+    float num[E] = {};
+    for (int z = 0; z < ns; z++) M = fmaxf(M, wml[z * rows + row].x);
+#pragma unroll 4
+    for (int z = 0; z < ns; z++) {
+        const float2 ml = wml[z * rows + row];
+        const float* o = ws + (z * rows + row) * D + lane * E;
+        const float f = __builtin_amdgcn_exp2f(ml.x - M);
+#pragma unroll
+        for (int e = 0; e < E; e++) num[e] += f * o[e];
+        den += f * ml.y;
+    }
+    const int64_t off = ((int64_t)s * G * KVH + (int64_t)kvh * G + (r - s * G)) * D;
+    bool nf = false;
+#pragma unroll
+    for (int e = 0; e < E; e++) {
+        const float y = num[e] / den;
+        nf = nf || !(__builtin_fabsf(y) <= 3.0e38f);
+        out[off + lane * E + e] = (f16)y;
+    }
+    if (__any(nf))  // not with finite inputs
+        attn_row_general<D>(q + off, k + (int64_t)kvh * D, v + (int64_t)kvh * D, (int64_t)KVH * D, len0 + s, scale,
+                            out + off, lane);
+}
+
+// The tile kernel's calls: fp16, head_dim 64 or 128, 16-byte aligned q, K and
+// V and 8-byte aligned out (its loads and stores), byte offsets within one
+// kv head's K and V rows and row numbers in 31 bits, and a positive scale (it
+// takes the maximum before scaling).
+bool attention_prefill_ok(const void* out, const void* q, const void* k, const void* v, int64_t n_q, int64_t len0,
+                          int64_t H, int64_t KVH, int64_t D, float scale, int dtype)
+{
+    return dtype == VVH_F16 && (D == 64 || D == 128) && scale > 0.0f && scale < INFINITY &&
+           ((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k) | reinterpret_cast<uintptr_t>(v)) & 15) == 0 &&
+           (reinterpret_cast<uintptr_t>(out) & 7) == 0 && n_q * (H / KVH) <= (1 << 30) &&
+           (len0 + n_q) * KVH * D * 2 < ((int64_t)1 << 31);
+}
+
+// Rows per block (32: 4 waves, one 32-key group each; 64: 8 waves) and blocks
+// sharing a row block's keys, the least of a model of the call fitted to forced
+// choices (graph replay): a stage of 128 keys costs a block about 1.4 us with
+// either shape, and the call's time follows its longest block or, with more
+// blocks than fit the chip at once (one per CU at head_dim 128, two at 64),
+// their sum; a split call adds the merge's launch and its partials, written
+// and read at about 3 TB/s.  Measured, 32 rows / 64 rows, splits in brackets:
+// 512 queries, 14 heads on 2 of 64: 7.7 / 9.2 us (2: 12.1 / 12.1); 2048, 12 on 2
+// of 128: 51.4 / 33.7; 500 after 3500 positions, same heads: 46.5 / 46.7 (2:
+// 53.1 / 33.8, 4: - / 40.1); 7 after 4000: 45.6 / 44.7 (8: 15.2 / 15.1); 256 from
+// the start: 9.0 / 10.7; 1500, 32 on 4 of 64: 31.3 / 28.1.
+AttnPrefillPlan attention_prefill_plan(int64_t n_q, int64_t len0, int64_t H, int64_t KVH, int64_t D, int64_t cus)
+{
+    const int64_t R = n_q * (H / KVH), slots = D == 64 ? 2 * cus : cus;
+    const int64_t longest = (len0 + n_q - 1 + 127) / 128;
+    const double mean = (double)(len0 + n_q / 2 + 127) / 128.0;
+    AttnPrefillPlan best{};
+    double best_t = INFINITY;
+    for (const int64_t rows : {32, 64}) {
+        const int64_t blocks = (R + rows - 1) / rows * KVH;
+        const int64_t smax = std::max<int64_t>(1, std::min<int64_t>({longest, slots / blocks, 32}));
+        for (int64_t sp = 1; sp <= smax; sp++) {
+            const double st = std::max((double)((longest + sp - 1) / sp), (double)blocks * mean / (double)slots);
+            double t = (rows == 32 ? 2.0 : 3.0) + 1.42 * st;
+            if (sp > 1) t += 3.0 + (double)(sp * n_q * H * (D + 2) * 8) / 3e6;
+            if (t < best_t) {
+                best_t = t;
+                best = AttnPrefillPlan{rows, blocks, sp};
+            }
+        }
+    }
+    return best;
+}
+
+int64_t attention_prefill_ws_floats(const AttnPrefillPlan& p, int64_t n_q, int64_t H, int64_t D)
+{
+    return p.splits > 1 ? p.splits * n_q * H * (D + 2) : 0;
+}
+
+int launch_attention_prefill(const AttnPrefillPlan& p, void* out, const void* q, const void* k, const void* v,
+                             int64_t n_q, int64_t len0, int64_t H, int64_t KVH, int64_t D, float scale, float* ws,
+                             void* stream)
+{
+    const float sl = (float)((double)scale * 1.4426950408889634);
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    auto go = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3((unsigned)p.blocks, (unsigned)p.splits), dim3(unsigned(8 * p.rows)), 0, s,
+                           (const f16*)q,
+                           (const f16*)k, (const f16*)v, (int32_t)n_q, (int32_t)len0, (int32_t)KVH, (int32_t)(H / KVH),
+                           scale, sl, (f16*)out, ws);
+    };
+    if (D == 64) p.rows == 32 ? go(k_attention_prefill<64, 1>) : go(k_attention_prefill<64, 2>);
+    else p.rows == 32 ? go(k_attention_prefill<128, 1>) : go(k_attention_prefill<128, 2>);
+    if (p.splits > 1) {
+        const dim3 grid((unsigned)((n_q * H + 3) / 4));
+        auto merge = [&](auto kern) {
+            hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, (const f16*)q, (const f16*)k, (const f16*)v, (int32_t)n_q,
+                               (int32_t)len0, (int32_t)KVH, (int32_t)(H / KVH), scale, (int32_t)p.splits, (f16*)out, ws);
+        };
+        D == 64 ? merge(k_attention_prefill_merge<64>) : merge(k_attention_prefill_merge<128>);
+    }
+    return (int)hipGetLastError();
+}
+
+}  // namespace vvh

@@ -327,6 +327,21 @@ int launch_embedding(void* out, const float* table, int64_t token, int64_t hidde
 int64_t attention_max_len();
 int launch_attention(void* out, const void* q, const void* k, const void* v, int64_t n_q, int64_t len0, int64_t H,
                      int64_t KVH, int64_t D, float scale, int dtype, void* stream);
+// The matrix-core form (attention_kernels.hip): whether it serves a call, its
+// tiles and splits on a device of `cus` CUs, and its launch (ws:
+// attention_prefill_ws_floats() floats when splits > 1).
+bool attention_prefill_ok(const void* out, const void* q, const void* k, const void* v, int64_t n_q, int64_t len0,
+                          int64_t H, int64_t KVH, int64_t D, float scale, int dtype);
+struct AttnPrefillPlan {
+    int64_t rows;    // (query, head) rows per block: 32 or 64
+    int64_t blocks;  // row blocks of all kv heads
+    int64_t splits;  // blocks that share a row block's keys (> 1: workspace and a merge launch)
+};
+AttnPrefillPlan attention_prefill_plan(int64_t n_q, int64_t len0, int64_t H, int64_t KVH, int64_t D, int64_t cus);
+int64_t attention_prefill_ws_floats(const AttnPrefillPlan& p, int64_t n_q, int64_t H, int64_t D);
+int launch_attention_prefill(const AttnPrefillPlan& p, void* out, const void* q, const void* k, const void* v,
+                             int64_t n_q, int64_t len0, int64_t H, int64_t KVH, int64_t D, float scale, float* ws,
+                             void* stream);
 // n_q = 1 fast path: grouped heads, split over the sequence into nb blocks
 // per kv head.  mfma: the fp16 matrix-core kernel (head_dim 64 or 128), which
 // merges the blocks in the same launch and, with nb > 1, needs a zeroed

@@ -197,6 +197,27 @@ int counters_for(void* stream, unsigned** out)
     return VVH_OK;
 }
 
+// The stream's workspace of `bytes`, for calls that can do without: false
+// where it would have to grow while the stream is being captured, or cannot.
+bool workspace_try(void* stream, std::size_t bytes, float** ws)
+{
+    bool have;
+    {
+        std::lock_guard<std::mutex> lock(g_wsmu);
+        const auto it = g_ws.find(stream);
+        have = it != g_ws.end() && it->second.bytes >= bytes;
+    }
+    if (!have) {
+        hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(static_cast<hipStream_t>(stream), &st) != hipSuccess) {
+            (void)hipGetLastError();
+            return false;
+        }
+        if (st != hipStreamCaptureStatusNone) return false;
+    }
+    return workspace_for(stream, bytes, ws) == VVH_OK;
+}
+
 // ---- fixed scratch of vvh_linear_q8_dev_noalloc ------------------------------
 // The split-K partial planes of the allocation-free entry point live in this
 // file-scope device array: the code object holds it on every device the
@@ -2050,6 +2071,20 @@ VVH_API int vvh_attention(void* out, const void* q, const void* k, const void* v
         return ret_launch(launch_attention_decode(p, out, q, k, v, (int64_t)len0, (int64_t)num_heads,
                                                   (int64_t)num_kv_heads, (int64_t)head_dim, scale, ws, cnt, dtype,
                                                   stream),
+                          "attention launch");
+    }
+    if (attention_prefill_ok(out, q, k, v, (int64_t)n_q, (int64_t)len0, (int64_t)num_heads, (int64_t)num_kv_heads,
+                             (int64_t)head_dim, scale, dtype)) {
+        AttnPrefillPlan p = attention_prefill_plan((int64_t)n_q, (int64_t)len0, (int64_t)num_heads,
+                                                   (int64_t)num_kv_heads, (int64_t)head_dim,
+                                                   g_cu_count > 0 ? g_cu_count : 256);
+        // splits need the stream's workspace; without it (a capture that
+        // cannot allocate, no memory) each block takes all its keys
+        float* ws = nullptr;
+        const int64_t wsf = attention_prefill_ws_floats(p, (int64_t)n_q, (int64_t)num_heads, (int64_t)head_dim);
+        if (wsf > 0 && !workspace_try(stream, (std::size_t)wsf * 4, &ws)) p.splits = 1;
+        return ret_launch(launch_attention_prefill(p, out, q, k, v, (int64_t)n_q, (int64_t)len0, (int64_t)num_heads,
+                                                   (int64_t)num_kv_heads, (int64_t)head_dim, scale, ws, stream),
                           "attention launch");
     }
     return ret_launch(launch_attention(out, q, k, v, (int64_t)n_q, (int64_t)len0, (int64_t)num_heads,
