@@ -32,6 +32,37 @@ __device__ __forceinline__ float ldf(const T* p, int64_t i) { return (float)p[i]
 template <typename T>
 __device__ __forceinline__ void stf(T* p, int64_t i, float v) { p[i] = (T)v; }
 
+// 8 consecutive elements at p (16-byte aligned) as fp32
+__device__ __forceinline__ void load8(const f16* p, float f[8])
+{
+    const h8 v = *reinterpret_cast<const h8*>(p);
+#pragma unroll
+    for (int e = 0; e < 8; e++) f[e] = (float)v[e];
+}
+__device__ __forceinline__ void load8(const float* p, float f[8])
+{
+    const f4 a = *reinterpret_cast<const f4*>(p), b = *reinterpret_cast<const f4*>(p + 4);
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        f[e] = a[e];
+        f[4 + e] = b[e];
+    }
+}
+
+// 8 consecutive elements at p (16-byte aligned), rounded once to T
+__device__ __forceinline__ void store8(f16* p, const float f[8])
+{
+    h8 v;
+#pragma unroll
+    for (int e = 0; e < 8; e++) v[e] = (f16)f[e];
+    *reinterpret_cast<h8*>(p) = v;
+}
+__device__ __forceinline__ void store8(float* p, const float f[8])
+{
+    *reinterpret_cast<f4*>(p) = f4{f[0], f[1], f[2], f[3]};
+    *reinterpret_cast<f4*>(p + 4) = f4{f[4], f[5], f[6], f[7]};
+}
+
 __device__ __forceinline__ float silu_ref(float v) { return v * (1.0f / (1.0f + expf(-v))); }
 
 // Block-wide sum / max over 256 threads (4 waves); `red` holds 4 floats.
@@ -65,19 +96,62 @@ __global__ __launch_bounds__(256) void k_eltwise(T* __restrict__ out, const T* _
     }
 }
 
+// The same in chunks of 8 values per thread (16-byte loads and stores), for
+// arrays of 16-byte aligned pointers; the last n % 8 values go one per thread
+// of the last block.  Not for silu alone, whose product the compiler rounds to
+// fp16 directly in k_eltwise and not here.
+template <typename T, int OP>
+__global__ __launch_bounds__(256) void k_eltwise_vec(T* __restrict__ out, const T* __restrict__ x,
+                                                     const T* __restrict__ y, int64_t n)
+{
+    auto one = [](float a, float b) {
+        if constexpr (OP == VVH_OP_ADD) return a + b;
+        else if constexpr (OP == VVH_OP_MUL) return a * b;
+        else return silu_mul_ref(a, b);
+    };
+    const int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x, nc = n / 8;
+    if (c < nc) {
+        float a[8], b[8], r[8];
+        load8(x + 8 * c, a);
+        load8(y + 8 * c, b);
+#pragma unroll
+        for (int e = 0; e < 8; e++) r[e] = one(a[e], b[e]);
+        store8(out + 8 * c, r);
+    }
+    if (blockIdx.x == gridDim.x - 1 && 8 * nc + threadIdx.x < n) {
+        const int64_t i = 8 * nc + threadIdx.x;
+        stf(out, i, one(ldf(x, i), ldf(y, i)));
+    }
+}
+
+// Values from which the chunks pay: below, fewer and longer threads leave CUs
+// idle (graph replay, fp16 silu_mul: 1.1 M values 3.2 us either way, 2.5 M 4.7 ->
+// 4.6, 18.4 M, a 2048-token 1.5B prompt, 22.9 -> 20.5: 5.4 TB/s, the division
+// and the exponential of each value bound it).
+constexpr int64_t kEltwiseVecMin = 1 << 21;
+
 int launch_eltwise(int op, void* out, const void* x, const void* y, int64_t n, int dtype, void* stream)
 {
+    const bool vec = op != VVH_OP_SILU && n >= kEltwiseVecMin && n / 2048 < INT32_MAX &&
+                     ((reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(x) |
+                       reinterpret_cast<uintptr_t>(y)) & 15) == 0;
     const int64_t want = (n + 255) / 256;
-    const dim3 grid((unsigned)(want < 8192 ? (want > 0 ? want : 1) : 8192));
+    const dim3 grid((unsigned)(vec ? (n / 8 + 255) / 256 : want < 8192 ? (want > 0 ? want : 1) : 8192));
     hipStream_t s = static_cast<hipStream_t>(stream);
-#define VVH_EW(T)                                                                                              \
-    switch (op) {                                                                                              \
-        case VVH_OP_ADD: hipLaunchKernelGGL((k_eltwise<T, VVH_OP_ADD>), grid, dim3(256), 0, s, (T*)out, (const T*)x, (const T*)y, n); break; \
-        case VVH_OP_MUL: hipLaunchKernelGGL((k_eltwise<T, VVH_OP_MUL>), grid, dim3(256), 0, s, (T*)out, (const T*)x, (const T*)y, n); break; \
-        case VVH_OP_SILU: hipLaunchKernelGGL((k_eltwise<T, VVH_OP_SILU>), grid, dim3(256), 0, s, (T*)out, (const T*)x, (const T*)y, n); break; \
-        default: hipLaunchKernelGGL((k_eltwise<T, VVH_OP_SILU_MUL>), grid, dim3(256), 0, s, (T*)out, (const T*)x, (const T*)y, n); break; \
+#define VVH_EWV(T, OP)                                                                                          \
+    if (vec) hipLaunchKernelGGL((k_eltwise_vec<T, OP>), grid, dim3(256), 0, s, (T*)out, (const T*)x, (const T*)y, n); \
+    else hipLaunchKernelGGL((k_eltwise<T, OP>), grid, dim3(256), 0, s, (T*)out, (const T*)x, (const T*)y, n);
+#define VVH_EW(T)                                    \
+    switch (op) {                                    \
+        case VVH_OP_ADD: VVH_EWV(T, VVH_OP_ADD) break;   \
+        case VVH_OP_MUL: VVH_EWV(T, VVH_OP_MUL) break;   \
+        case VVH_OP_SILU:                            \
+            hipLaunchKernelGGL((k_eltwise<T, VVH_OP_SILU>), grid, dim3(256), 0, s, (T*)out, (const T*)x, (const T*)y, n); \
+            break;                                   \
+        default: VVH_EWV(T, VVH_OP_SILU_MUL) break;      \
     }
     if (dtype == VVH_F16) { VVH_EW(f16) } else { VVH_EW(float) }
+#undef VVH_EWV
 #undef VVH_EW
     return (int)hipGetLastError();
 }
@@ -159,10 +233,62 @@ __global__ __launch_bounds__(256) void k_rms_norm(T* __restrict__ out, const T* 
     for (int64_t i = threadIdx.x; i < n; i += 256) stf(orow, i, rms_apply(ldf(xr, i), rms, w[i]));
 }
 
+// Many rows of up to 2048 values: one wave per row, its chunks in registers
+// between the sum and the output (the block per row above reads the row once
+// per wave).  Same sums in the same order, so the same bits.
+template <typename T>
+__global__ __launch_bounds__(256) void k_rms_norm_rows(T* __restrict__ out, const T* __restrict__ x,
+                                                       const float* __restrict__ w, int64_t rows, int64_t n, float eps)
+{
+    constexpr int RJ = 4;
+    const int lane = threadIdx.x & 63;
+    const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (row >= rows) return;
+    const T* xr = x + row * n;
+    T* orow = out + row * n;
+    const int64_t nc = n / 8;
+    float v[RJ][8], ss = 0.0f;
+#pragma unroll
+    for (int j = 0; j < RJ; j++) load8(xr + 8 * (lane + 64 * j < nc ? lane + 64 * j : nc - 1), v[j]);
+#pragma unroll
+    for (int j = 0; j < RJ; j++) {
+        float z[8];
+#pragma unroll
+        for (int e = 0; e < 8; e++) z[e] = lane + 64 * j < nc ? v[j][e] : 0.0f;
+        ss = rms_sumsq8(ss, z);
+    }
+    const float rms = rms_of(wave_sum_xor(ss), n, eps);
+#pragma unroll
+    for (int j = 0; j < RJ; j++) {
+        const int64_t c = lane + 64 * j;
+        if (c < nc) {
+            float wf[8], r[8];
+            load8(w + 8 * c, wf);
+#pragma unroll
+            for (int e = 0; e < 8; e++) r[e] = rms_apply(v[j][e], rms, wf[e]);
+            store8(orow + 8 * c, r);
+        }
+    }
+}
+
+// Rows from which a wave per row pays (graph replay, fp16: 512 rows of 896 3.2 ->
+// 3.0 us, 2048 of 1536 7.5 -> 4.6; 256 of 896 2.7 -> 2.9).
+constexpr int64_t kRmsRowsMin = 512;
+
 int launch_rms_norm(void* out, const void* x, const float* w, int64_t rows, int64_t n, float eps, int dtype,
                     void* stream)
 {
     hipStream_t s = static_cast<hipStream_t>(stream);
+    if (rows >= kRmsRowsMin && n % 8 == 0 && n <= 2048 &&
+        ((reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w)) & 15) == 0) {
+        const dim3 grid((unsigned)((rows + 3) / 4));
+        if (dtype == VVH_F16)
+            hipLaunchKernelGGL(k_rms_norm_rows<f16>, grid, dim3(256), 0, s, (f16*)out, (const f16*)x, w, rows, n, eps);
+        else
+            hipLaunchKernelGGL(k_rms_norm_rows<float>, grid, dim3(256), 0, s, (float*)out, (const float*)x, w, rows, n,
+                               eps);
+        return (int)hipGetLastError();
+    }
     if (dtype == VVH_F16)
         hipLaunchKernelGGL(k_rms_norm<f16>, dim3((unsigned)rows), dim3(256), 0, s, (f16*)out, (const f16*)x, w, n, eps);
     else
@@ -255,6 +381,94 @@ __global__ __launch_bounds__(256) void k_rope(T* __restrict__ q, T* __restrict__
     }
 }
 
+// Many positions (a prompt): a block takes 256 / (D / 2) of them, works out
+// each position's D / 2 cosines and sines once (in k_rope every head does, in
+// fp64), and rotates the rows of every head in chunks of 8 pairs.  D a power of
+// two from 16 to 512, 16-byte aligned arrays; the same bits as k_rope.
+template <typename T, bool APPEND>
+__global__ __launch_bounds__(256) void k_rope_rows(T* __restrict__ q, T* __restrict__ k, int64_t S, int32_t H,
+                                                   int32_t KVH, int32_t D, int64_t pos, float theta,
+                                                   const T* __restrict__ v, T* __restrict__ kc, T* __restrict__ vc)
+{
+    __shared__ __align__(16) float cs[256], sn[256];
+    const int half = D / 2, P = 256 / half, hc = half / 8;  // hc: chunks of 8 pairs per head row
+    const int64_t s0 = (int64_t)blockIdx.x * P;
+    {
+        const int p = threadIdx.x / half, i = threadIdx.x - p * half;
+        rope_cs(pos + s0 + p, i, D, theta, cs[threadIdx.x], sn[threadIdx.x]);
+    }
+    __syncthreads();
+    const int heads = H + KVH, per = heads * hc;  // chunks per position: q's heads, then k's
+    const int np = S - s0 < P ? (int)(S - s0) : P;
+    for (int g = threadIdx.x; g < np * per; g += 256) {
+        const int p = g / per, r = g - p * per, h = r / hc, i = (r - h * hc) * 8;
+        const int64_t s = s0 + p, kr = (s * KVH + (h - H)) * D;
+        T* base = h < H ? q + (s * H + h) * D : k + kr;
+        float x0[8], x1[8], c[8], d[8], r0[8], r1[8];
+        load8(base + i, x0);
+        load8(base + half + i, x1);
+        load8(cs + p * half + i, c);
+        load8(sn + p * half + i, d);
+#pragma unroll
+        for (int e = 0; e < 8; e++) rope_apply(x0[e], x1[e], c[e], d[e], r0[e], r1[e]);
+        store8(base + i, r0);
+        store8(base + half + i, r1);
+        if constexpr (APPEND) {
+            if (h >= H) {
+                const int64_t dst = pos * KVH * D + kr;
+                store8(kc + dst + i, r0);
+                store8(kc + dst + half + i, r1);
+                constexpr int W = sizeof(T) / 2;  // 16-byte pieces of 8 values
+#pragma unroll
+                for (int e = 0; e < 2 * W; e++) {
+                    const int o = (e / W) * half + i + (e % W) * (8 / W);
+                    *reinterpret_cast<u4*>(vc + dst + o) = *reinterpret_cast<const u4*>(v + kr + o);
+                }
+            }
+        }
+    }
+}
+
+// Whether the form above serves a call: its shapes, and enough pairs that
+// sharing a position's angles over the heads pays for the blocks it leaves
+// unused (graph replay, 0.5B heads, 256 / 512 positions: 4.0 / 5.4 us with a
+// thread per pair, 4.1 / 4.2 here; 2048 positions of the 1.5B heads 24.1 -> 6.4).
+constexpr int64_t kRopeRowsMin = 200000;
+static bool rope_rows_ok(const void* q, const void* k, const void* v, const void* kc, const void* vc, int64_t S,
+                         int64_t H, int64_t KVH, int64_t D)
+{
+    return S * (H + KVH) * (D / 2) >= kRopeRowsMin && D >= 16 && D <= 512 && (D & (D - 1)) == 0 && H + KVH <= 65535 &&
+           S <= (int64_t)INT32_MAX && ((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k) |
+             reinterpret_cast<uintptr_t>(v) | reinterpret_cast<uintptr_t>(kc) | reinterpret_cast<uintptr_t>(vc)) & 15) == 0;
+}
+
+template <bool APPEND>
+static int rope_go(void* q, void* k, const void* v, void* kc, void* vc, int64_t S, int64_t H, int64_t KVH, int64_t D,
+                   int64_t pos, float theta, int dtype, hipStream_t s)
+{
+    if (rope_rows_ok(q, k, v, kc, vc, S, H, KVH, D)) {
+        const int64_t P = 512 / D;
+        const dim3 grid((unsigned)((S + P - 1) / P));
+        if (dtype == VVH_F16)
+            hipLaunchKernelGGL((k_rope_rows<f16, APPEND>), grid, dim3(256), 0, s, (f16*)q, (f16*)k, S, (int32_t)H,
+                               (int32_t)KVH, (int32_t)D, pos, theta, (const f16*)v, (f16*)kc, (f16*)vc);
+        else
+            hipLaunchKernelGGL((k_rope_rows<float, APPEND>), grid, dim3(256), 0, s, (float*)q, (float*)k, S, (int32_t)H,
+                               (int32_t)KVH, (int32_t)D, pos, theta, (const float*)v, (float*)kc, (float*)vc);
+        return (int)hipGetLastError();
+    }
+    const int64_t total = S * (H + KVH) * (D / 2);
+    const int64_t want = (total + 255) / 256;
+    const dim3 grid((unsigned)(want < 4096 ? (want > 0 ? want : 1) : 4096));
+    if (dtype == VVH_F16)
+        hipLaunchKernelGGL((k_rope<f16, APPEND>), grid, dim3(256), 0, s, (f16*)q, (f16*)k, S, H, KVH, D, pos, theta,
+                           (const f16*)v, (f16*)kc, (f16*)vc);
+    else
+        hipLaunchKernelGGL((k_rope<float, APPEND>), grid, dim3(256), 0, s, (float*)q, (float*)k, S, H, KVH, D, pos,
+                           theta, (const float*)v, (float*)kc, (float*)vc);
+    return (int)hipGetLastError();
+}
+
 __global__ __launch_bounds__(256) void k_rope_freq(float* __restrict__ out, int64_t D, float theta)
 {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -291,33 +505,14 @@ int launch_rope_table(float* out, const float* freq, int64_t positions, int64_t 
 int launch_rope(void* q, void* k, int64_t S, int64_t H, int64_t KVH, int64_t D, int64_t pos, float theta, int dtype,
                 void* stream)
 {
-    const int64_t total = S * (H + KVH) * (D / 2);
-    const int64_t want = (total + 255) / 256;
-    const dim3 grid((unsigned)(want < 4096 ? (want > 0 ? want : 1) : 4096));
-    hipStream_t s = static_cast<hipStream_t>(stream);
-    if (dtype == VVH_F16)
-        hipLaunchKernelGGL((k_rope<f16, false>), grid, dim3(256), 0, s, (f16*)q, (f16*)k, S, H, KVH, D, pos, theta,
-                           nullptr, nullptr, nullptr);
-    else
-        hipLaunchKernelGGL((k_rope<float, false>), grid, dim3(256), 0, s, (float*)q, (float*)k, S, H, KVH, D, pos,
-                           theta, nullptr, nullptr, nullptr);
-    return (int)hipGetLastError();
+    return rope_go<false>(q, k, nullptr, nullptr, nullptr, S, H, KVH, D, pos, theta, dtype,
+                          static_cast<hipStream_t>(stream));
 }
 
 int launch_rope_append(void* q, void* k, const void* v, void* kc, void* vc, int64_t S, int64_t H, int64_t KVH,
                        int64_t D, int64_t pos, float theta, int dtype, void* stream)
 {
-    const int64_t total = S * (H + KVH) * (D / 2);
-    const int64_t want = (total + 255) / 256;
-    const dim3 grid((unsigned)(want < 4096 ? (want > 0 ? want : 1) : 4096));
-    hipStream_t s = static_cast<hipStream_t>(stream);
-    if (dtype == VVH_F16)
-        hipLaunchKernelGGL((k_rope<f16, true>), grid, dim3(256), 0, s, (f16*)q, (f16*)k, S, H, KVH, D, pos, theta,
-                           (const f16*)v, (f16*)kc, (f16*)vc);
-    else
-        hipLaunchKernelGGL((k_rope<float, true>), grid, dim3(256), 0, s, (float*)q, (float*)k, S, H, KVH, D, pos,
-                           theta, (const float*)v, (float*)kc, (float*)vc);
-    return (int)hipGetLastError();
+    return rope_go<true>(q, k, v, kc, vc, S, H, KVH, D, pos, theta, dtype, static_cast<hipStream_t>(stream));
 }
 
 // ---------------------------------------------------------------------------
@@ -433,23 +628,6 @@ __host__ __device__ inline int attn_lanes(int D)
     int L = 1;
     while (L * 8 < D) L <<= 1;
     return L;
-}
-
-// 8 consecutive elements at p (16-byte aligned) as fp32
-__device__ __forceinline__ void load8(const f16* p, float f[8])
-{
-    const h8 v = *reinterpret_cast<const h8*>(p);
-#pragma unroll
-    for (int e = 0; e < 8; e++) f[e] = (float)v[e];
-}
-__device__ __forceinline__ void load8(const float* p, float f[8])
-{
-    const f4 a = *reinterpret_cast<const f4*>(p), b = *reinterpret_cast<const f4*>(p + 4);
-#pragma unroll
-    for (int e = 0; e < 4; e++) {
-        f[e] = a[e];
-        f[4 + e] = b[e];
-    }
 }
 
 // ONE: the block's span is a single sub-chunk (per_block <= C), so there is
