@@ -1,12 +1,12 @@
-"""vvh_attention of several queries on the matrix cores (fp16, head_dim 64 and
-128) against causal attention in 64 bits (backend_naive.cc:344-378), at the
-edges of its tiles: rows of 32, 64 and 128 (query, head) pairs, stages of 64
-and 128 keys, one query more or less than they hold.
+"""vvh_attention of several queries on the matrix cores (head_dim 64 and 128)
+against causal attention in 64 bits (backend_naive.cc:344-378), at the edges of
+its tiles: rows of 32 and 64 (query, head) pairs, stages of 64 and 128 keys, one
+query more or less than they hold, keys split over blocks or not.
 
-Tolerance per element: the output's rounding to fp16 (half an ulp, 2^-11 of
-the value), plus the scores' fp32 sums (|score| up to about 8 with products of
-22 + bits: 2e-6 of the weight each) and the weights' 22 bits, together below
-1e-5 of the largest |v|.
+Tolerance per element: the output's rounding (fp16: half an ulp, 2^-11 of the
+value), plus the scores' fp32 sums (|score| up to about 8, so 2e-6 of each
+weight) and the weights' 22 bits or more, together below 1e-5 of the largest
+|v|.
 """
 import numpy as np
 import pytest
@@ -15,7 +15,12 @@ from vvllm_amd import capi
 
 pytestmark = pytest.mark.gpu
 
-F16 = capi.F16
+F16, F32 = capi.F16, capi.F32
+ULP = {F16: 2.0 ** -11, F32: 0.0}
+
+
+def npd(d):
+    return np.float32 if d == F32 else np.float16
 
 
 def reference(q, k, v, len0, scale):
@@ -31,20 +36,20 @@ def reference(q, k, v, len0, scale):
     return out
 
 
-def run(q, k, v, len0, scale):
+def run(q, k, v, len0, scale, d):
     n_q, H, D = q.shape
     dq, dk, dv = (capi.DevBuf.from_array(a) for a in (q, k, v))
-    do = capi.DevBuf(n_q * H * D * 2)
-    capi.call("vvh_attention", do.ptr, dq.ptr, dk.ptr, dv.ptr, n_q, len0, H, k.shape[1], D, scale, F16, None)
+    do = capi.DevBuf(q.nbytes)
+    capi.call("vvh_attention", do.ptr, dq.ptr, dk.ptr, dv.ptr, n_q, len0, H, k.shape[1], D, scale, d, None)
     capi.sync()
-    return do.to_array(np.float16, (n_q, H, D)).astype(np.float64)
+    return do.to_array(npd(d), (n_q, H, D)).astype(np.float64)
 
 
-def draw(n_q, len0, H, KVH, D):
+def draw(n_q, len0, H, KVH, D, d):
     rng = np.random.default_rng(n_q * 1000 + len0 + H)
     T = len0 + n_q - 1
-    return (rng.normal(0, 2, (n_q, H, D)).astype(np.float16), rng.normal(0, 1, (T, KVH, D)).astype(np.float16),
-            rng.normal(0, 1, (T, KVH, D)).astype(np.float16), float(1 / np.sqrt(D)))
+    return (rng.normal(0, 2, (n_q, H, D)).astype(npd(d)), rng.normal(0, 1, (T, KVH, D)).astype(npd(d)),
+            rng.normal(0, 1, (T, KVH, D)).astype(npd(d)), float(1 / np.sqrt(D)))
 
 
 # G = H / KVH rows per query
@@ -53,29 +58,31 @@ CASES = [(2, 1, 14, 2, 64), (5, 1, 7, 1, 64), (33, 1, 1, 1, 64), (31, 97, 2, 2, 
          (700, 200, 12, 2, 128), (1025, 1, 64, 8, 64), (1100, 60, 64, 8, 128)]
 
 
+@pytest.mark.parametrize("d", [F32, F16])
 @pytest.mark.parametrize("n_q,len0,H,KVH,D", CASES)
-def test_prefill(gpu, n_q, len0, H, KVH, D):
-    print(f"[case] prefill attention n_q={n_q} len0={len0} H={H} KVH={KVH} D={D}", flush=True)
-    q, k, v, scale = draw(n_q, len0, H, KVH, D)
-    got, ref = run(q, k, v, len0, scale), reference(q, k, v, len0, scale)
-    assert (np.abs(got - ref) <= 2.0 ** -11 * np.abs(ref) + 1e-5 * np.abs(v).max()).all()
+def test_prefill(gpu, n_q, len0, H, KVH, D, d):
+    print(f"[case] prefill attention n_q={n_q} len0={len0} H={H} KVH={KVH} D={D} dtype={d}", flush=True)
+    q, k, v, scale = draw(n_q, len0, H, KVH, D, d)
+    got, ref = run(q, k, v, len0, scale, d), reference(q, k, v, len0, scale)
+    assert (np.abs(got - ref) <= ULP[d] * np.abs(ref) + 1e-5 * np.abs(v).max()).all()
 
 
 @pytest.mark.parametrize("n_q,len0,H,KVH,D", [(40, 3, 6, 2, 64), (70, 30, 12, 2, 128), (1100, 1, 64, 8, 64)])
+@pytest.mark.parametrize("d", [F32, F16])
 @pytest.mark.parametrize("bad", [np.inf, np.nan, 65504.0])
-def test_prefill_unseen_rows(gpu, n_q, len0, H, KVH, D, bad):
+def test_prefill_unseen_rows(gpu, n_q, len0, H, KVH, D, d, bad):
     """A query's result does not depend on keys and values past its last
     visible position, whatever they hold; queries that see them carry them."""
-    print(f"[case] unseen rows n_q={n_q} len0={len0} D={D} bad={bad}", flush=True)
-    q, k, v, scale = draw(n_q, len0, H, KVH, D)
+    print(f"[case] unseen rows n_q={n_q} len0={len0} D={D} dtype={d} bad={bad}", flush=True)
+    q, k, v, scale = draw(n_q, len0, H, KVH, D, d)
     t = len0 + n_q - 4  # visible to the last three queries only
     v[t, KVH - 1, 5] = bad
     k[t + 1, 0, 3] = bad
-    got = run(q, k, v, len0, scale)
+    got = run(q, k, v, len0, scale, d)
     clean_k, clean_v = k.copy(), v.copy()
     clean_v[t, KVH - 1, 5] = clean_k[t + 1, 0, 3] = 0
     ref = reference(q, clean_k, clean_v, len0, scale)
     early = slice(0, n_q - 3)
-    assert (np.abs(got - ref)[early] <= 2.0 ** -11 * np.abs(ref)[early] + 1e-5 * np.abs(clean_v).max()).all()
+    assert (np.abs(got - ref)[early] <= ULP[d] * np.abs(ref)[early] + 1e-5 * np.abs(clean_v).max()).all()
     if not np.isfinite(bad):
         assert not np.isfinite(got[n_q - 3:, H - 1, 5]).any()

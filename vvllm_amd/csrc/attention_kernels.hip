@@ -38,9 +38,9 @@ __device__ __forceinline__ int attn_swz(int r)
 // result from the tiles is not finite: a key past a row's last visible one
 // has weight 0 in the tiles, and 0 times an infinity or NaN of its V row
 // would reach the sums.
-template <int D>
-__device__ void attn_row_general(const f16* __restrict__ qr, const f16* __restrict__ kh, const f16* __restrict__ vh,
-                                 int64_t kvs, int len, float scale, f16* __restrict__ orow, int lane)
+template <typename T, int D>
+__device__ void attn_row_general(const T* __restrict__ qr, const T* __restrict__ kh, const T* __restrict__ vh,
+                                 int64_t kvs, int len, float scale, T* __restrict__ orow, int lane)
 {
     constexpr int E = D / 64;
     float qv[E], o[E];
@@ -64,7 +64,7 @@ __device__ void attn_row_general(const f16* __restrict__ qr, const f16* __restri
         for (int e = 0; e < E; e++) o[e] += p * (float)vh[t * kvs + lane * E + e];
     }
 #pragma unroll
-    for (int e = 0; e < E; e++) orow[lane * E + e] = (f16)o[e];
+    for (int e = 0; e < E; e++) orow[lane * E + e] = (T)o[e];
 }
 
 }  // namespace
@@ -324,17 +324,232 @@ __global__ __launch_bounds__(256 * RG) void k_attention_prefill(
         if (r0 + rr >= R) break;
         if (!__builtin_amdgcn_readfirstlane(bad[rr])) continue;  // always, with finite inputs
         const int64_t off = row_off(r0 + rr);
-        attn_row_general<D>(q + off, kh, vh, kvs, len0 + (r0 + rr) / G, scale, out + off, lane);
+        attn_row_general<f16, D>(q + off, kh, vh, kvs, len0 + (r0 + rr) / G, scale, out + off, lane);
+    }
+}
+
+// ---------------------------------------------------------------------------
+// fp32 q, K and V, head_dim 64 or 128, on v_mfma_f32_32x32x2_f32: the same
+// rows, tiles, softmax and merge, with exact fp32 products and sums throughout
+// (no operand is split or rounded).  A stage holds 8192 / D keys (64 KB of K
+// and V); KG waves share them, RG row groups, 4 waves in all, one block per CU.
+// The assignment of dims (K q^T) and keys (V^T p) to an MFMA's two k slots is
+// free as long as both operands share it:
+//   K q^T   slot hb = lane / 32 takes dims hb D / 2 + j, so a 16-byte read of a
+//           K row feeds 4 MFMAs, and a lane keeps D / 2 dims of its query row;
+//   V^T p   slot hb takes the lane's own keys 8 (i / 4) + 4 hb + i % 4; row r of
+//           dim tile e is dim DE r + e, so a read of DE consecutive values of a V
+//           row feeds the DE tiles.
+// The exponent adds the low half of scale log2 e (scale_lo), which fp32 rounds
+// off, and the running maximum follows every new one, so that the largest
+// weights have the smallest exponents to round.
+// Bound by the fp32 matrix rate (64 clocks per MFMA, D / 2 + 16 DE of them per
+// 32 x 32 scores).
+// ---------------------------------------------------------------------------
+template <int D, int RG, int KG>
+__global__ __launch_bounds__(256) void k_attention_prefill_f32(
+    const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v, int32_t n_q, int32_t len0,
+    int32_t KVH, int32_t G, float scale, float scale_log2, float scale_lo, float* __restrict__ out,
+    float* __restrict__ ws)
+{
+    static_assert(RG * KG == 4, "4 waves");
+    constexpr int ROWS = 32 * RG;
+    constexpr int KS = 32 * KG;           // keys per stage
+    constexpr int CPR = D / 4;            // 16-byte chunks per row
+    constexpr int RPP = 64 / CPR;         // rows per 1 KB load
+    constexpr int LP = KS / RPP / 4;      // loads of K (and of V) per wave and stage
+    constexpr int DE = D / 32;
+    constexpr int kStage = 2 * KS * D;    // floats: K rows, then V rows
+    static_assert(kStage >= 2 * 32 * D, "two waves' O in each stage");
+    typedef float fe __attribute__((ext_vector_type(DE)));
+    __shared__ __align__(1024) float sm0[kStage], sm1[kStage];
+    __shared__ float wm[4][32], wl[4][32];
+    __shared__ int32_t bad[ROWS];
+
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int rg = wave % RG, kg = wave / RG;
+    const int ln = lane & 31, hb = lane >> 5;
+    const int H = G * KVH;
+    const int R = n_q * G, nrb = (R + ROWS - 1) / ROWS;
+    const int kvh = blockIdx.x % KVH, rb = nrb - 1 - (int)(blockIdx.x / KVH);  // longest rows first
+    const int r0 = rb * ROWS, wr0 = r0 + rg * 32;
+    const int total = len0 + n_q - 1;
+    const int blk_last = (r0 + ROWS < R ? r0 + ROWS : R) - 1;
+    const int all_stages = (len0 + blk_last / G + KS - 1) / KS;
+    const int ns = (int)gridDim.y, per = (all_stages + ns - 1) / ns;
+    const int st0 = (int)blockIdx.y * per, st1 = st0 + per < all_stages ? st0 + per : all_stages;
+    const bool active = wr0 < R;
+    const int wlast = wr0 + 31 < R ? wr0 + 31 : R - 1;
+    const int row = wr0 + ln < R ? wr0 + ln : R - 1;
+    const int qs = row / G;
+    const int lim = len0 + qs;
+    const int wmin = active ? len0 + wr0 / G : 0, wmax = active ? len0 + wlast / G : 0;
+    const int64_t kvs = (int64_t)KVH * D;
+    const float* kh = k + (int64_t)kvh * D;
+    const float* vh = v + (int64_t)kvh * D;
+    const int64_t q_off = ((int64_t)qs * H + (int64_t)kvh * G + (row - qs * G)) * D;
+
+    const uint32_t kv_bytes = (uint32_t)(((int64_t)total * kvs - (int64_t)kvh * D) * 4);
+    const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(kh), 0, (int)kv_bytes, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(vh), 0, (int)kv_bytes, 0x00020000);
+    const uint32_t stride = (uint32_t)(kvs * 4);
+    auto stage = [&](auto P) -> float* {
+        if constexpr (decltype(P)::value == 0) return sm0;
+        else return sm1;
+    };
+    // LDS slot of chunk c of row r: c ^ (r % 16) (16 rows of one chunk in 16 bank groups)
+    auto issue = [&](auto P, int st) {
+        float* sk = stage(P);
+        float* sv = sk + KS * D;
+#pragma unroll
+        for (int i = 0; i < LP; i++) {
+            const int p = wave * LP + i, r = p * RPP + lane / CPR;
+            const int c = (lane % CPR) ^ (r & 15);
+            const int key = st * KS + r < total ? st * KS + r : total - 1;
+            const uint32_t off = (uint32_t)key * stride + (uint32_t)c * 16;
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, sk + p * 256, 16, off, 0, 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rv, sv + p * 256, 16, off, 0, 0, 0);
+        }
+    };
+
+    constexpr auto P0 = std::integral_constant<int, 0>{};
+    constexpr auto P1 = std::integral_constant<int, 1>{};
+    if (st0 < st1) issue(P0, st0);
+    f4 qf[D / 8];
+#pragma unroll
+    for (int j = 0; j < D / 8; j++) qf[j] = *reinterpret_cast<const f4*>(q + q_off + hb * (D / 2) + 4 * j);
+    float m = -1e30f, l = 0.0f;
+    f16v o[DE];
+#pragma unroll
+    for (int e = 0; e < DE; e++) o[e] = f16v{};
+
+    auto step = [&](auto P, auto PN, int st) {
+        wait_vmcnt<0>();
+        lds_barrier();  // stage st in LDS for every wave; every wave is done with stage st - 1
+        if (st + 1 < st1) issue(PN, st + 1);
+        const int k0 = st * KS + kg * 32;
+        if (k0 >= wmax) return;
+        const float* sk = stage(P) + kg * 32 * D;
+        const float* sv = sk + KS * D;
+        f16v s = f16v{};
+#pragma unroll
+        for (int j = 0; j < D / 8; j++) {
+            const f4 kf = *reinterpret_cast<const f4*>(sk + ln * D + (((hb * (CPR / 2) + j) ^ (ln & 15)) * 4));
+#pragma unroll
+            for (int w = 0; w < 4; w++) s = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[w], qf[j][w], s, 0, 0, 0);
+        }
+        if (k0 + 32 > wmin) {  // keys past some row's last visible one
+#pragma unroll
+            for (int i = 0; i < 16; i++)
+                if (k0 + 8 * (i / 4) + 4 * hb + i % 4 >= lim) s[i] = -INFINITY;
+        }
+        float mx = s[0];
+#pragma unroll
+        for (int i = 1; i < 16; i++) mx = fmaxf(mx, s[i]);
+        mx = max_x32(mx) * scale_log2;
+        const bool up = mx > m;
+        if (__any(up)) {
+            const float mn = up ? mx : m, corr = __builtin_amdgcn_exp2f(m - mn);
+            m = mn;
+            l *= corr;
+#pragma unroll
+            for (int e = 0; e < DE; e++) o[e] *= corr;
+        }
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            // a masked score is -inf; its low part would make it NaN (-inf + inf) when scale_lo < 0
+            const float x = __builtin_fmaf(s[i], scale_log2, -m);
+            const float p = __builtin_amdgcn_exp2f(s[i] > -INFINITY ? __builtin_fmaf(s[i], scale_lo, x) : x);
+            l += p;
+            const int r = 8 * (i / 4) + 4 * hb + i % 4;
+            // dims DE ln .. + DE - 1 of V row r
+            const fe vf = *reinterpret_cast<const fe*>(sv + r * D + ((ln * DE / 4) ^ (r & 15)) * 4 + (ln * DE) % 4);
+#pragma unroll
+            for (int e = 0; e < DE; e++) o[e] = __builtin_amdgcn_mfma_f32_32x32x2f32(vf[e], p, o[e], 0, 0, 0);
+        }
+    };
+    for (int st = st0; st < st1; st += 2) {
+        step(P0, P1, st);
+        if (st + 1 < st1) step(P1, P0, st + 1);
+    }
+    l = sum_x32(l);
+
+    lds_barrier();  // every wave is done with the stages
+    // wave w's O rows of D floats, two waves per stage, 16-byte chunk c of row r at slot c ^ (r % 16)
+    auto os = [&](int w, int r, int c) {
+        return reinterpret_cast<f4*>((w < 2 ? sm0 : sm1) + (w & 1) * 32 * D) + r * (D / 4) + (c ^ (r & 15));
+    };
+    if (hb == 0) {
+        wm[wave][ln] = m;
+        wl[wave][ln] = l;
+    }
+    if (tid < ROWS) bad[tid] = 0;
+#pragma unroll
+    for (int i = 0; i < 16; i += 4 / DE) {
+        // DE consecutive dims per accumulator index: 4 / DE indices make a chunk
+        const int d = DE * (8 * (i / 4) + 4 * hb + i % 4);
+        f4 w;
+#pragma unroll
+        for (int j = 0; j < 4 / DE; j++)
+#pragma unroll
+            for (int e = 0; e < DE; e++) w[DE * j + e] = o[e][i + j];
+        *os(wave, ln, d / 4) = w;
+    }
+    __syncthreads();
+    auto row_off = [&](int r) {
+        const int s_ = r / G;
+        return ((int64_t)s_ * H + (int64_t)kvh * G + (r - s_ * G)) * D;
+    };
+    const int64_t pr0 = ((int64_t)blockIdx.y * KVH + kvh) * R + r0;
+    f4* wo = reinterpret_cast<f4*>(ws);
+    float2* wml = reinterpret_cast<float2*>(ws + (int64_t)ns * KVH * R * D);
+    for (int idx = tid; idx < ROWS * (D / 4); idx += 256) {
+        const int rr = idx / (D / 4), c = idx % (D / 4);
+        if (r0 + rr >= R) break;
+        const int w0 = rr / 32, ri = rr & 31;
+        float M = wm[w0][ri];
+#pragma unroll
+        for (int g = 1; g < KG; g++) M = fmaxf(M, wm[w0 + g * RG][ri]);
+        f4 num = f4{0.0f, 0.0f, 0.0f, 0.0f};
+        float den = 0.0f;
+#pragma unroll
+        for (int g = 0; g < KG; g++) {
+            const float f = __builtin_amdgcn_exp2f(wm[w0 + g * RG][ri] - M);
+            num += f * *os(w0 + g * RG, ri, c);
+            den += f * wl[w0 + g * RG][ri];
+        }
+        if (ns == 1) {
+            f4 y;
+            bool nf = false;
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                y[j] = num[j] / den;
+                nf = nf || !(__builtin_fabsf(y[j]) <= 3.4e38f);
+            }
+            if (nf) bad[rr] = 1;
+            *reinterpret_cast<f4*>(out + row_off(r0 + rr) + 4 * c) = y;
+        } else {
+            wo[(pr0 + rr) * (D / 4) + c] = num;
+            if (c == 0) wml[pr0 + rr] = make_float2(M, den);
+        }
+    }
+    if (ns > 1) return;  // k_attention_prefill_merge finishes the rows
+    __syncthreads();
+    for (int rr = wave; rr < ROWS; rr += 4) {
+        if (r0 + rr >= R) break;
+        if (!__builtin_amdgcn_readfirstlane(bad[rr])) continue;  // always, with finite inputs
+        const int64_t off = row_off(r0 + rr);
+        attn_row_general<float, D>(q + off, kh, vh, kvs, len0 + (r0 + rr) / G, scale, out + off, lane);
     }
 }
 
 // The rows of a call whose keys were split over ns blocks: a wave per row sums
 // the splits' numerators and denominators under their common maximum, in order.
-template <int D>
-__global__ __launch_bounds__(256) void k_attention_prefill_merge(const f16* __restrict__ q, const f16* __restrict__ k,
-                                                                 const f16* __restrict__ v, int32_t n_q, int32_t len0,
+template <typename T, int D>
+__global__ __launch_bounds__(256) void k_attention_prefill_merge(const T* __restrict__ q, const T* __restrict__ k,
+                                                                 const T* __restrict__ v, int32_t n_q, int32_t len0,
                                                                  int32_t KVH, int32_t G, float scale, int32_t ns,
-                                                                 f16* __restrict__ out, const float* __restrict__ ws)
+                                                                 T* __restrict__ out, const float* __restrict__ ws)
 {
     constexpr int E = D / 64;
     const int lane = threadIdx.x & 63, R = n_q * G;
@@ -361,51 +576,62 @@ __global__ __launch_bounds__(256) void k_attention_prefill_merge(const f16* __re
     for (int e = 0; e < E; e++) {
         const float y = num[e] / den;
         nf = nf || !(__builtin_fabsf(y) <= 3.0e38f);
-        out[off + lane * E + e] = (f16)y;
+        out[off + lane * E + e] = (T)y;
     }
     if (__any(nf))  // not with finite inputs
-        attn_row_general<D>(q + off, k + (int64_t)kvh * D, v + (int64_t)kvh * D, (int64_t)KVH * D, len0 + s, scale,
+        attn_row_general<T, D>(q + off, k + (int64_t)kvh * D, v + (int64_t)kvh * D, (int64_t)KVH * D, len0 + s, scale,
                             out + off, lane);
 }
 
-// The tile kernel's calls: fp16, head_dim 64 or 128, 16-byte aligned q, K and
-// V and 8-byte aligned out (its loads and stores), byte offsets within one
-// kv head's K and V rows and row numbers in 31 bits, and a positive scale (it
-// takes the maximum before scaling).
+// The tile kernels' calls: head_dim 64 or 128, 16-byte aligned q, K and V and
+// 16-byte (fp16: 8-byte) aligned out (their loads and stores), byte offsets
+// within one kv head's K and V rows and row numbers in 31 bits, and a positive
+// scale (they take the maximum before scaling).
+// fp32 calls over fewer than 128 positions keep k_attention while its blocks,
+// one per head and query, fit the chip at once: a single stage here costs more
+// (graph replay: 38 queries, 12 heads of 128, 7.2 us against 13.6; 15, 24 of 64, 4.9
+// against 8.2; 7 queries after 360 positions, 14 of 64, 15.3 against 13.3).
 bool attention_prefill_ok(const void* out, const void* q, const void* k, const void* v, int64_t n_q, int64_t len0,
                           int64_t H, int64_t KVH, int64_t D, float scale, int dtype)
 {
-    return dtype == VVH_F16 && (D == 64 || D == 128) && scale > 0.0f && scale < INFINITY &&
+    const int64_t es = dtype == VVH_F16 ? 2 : 4;
+    if (dtype == VVH_F32 && len0 + n_q - 1 < 128 && n_q * H <= 2048) return false;
+    return (D == 64 || D == 128) && scale > 0.0f && scale < INFINITY &&
            ((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k) | reinterpret_cast<uintptr_t>(v)) & 15) == 0 &&
-           (reinterpret_cast<uintptr_t>(out) & 7) == 0 && n_q * (H / KVH) <= (1 << 30) &&
-           (len0 + n_q) * KVH * D * 2 < ((int64_t)1 << 31);
+           (reinterpret_cast<uintptr_t>(out) & (uintptr_t)(4 * es - 1)) == 0 && n_q * (H / KVH) <= (1 << 30) &&
+           (len0 + n_q) * KVH * D * es < ((int64_t)1 << 31);
 }
 
 // Rows per block (32: 4 waves, one 32-key group each; 64: 8 waves) and blocks
 // sharing a row block's keys, the least of a model of the call fitted to forced
-// choices (graph replay): a stage of 128 keys costs a block about 1.4 us with
-// either shape, and the call's time follows its longest block or, with more
-// blocks than fit the chip at once (one per CU at head_dim 128, two at 64),
-// their sum; a split call adds the merge's launch and its partials, written
-// and read at about 3 TB/s.  Measured, 32 rows / 64 rows, splits in brackets:
+// choices (graph replay): a stage of 128 keys costs a block about 1.4 us at
+// head_dim 128 and 1.1 at 64 with either shape, and the call's time follows its
+// longest block or, with more blocks than fit the chip at once (one per CU at
+// head_dim 128, two at 64), their sum; a split call adds the merge's launch and
+// its partials, written and read at about 1.5 TB/s.  Measured, 32 rows / 64 rows, splits in brackets:
 // 512 queries, 14 heads on 2 of 64: 7.7 / 9.2 us (2: 12.1 / 12.1); 2048, 12 on 2
 // of 128: 51.4 / 33.7; 500 after 3500 positions, same heads: 46.5 / 46.7 (2:
 // 53.1 / 33.8, 4: - / 40.1); 7 after 4000: 45.6 / 44.7 (8: 15.2 / 15.1); 256 from
 // the start: 9.0 / 10.7; 1500, 32 on 4 of 64: 31.3 / 28.1.
-AttnPrefillPlan attention_prefill_plan(int64_t n_q, int64_t len0, int64_t H, int64_t KVH, int64_t D, int64_t cus)
+AttnPrefillPlan attention_prefill_plan(int64_t n_q, int64_t len0, int64_t H, int64_t KVH, int64_t D, int dtype,
+                                       int64_t cus)
 {
-    const int64_t R = n_q * (H / KVH), slots = D == 64 ? 2 * cus : cus;
-    const int64_t longest = (len0 + n_q - 1 + 127) / 128;
-    const double mean = (double)(len0 + n_q / 2 + 127) / 128.0;
+    const bool f32 = dtype == VVH_F32;
+    const int64_t R = n_q * (H / KVH), slots = D == 64 && !f32 ? 2 * cus : cus;
+    const int64_t keys = f32 ? 8192 / D : 128;  // per stage
+    const int64_t longest = (len0 + n_q - 1 + keys - 1) / keys;
+    const double mean = (double)(len0 + n_q / 2 + keys - 1) / (double)keys;
+    const double stage_us = f32 ? (D == 64 ? 2.0 : 3.9) : (D == 64 ? 1.1 : 1.42);
     AttnPrefillPlan best{};
     double best_t = INFINITY;
     for (const int64_t rows : {32, 64}) {
+        if (f32 && rows != (D == 64 ? 32 : 64)) continue;  // 4 waves: 4 key groups, or 2 of each
         const int64_t blocks = (R + rows - 1) / rows * KVH;
         const int64_t smax = std::max<int64_t>(1, std::min<int64_t>({longest, slots / blocks, 32}));
         for (int64_t sp = 1; sp <= smax; sp++) {
             const double st = std::max((double)((longest + sp - 1) / sp), (double)blocks * mean / (double)slots);
-            double t = (rows == 32 ? 2.0 : 3.0) + 1.42 * st;
-            if (sp > 1) t += 3.0 + (double)(sp * n_q * H * (D + 2) * 8) / 3e6;
+            double t = (rows == 32 ? 2.0 : 3.0) + stage_us * st;
+            if (sp > 1) t += 5.0 + 0.1 * (double)sp + (double)(sp * n_q * H * (D + 2) * 8) / 1.5e6;
             if (t < best_t) {
                 best_t = t;
                 best = AttnPrefillPlan{rows, blocks, sp};
@@ -421,27 +647,36 @@ int64_t attention_prefill_ws_floats(const AttnPrefillPlan& p, int64_t n_q, int64
 }
 
 int launch_attention_prefill(const AttnPrefillPlan& p, void* out, const void* q, const void* k, const void* v,
-                             int64_t n_q, int64_t len0, int64_t H, int64_t KVH, int64_t D, float scale, float* ws,
-                             void* stream)
+                             int64_t n_q, int64_t len0, int64_t H, int64_t KVH, int64_t D, float scale, int dtype,
+                             float* ws, void* stream)
 {
-    const float sl = (float)((double)scale * 1.4426950408889634);
+    const double sd = (double)scale * 1.4426950408889634;
+    const float sl = (float)sd;
+    const dim3 grid((unsigned)p.blocks, (unsigned)p.splits), mgrid((unsigned)((n_q * H + 3) / 4));
+    const int32_t nq = (int32_t)n_q, l0 = (int32_t)len0, kvh = (int32_t)KVH, g = (int32_t)(H / KVH);
     hipStream_t s = static_cast<hipStream_t>(stream);
+    auto merge = [&]<typename T>(auto kern, T* o) {
+        if (p.splits > 1)
+            hipLaunchKernelGGL(kern, mgrid, dim3(256), 0, s, (const T*)q, (const T*)k, (const T*)v, nq, l0, kvh, g, scale,
+                               (int32_t)p.splits, o, ws);
+    };
+    if (dtype == VVH_F32) {
+        auto go = [&](auto kern) {
+            hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, (const float*)q, (const float*)k, (const float*)v, nq, l0, kvh,
+                               g, scale, sl, (float)(sd - (double)sl), (float*)out, ws);
+        };
+        D == 64 ? go(k_attention_prefill_f32<64, 1, 4>) : go(k_attention_prefill_f32<128, 2, 2>);
+        D == 64 ? merge(k_attention_prefill_merge<float, 64>, (float*)out)
+                : merge(k_attention_prefill_merge<float, 128>, (float*)out);
+        return (int)hipGetLastError();
+    }
     auto go = [&](auto kern) {
-        hipLaunchKernelGGL(kern, dim3((unsigned)p.blocks, (unsigned)p.splits), dim3(unsigned(8 * p.rows)), 0, s,
-                           (const f16*)q,
-                           (const f16*)k, (const f16*)v, (int32_t)n_q, (int32_t)len0, (int32_t)KVH, (int32_t)(H / KVH),
-                           scale, sl, (f16*)out, ws);
+        hipLaunchKernelGGL(kern, grid, dim3(unsigned(8 * p.rows)), 0, s, (const f16*)q, (const f16*)k, (const f16*)v, nq,
+                           l0, kvh, g, scale, sl, (f16*)out, ws);
     };
     if (D == 64) p.rows == 32 ? go(k_attention_prefill<64, 1>) : go(k_attention_prefill<64, 2>);
     else p.rows == 32 ? go(k_attention_prefill<128, 1>) : go(k_attention_prefill<128, 2>);
-    if (p.splits > 1) {
-        const dim3 grid((unsigned)((n_q * H + 3) / 4));
-        auto merge = [&](auto kern) {
-            hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, (const f16*)q, (const f16*)k, (const f16*)v, (int32_t)n_q,
-                               (int32_t)len0, (int32_t)KVH, (int32_t)(H / KVH), scale, (int32_t)p.splits, (f16*)out, ws);
-        };
-        D == 64 ? merge(k_attention_prefill_merge<64>) : merge(k_attention_prefill_merge<128>);
-    }
+    D == 64 ? merge(k_attention_prefill_merge<f16, 64>, (f16*)out) : merge(k_attention_prefill_merge<f16, 128>, (f16*)out);
     return (int)hipGetLastError();
 }
 

@@ -337,11 +337,12 @@ struct AttnPrefillPlan {
     int64_t blocks;  // row blocks of all kv heads
     int64_t splits;  // blocks that share a row block's keys (> 1: workspace and a merge launch)
 };
-AttnPrefillPlan attention_prefill_plan(int64_t n_q, int64_t len0, int64_t H, int64_t KVH, int64_t D, int64_t cus);
+AttnPrefillPlan attention_prefill_plan(int64_t n_q, int64_t len0, int64_t H, int64_t KVH, int64_t D, int dtype,
+                                       int64_t cus);
 int64_t attention_prefill_ws_floats(const AttnPrefillPlan& p, int64_t n_q, int64_t H, int64_t D);
 int launch_attention_prefill(const AttnPrefillPlan& p, void* out, const void* q, const void* k, const void* v,
-                             int64_t n_q, int64_t len0, int64_t H, int64_t KVH, int64_t D, float scale, float* ws,
-                             void* stream);
+                             int64_t n_q, int64_t len0, int64_t H, int64_t KVH, int64_t D, float scale, int dtype,
+                             float* ws, void* stream);
 // n_q = 1 fast path: grouped heads, split over the sequence into nb blocks
 // per kv head.  mfma: the fp16 matrix-core kernel (head_dim 64 or 128), which
 // merges the blocks in the same launch and, with nb > 1, needs a zeroed

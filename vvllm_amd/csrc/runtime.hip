@@ -2076,7 +2076,7 @@ VVH_API int vvh_attention(void* out, const void* q, const void* k, const void* v
     if (attention_prefill_ok(out, q, k, v, (int64_t)n_q, (int64_t)len0, (int64_t)num_heads, (int64_t)num_kv_heads,
                              (int64_t)head_dim, scale, dtype)) {
         AttnPrefillPlan p = attention_prefill_plan((int64_t)n_q, (int64_t)len0, (int64_t)num_heads,
-                                                   (int64_t)num_kv_heads, (int64_t)head_dim,
+                                                   (int64_t)num_kv_heads, (int64_t)head_dim, dtype,
                                                    g_cu_count > 0 ? g_cu_count : 256);
         // splits need the stream's workspace; without it (a capture that
         // cannot allocate, no memory) each block takes all its keys
@@ -2084,7 +2084,7 @@ VVH_API int vvh_attention(void* out, const void* q, const void* k, const void* v
         const int64_t wsf = attention_prefill_ws_floats(p, (int64_t)n_q, (int64_t)num_heads, (int64_t)head_dim);
         if (wsf > 0 && !workspace_try(stream, (std::size_t)wsf * 4, &ws)) p.splits = 1;
         return ret_launch(launch_attention_prefill(p, out, q, k, v, (int64_t)n_q, (int64_t)len0, (int64_t)num_heads,
-                                                   (int64_t)num_kv_heads, (int64_t)head_dim, scale, ws, stream),
+                                                   (int64_t)num_kv_heads, (int64_t)head_dim, scale, dtype, ws, stream),
                           "attention launch");
     }
     return ret_launch(launch_attention(out, q, k, v, (int64_t)n_q, (int64_t)len0, (int64_t)num_heads,
