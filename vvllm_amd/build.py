@@ -30,7 +30,7 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 CXX = os.environ.get("CXX", "g++")
 
 HIP_SOURCES = ["runtime.hip", "linear_kernels.hip", "gemm_kernels.hip", "model_kernels.hip", "attention_kernels.hip",
-               "aux_kernels.hip"]
+               "dense_kernels.hip", "aux_kernels.hip"]
 HIP_FLAGS = [
     "--offload-arch=gfx950",
     "-O3",

@@ -373,6 +373,18 @@ int launch_zero_u32(unsigned* p, int64_t n, void* stream);
 int launch_copy2(void* d0, const void* s0, void* d1, const void* s1, int64_t bytes, void* stream);
 int launch_dense(void* out, const void* x, const void* w, int wdtype, const float* bias, const void* res, int64_t M,
                  int64_t N, int64_t K, int dtype, void* stream);
+// The matrix-core form for more than 4 rows (dense_kernels.hip): whether it
+// serves a call, its tiles and k splits on a device of `cus` CUs, and its launch
+// (ws: dense_ws_floats() floats when splits > 1).
+struct DensePlan {
+    int64_t bm;      // rows of a block tile
+    int64_t splits;
+};
+bool dense_mfma_ok(const void* x, const void* w, int wdtype, int64_t M, int64_t N, int64_t K, int dtype);
+DensePlan dense_plan(int64_t M, int64_t N, int64_t K, int dtype, int64_t cus);
+int64_t dense_ws_floats(const DensePlan& p, int64_t M, int64_t N);
+int launch_dense_mfma(const DensePlan& p, void* out, const void* x, const void* w, const float* bias, const void* res,
+                      int64_t M, int64_t N, int64_t K, int dtype, float* ws, void* stream);
 int launch_matmul(void* out, const void* A, const float* B, int64_t M, int64_t N, int64_t K, int dtype, void* stream);
 // ws: argmax_ws_bytes(n) bytes (none for n <= 2048)
 int64_t argmax_ws_bytes(int64_t n);

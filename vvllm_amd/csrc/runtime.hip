@@ -2132,6 +2132,16 @@ VVH_API int vvh_dense(void* out, const void* x, const void* dev_weight, int wdty
     if (!out || (K > 0 && (!x || !dev_weight))) return fail(VVH_ERR_INVALID_ARG, "null pointer");
     if ((N + 3) / 4 > INT32_MAX) return fail(VVH_ERR_UNSUPPORTED, "N too large");
     REQUIRE_INIT();
+    if (dense_mfma_ok(x, dev_weight, wdtype, (int64_t)M, (int64_t)N, (int64_t)K, dtype)) {
+        DensePlan p = dense_plan((int64_t)M, (int64_t)N, (int64_t)K, dtype, g_cu_count > 0 ? g_cu_count : 256);
+        // k splits need the stream's workspace; without it one block takes all of a tile's k
+        float* ws = nullptr;
+        const int64_t wsf = dense_ws_floats(p, (int64_t)M, (int64_t)N);
+        if (wsf > 0 && !workspace_try(stream, (std::size_t)wsf * 4, &ws)) p.splits = 1;
+        return ret_launch(launch_dense_mfma(p, out, x, dev_weight, dev_bias, residual, (int64_t)M, (int64_t)N, (int64_t)K,
+                                            dtype, ws, stream),
+                          "dense launch");
+    }
     return ret_launch(launch_dense(out, x, dev_weight, wdtype, dev_bias, residual, (int64_t)M, (int64_t)N, (int64_t)K,
                                    dtype, stream),
                       "dense launch");
