@@ -1,0 +1,105 @@
+"""Plans that run as one grouped launch: problems that share their activations
+on the GEMM (q/k/v, gate and up of a prompt; fp16, and fp32 split into fp16
+halves once), and fp32 decode problems.  Against 64-bit sums, at group sizes
+2-4, column counts that are no multiple of a tile or of 8, row counts at the
+edges of the tiles and of the dispatch, k split or not; and in a captured graph
+replayed between eager runs.
+
+Tolerance per element: one rounding to the output type, the fp32 sums (no
+product passes through more than K / 8 additions of partial sums of at most
+sum |x w|, scaled), and for split fp32 activations 2^-21 of each |x w|.
+"""
+import ctypes
+
+import numpy as np
+import pytest
+
+from vvllm_amd import capi
+
+pytestmark = pytest.mark.gpu
+
+F16, F32 = capi.F16, capi.F32
+
+
+def npd(d):
+    return np.float32 if d == F32 else np.float16
+
+
+def build(rng, M, Ns, K, d, same_x=True):
+    dev, probs, refs = [], [], []
+    x = rng.normal(0, 1, (M, K)).astype(npd(d))
+    dx = capi.DevBuf.from_array(x)
+    for i, N in enumerate(Ns):
+        q = rng.integers(-127, 128, (N, K)).astype(np.int8)
+        s = rng.uniform(1e-4, 3e-4, N).astype(np.float32)
+        b = rng.normal(0, 1, N).astype(np.float32) if i % 2 == 0 else None
+        r = rng.normal(0, 1, (M, N)).astype(npd(d)) if i == 1 else None
+        xi, dxi = (x, dx) if same_x else (lambda a: (a, capi.DevBuf.from_array(a)))(rng.normal(0, 1, (M, K)).astype(npd(d)))
+        do = capi.DevBuf(M * N * x.itemsize)
+        bufs = [capi.DevBuf.from_array(a) if a is not None else None for a in (q, s, b, r)]
+        dev += bufs + [do, dxi]
+        p = [t.ptr if t is not None else None for t in bufs]
+        probs.append(capi.Q8Problem(out=do.ptr, inp=dxi.ptr, residual=p[3], weight=p[0], scales=p[1], bias=p[2], M=M, N=N,
+                                    K=K))
+        w = q.astype(np.float64) * s[:, None].astype(np.float64)
+        y, mag = xi.astype(np.float64) @ w.T, np.abs(xi).astype(np.float64) @ np.abs(w).T
+        for t in (b, r):
+            if t is not None:
+                y, mag = y + t, mag + np.abs(t)
+        refs.append((do, y, mag))
+    h = ctypes.c_uint64()
+    capi.call("vvh_plan_create", (capi.Q8Problem * len(Ns))(*probs), len(Ns), d, d, ctypes.byref(h))
+    return h.value, refs, dev
+
+
+def check(refs, M, K, d):
+    for do, y, mag in refs:
+        got = do.to_array(npd(d), y.shape).astype(np.float64)
+        ulp = 2.0 ** -11 if d == F16 else 2.0 ** -24
+        assert (np.abs(got - y) <= ulp * np.abs(y) + (K / 8 * 2.0 ** -24 + (2.0 ** -21 if d == F32 else 0)) * mag).all()
+
+
+def launches(plan):
+    n = ctypes.c_int()
+    capi.call("vvh_plan_launches", plan, ctypes.byref(n))
+    return n.value
+
+
+GEMM = [(17, (896, 128, 128), 896), (33, (200, 72), 512), (64, (256, 256, 1536), 1536), (130, (100, 129, 64, 1000), 576),
+        (333, (896, 128, 128), 896), (512, (4864, 4864), 896), (700, (1536, 256, 256), 1536), (1500, (8960, 8960), 256),
+        (40, (128, 64), 8960)]
+
+
+@pytest.mark.parametrize("d", [F32, F16])
+@pytest.mark.parametrize("M,Ns,K", GEMM)
+def test_gemm_group(gpu, M, Ns, K, d):
+    print(f"[case] gemm group M={M} N={Ns} K={K} dtype={d}", flush=True)
+    plan, refs, dev = build(np.random.default_rng(M + K), M, Ns, K, d)
+    assert launches(plan) == 1
+    for _ in range(2):
+        capi.call("vvh_plan_run", plan, None)
+    capi.sync()
+    check(refs, M, K, d)
+    capi.call("vvh_plan_destroy", plan)
+
+
+@pytest.mark.parametrize("M,Ns,K,same_x", [(1, (896, 128, 128), 896, True), (1, (4864, 4864), 896, False),
+                                           (3, (100, 17, 16, 33), 4864, False), (15, (896, 128), 1000 - 8, True),
+                                           (20, (64, 48), 208, True)])
+def test_gemv_f32_group(gpu, M, Ns, K, same_x):
+    print(f"[case] gemv group M={M} N={Ns} K={K}", flush=True)
+    plan, refs, dev = build(np.random.default_rng(M + K), M, Ns, K, F32, same_x)
+    assert launches(plan) == 1
+    capi.call("vvh_plan_run", plan, None)
+    capi.sync()
+    check(refs, M, K, F32)
+    capi.call("vvh_plan_destroy", plan)
+
+
+def test_different_inputs_run_one_by_one(gpu):
+    plan, refs, dev = build(np.random.default_rng(9), 100, (128, 192), 512, F16, same_x=False)
+    assert launches(plan) == 2
+    capi.call("vvh_plan_run", plan, None)
+    capi.sync()
+    check(refs, 100, 512, F16)
+    capi.call("vvh_plan_destroy", plan)

@@ -133,29 +133,31 @@ __global__ __launch_bounds__(256) void k_fill_normal(T* __restrict__ d, int64_t 
 
 // ---------------------------------------------------------------------------
 // fp32 activations for the fp16 MFMA GEMM: row m of x [M, K] becomes row m of
-// xs [M, 2K] fp16, the high parts hi_k = fp16(x_k * s) followed by the low
-// parts lo_k = fp16(x_k * s - hi_k), with s = 2^p chosen per row so that the
+// xs [M, 2K] fp16, the low parts lo_k = fp16(x_k * s - hi_k) followed by the high
+// parts hi_k = fp16(x_k * s), with s = 2^p chosen per row so that the
 // row's largest |x| * s lies in [2^14, 2^15) (in range for fp16 with room for
 // its 11-bit significand), and rs[m] = 1/s.  x_k * s is exact (a power of
 // two), x_k * s - hi_k is exact (Sterbenz), so hi + lo carries x_k * s to
 // about 22 bits (or to the fp16 subnormal step 2^-24 of the scaled row); the
 // int8 x fp16 products of both parts are exact in the GEMM's fp32
-// accumulation.  A row without a finite nonzero maximum (all zeros, or
+// accumulation.  The low parts come first: while their sum grows it is small,
+// and so are its roundings; after the high parts each would round the whole
+// sum (error against 64 bits of unsplit calls: K = 896 3.1e-7 -> 1.6e-7).
+// A row without a finite nonzero maximum (all zeros, or
 // containing Inf or NaN) keeps s = 1, so Inf and NaN reach the sums as such.
-// One block per row.
+// One block per row, read once: C chunks of 4 values per thread (K % 4 == 0,
+// 16-byte aligned rows), or two passes.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_split_f32(const float* __restrict__ x, int64_t K, f16* __restrict__ xs,
-                                                   float* __restrict__ rs)
+__device__ __forceinline__ float split_max(float mx, float x)
 {
-    __shared__ float part[4];
-    const int64_t m = blockIdx.x;
-    const float* xr = x + m * K;
-    float mx = 0.0f;
     // an Inf or NaN anywhere in the row makes the row maximum Inf
-    for (int64_t k = threadIdx.x; k < K; k += 256) {
-        const float v = __builtin_fabsf(xr[k]);
-        mx = __builtin_isfinite(v) ? fmaxf(mx, v) : __builtin_inff();
-    }
+    const float v = __builtin_fabsf(x);
+    return __builtin_isfinite(v) ? fmaxf(mx, v) : __builtin_inff();
+}
+
+// The row's scale s = 2^p from the threads' maxima; rs = 1/s.
+__device__ __forceinline__ float split_scale(float mx, float* part, float* rs)
+{
     for (int off = 32; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off));
     if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = mx;
     __syncthreads();
@@ -167,22 +169,81 @@ __global__ __launch_bounds__(256) void k_split_f32(const float* __restrict__ x, 
         p = 15 - e;                    // mx * 2^p in [2^14, 2^15)
         p = p < -126 ? -126 : (p > 126 ? 126 : p);
     }
-    const float s = ldexpf(1.0f, p);
-    if (threadIdx.x == 0) rs[m] = ldexpf(1.0f, -p);
-    f16* hr = xs + m * 2 * K;
-    for (int64_t k = threadIdx.x; k < K; k += 256) {
-        const float v = xr[k] * s;
-        const f16 hi = (f16)v;
-        hr[k] = hi;
-        hr[K + k] = __builtin_isfinite((float)hi) ? (f16)(v - (float)hi) : (f16)0.0f;
+    if (threadIdx.x == 0) *rs = ldexpf(1.0f, -p);
+    return ldexpf(1.0f, p);
+}
+
+__device__ __forceinline__ void split_parts(float v, f16& hi, f16& lo)
+{
+    hi = (f16)v;
+    lo = __builtin_isfinite((float)hi) ? (f16)(v - (float)hi) : (f16)0.0f;
+}
+
+__global__ __launch_bounds__(256) void k_split_f32(const float* __restrict__ x, int64_t K, f16* __restrict__ xs,
+                                                   float* __restrict__ rs)
+{
+    __shared__ float part[4];
+    const int64_t m = blockIdx.x;
+    const float* xr = x + m * K;
+    float mx = 0.0f;
+    for (int64_t k = threadIdx.x; k < K; k += 256) mx = split_max(mx, xr[k]);
+    const float s = split_scale(mx, part, rs + m);
+    f16* lr = xs + m * 2 * K;
+    for (int64_t k = threadIdx.x; k < K; k += 256) split_parts(xr[k] * s, lr[K + k], lr[k]);
+}
+
+template <int C>
+__global__ __launch_bounds__(256) void k_split_f32_rows(const float* __restrict__ x, int32_t K, f16* __restrict__ xs,
+                                                        float* __restrict__ rs)
+{
+    typedef float f4 __attribute__((ext_vector_type(4)));
+    typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+    __shared__ float part[4];
+    const int64_t m = blockIdx.x;
+    const f4* xr = reinterpret_cast<const f4*>(x + m * K);
+    const int kc = K / 4;
+    f4 v[C];
+#pragma unroll
+    for (int c = 0; c < C; c++) {
+        const int i = threadIdx.x + 256 * c;
+        v[c] = xr[i < kc ? i : kc - 1];  // past the row: its last chunk again
+    }
+    float mx = 0.0f;
+#pragma unroll
+    for (int c = 0; c < C; c++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) mx = split_max(mx, v[c][e]);
+    const float s = split_scale(mx, part, rs + m);
+    f16* lr = xs + m * 2 * K;
+#pragma unroll
+    for (int c = 0; c < C; c++) {
+        const int i = threadIdx.x + 256 * c;
+        if (i >= kc) continue;
+        h4 hi, lo;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            f16 h, l;
+            split_parts(v[c][e] * s, h, l);
+            hi[e] = h;
+            lo[e] = l;
+        }
+        *reinterpret_cast<h4*>(lr + 4 * i) = lo;
+        *reinterpret_cast<h4*>(lr + K + 4 * i) = hi;
     }
 }
 
 int launch_split_f32(const float* x, int64_t M, int64_t K, void* xs, float* rs, void* stream)
 {
     if (M <= 0) return 0;
-    hipLaunchKernelGGL(k_split_f32, dim3((unsigned)M), dim3(256), 0, static_cast<hipStream_t>(stream), x, K,
-                       static_cast<f16*>(xs), rs);
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    const dim3 grid((unsigned)M);
+    f16* o = static_cast<f16*>(xs);
+    const bool rows = K % 4 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(xs) % 8 == 0;
+    if (rows && K <= 1024) hipLaunchKernelGGL(k_split_f32_rows<1>, grid, dim3(256), 0, s, x, (int32_t)K, o, rs);
+    else if (rows && K <= 2048) hipLaunchKernelGGL(k_split_f32_rows<2>, grid, dim3(256), 0, s, x, (int32_t)K, o, rs);
+    else if (rows && K <= 5120) hipLaunchKernelGGL(k_split_f32_rows<5>, grid, dim3(256), 0, s, x, (int32_t)K, o, rs);
+    else if (rows && K <= 9216) hipLaunchKernelGGL(k_split_f32_rows<9>, grid, dim3(256), 0, s, x, (int32_t)K, o, rs);
+    else hipLaunchKernelGGL(k_split_f32, grid, dim3(256), 0, s, x, K, o, rs);
     return (int)hipGetLastError();
 }
 

@@ -69,7 +69,7 @@ struct LinArgs {
     // each and out gets M rows of N / 2 values silu(gate) * up
     int32_t glu;
     // fp32 activations on the GEMM: inp holds M rows of 2 * bk fp16 values
-    // (K = 2 * bk), the high and low fp16 parts of each fp32 activation
+    // (K = 2 * bk), the low and then the high fp16 parts of each fp32 activation
     // scaled by a power of two, and xrs[m] = that row's inverse scale; the
     // codes have rows of bk (0: K).
     int64_t bk;
@@ -81,6 +81,14 @@ struct LinArgs {
 constexpr int kDotInline = 4;
 struct DotGroup {
     LinArgs p[kDotInline];
+};
+// Grouped GEMM and grouped fp32 decode launches: problem i takes the blocks
+// [p[i].block_begin, p[i + 1].block_begin); b[i] = p[i + 1].block_begin, INT32_MAX
+// past the last problem.
+struct LinGroup {
+    DotGroup g;
+    int32_t b[kDotInline - 1];
+    int32_t blocks;
 };
 
 // Persistent streaming decode launch (k_stream).  Work is a sequence of
@@ -281,6 +289,8 @@ int linear_dev(void* out, const void* inp, const int8_t* w, const float* scales,
 // Launchers (linear_kernels.hip).  Return a hipError_t value as int.
 int launch_generic(const LinArgs& a, int act, int out, void* stream);
 int launch_gemv_f32(const LinArgs& a, int out, void* stream);
+// the problems of a group (one M) in one launch
+int launch_gemv_f32_group(const LinGroup& g, int out, void* stream);
 int launch_skinny(const LinArgs& a, int out, void* stream);
 int launch_skinny_grouped(const LinArgs* dev_table, int count, int64_t total_blocks, int out,
                           void* stream);
@@ -302,8 +312,12 @@ int launch_gemm(const LinArgs& a, int out, void* stream);
 int gemm3_tile_n(int layout);
 int gemm3_tile_m(int layout);
 int launch_gemm3(const LinArgs& a, int out, int layout, void* stream);
+// the problems of a group (one layout, nsplit and kstages) in one launch
+int launch_gemm3_group(const LinGroup& g, int out, int layout, void* stream);
 // sum of the a.nsplit partials in a.ws + epilogue (scale, bias, residual)
 int launch_splitk_reduce(const LinArgs& a, int out, void* stream);
+// the same for `count` problems of one M and nsplit
+int launch_splitk_reduce_group(const LinGroup& g, int count, int out, void* stream);
 // depth = weight loads in flight per lane (8 or 12); every problem must have
 // at least `depth` 64-wide k steps.  max_m = largest M of the launch.
 int launch_stream(const StreamArgs& s, int depth, int max_m, int out, int64_t blocks, void* stream);
@@ -401,7 +415,7 @@ int launch_convert(void* dst, int dst_dtype, const void* src, int src_dtype, int
                    void* stream);
 int launch_fill_normal(void* dst, int dtype, int64_t n, uint64_t seed, float mean, float std,
                        void* stream);
-// fp32 rows x [M, K] -> xs [M, 2K] fp16 (scaled high parts, then low parts)
+// fp32 rows x [M, K] -> xs [M, 2K] fp16 (scaled low parts, then high parts)
 // and rs [M] (inverse scales), the activations of an fp32 call on the GEMM
 int launch_split_f32(const float* x, int64_t M, int64_t K, void* xs, float* rs, void* stream);
 

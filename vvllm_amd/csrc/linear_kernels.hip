@@ -26,6 +26,7 @@
 
 #include <algorithm>
 #include <cstdlib>
+#include <type_traits>
 #include <utility>
 
 #include "common.h"
@@ -188,6 +189,15 @@ template <int MT, typename OT>
 __global__ __launch_bounds__(256) void k_gemv_f32(LinArgs a)
 {
     gemv_f32_body<MT, OT>(a, blockIdx.x, (int64_t)blockIdx.y * MT);
+}
+
+// The problems of a plan (q, k and v of a decode layer) in one launch.
+template <int MT, typename OT>
+__global__ __launch_bounds__(256) void k_gemv_f32_group(LinGroup l)
+{
+    const int b = blockIdx.x;
+    const LinArgs a = l.g.p[(b >= l.b[0]) + (b >= l.b[1]) + (b >= l.b[2])];
+    gemv_f32_body<MT, OT>(a, b - a.block_begin, (int64_t)blockIdx.y * MT);
 }
 
 // ---------------------------------------------------------------------------
@@ -1649,9 +1659,12 @@ __global__ __launch_bounds__(256) void k_splitk_reduce(LinArgs a)
 // in order; the group sums are added in group order through LDS.  The
 // result is ((sum of group 0) + sum of group 1) + ..., the same on every
 // run for a given split count.
-template <typename OT, int GR>
-__global__ __launch_bounds__(256) void k_splitk_reduce8(LinArgs a)
+template <typename OT, int GR, typename A = LinArgs>
+__global__ __launch_bounds__(256) void k_splitk_reduce8(A args)
 {
+    LinArgs a;
+    if constexpr (std::is_same_v<A, LinGroup>) a = args.g.p[blockIdx.y];  // one problem per grid row
+    else a = args;
     constexpr int G = 8;
     constexpr int CPB = 256 / GR;  // chunks per block, a multiple of 64: groups are whole waves
     __shared__ f4 part[GR > 1 ? GR - 1 : 1][CPB][2];
@@ -1767,13 +1780,52 @@ static void reduce8_go(const LinArgs& a, hipStream_t s)
     else hipLaunchKernelGGL((k_splitk_reduce8<OT, 1>), grid, dim3(256), 0, s, a);
 }
 
+static bool reduce8_ok(const LinArgs& a)
+{
+    return a.N % 8 == 0 && reinterpret_cast<uintptr_t>(a.out) % 16 == 0 &&
+           (!a.res || reinterpret_cast<uintptr_t>(a.res) % 16 == 0) &&
+           reinterpret_cast<uintptr_t>(a.scales) % 16 == 0 && (!a.bias || reinterpret_cast<uintptr_t>(a.bias) % 16 == 0);
+}
+
+template <typename OT>
+static void reduce8_group_go(const LinGroup& g, int count, int64_t M, int64_t n_sum, int64_t n_max, int32_t nsplit,
+                             hipStream_t s)
+{
+    const int gr = splitk_reduce_groups(M, n_sum, nsplit);
+    const int64_t chunks = M * (n_max / 8), cpb = 256 / gr;
+    const dim3 grid((unsigned)((chunks + cpb - 1) / cpb), (unsigned)count);
+    if (gr == 4) hipLaunchKernelGGL((k_splitk_reduce8<OT, 4, LinGroup>), grid, dim3(256), 0, s, g);
+    else if (gr == 2) hipLaunchKernelGGL((k_splitk_reduce8<OT, 2, LinGroup>), grid, dim3(256), 0, s, g);
+    else hipLaunchKernelGGL((k_splitk_reduce8<OT, 1, LinGroup>), grid, dim3(256), 0, s, g);
+}
+
+int launch_splitk_reduce_group(const LinGroup& g, int count, int out, void* stream)
+{
+    int64_t n_sum = 0, n_max = 0;
+    bool ok = true;
+    for (int i = 0; i < count; i++) {
+        ok = ok && reduce8_ok(g.g.p[i]);
+        n_sum += g.g.p[i].N;
+        n_max = std::max(n_max, g.g.p[i].N);
+    }
+    if (!ok) {
+        for (int i = 0; i < count; i++) {
+            const int e = launch_splitk_reduce(g.g.p[i], out, stream);
+            if (e != 0) return e;
+        }
+        return 0;
+    }
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    const LinArgs& a = g.g.p[0];
+    if (out == VVH_F32) reduce8_group_go<float>(g, count, a.M, n_sum, n_max, a.nsplit, s);
+    else reduce8_group_go<f16>(g, count, a.M, n_sum, n_max, a.nsplit, s);
+    return (int)hipGetLastError();
+}
+
 int launch_splitk_reduce(const LinArgs& a, int out, void* stream)
 {
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const bool vec = a.N % 8 == 0 && reinterpret_cast<uintptr_t>(a.out) % 16 == 0 &&
-                     (!a.res || reinterpret_cast<uintptr_t>(a.res) % 16 == 0) &&
-                     reinterpret_cast<uintptr_t>(a.scales) % 16 == 0 &&
-                     (!a.bias || reinterpret_cast<uintptr_t>(a.bias) % 16 == 0);
+    const bool vec = reduce8_ok(a);
     if (vec) {
         if (out == VVH_F32) reduce8_go<float>(a, s);
         else reduce8_go<f16>(a, s);
@@ -1807,6 +1859,26 @@ static void gemv_f32_launch(const LinArgs& a, int out, dim3 grid, hipStream_t s)
 {
     if (out == VVH_F32) hipLaunchKernelGGL((k_gemv_f32<MT, float>), grid, dim3(256), 0, s, a);
     else hipLaunchKernelGGL((k_gemv_f32<MT, f16>), grid, dim3(256), 0, s, a);
+}
+
+template <int MT>
+static void gemv_f32_group_launch(const LinGroup& l, int out, dim3 grid, hipStream_t s)
+{
+    if (out == VVH_F32) hipLaunchKernelGGL((k_gemv_f32_group<MT, float>), grid, dim3(256), 0, s, l);
+    else hipLaunchKernelGGL((k_gemv_f32_group<MT, f16>), grid, dim3(256), 0, s, l);
+}
+
+int launch_gemv_f32_group(const LinGroup& l, int out, void* stream)
+{
+    const int64_t M = l.g.p[0].M, mt = M <= 1 ? 1 : M <= 2 ? 2 : M <= 4 ? 4 : 8;
+    const dim3 grid((unsigned)l.blocks, (unsigned)((M + mt - 1) / mt));
+    switch (mt) {
+        case 1: gemv_f32_group_launch<1>(l, out, grid, S(stream)); break;
+        case 2: gemv_f32_group_launch<2>(l, out, grid, S(stream)); break;
+        case 4: gemv_f32_group_launch<4>(l, out, grid, S(stream)); break;
+        default: gemv_f32_group_launch<8>(l, out, grid, S(stream)); break;
+    }
+    return (int)hipGetLastError();
 }
 
 int launch_gemv_f32(const LinArgs& a, int out, void* stream)

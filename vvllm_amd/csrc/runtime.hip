@@ -106,6 +106,7 @@ struct Plan {
     int depth = 0;
     int dot_depth = 4;           // k_dot_grouped ring depth: the largest dot_depth of the problems
     int max_m = 0;
+    int group = 0;               // kGroupGemm or kGroupGemv: one launch of a plan that is none of the above
     void* dev_stream = nullptr;  // tile_prob, list, list_off
     float* rope_freq = nullptr;  // RoPE epilogue: the pair frequencies of the q and k rows
     float* rope_cs = nullptr;    // RoPE epilogue: cosine and sine of positions [0, rope_cs_n)
@@ -284,20 +285,23 @@ int workspace_get(const WsSource* src, void* stream, std::size_t bytes, float** 
 // 8.64; where 64 x 64 would halve the count (down at M = 512: 4 -> 2 splits,
 // 16.83 -> 17.72 us; 1.5B down at M = 256: 19.79 -> 24.91) the model keeps
 // 64 x 128.  *split_layout: the tile layout of a split call (4 or 5).
-int gemm_splits(int64_t M, int64_t N, int64_t stages, int* split_layout)
+// (A group of problems of one M counts their tiles and planes together:
+// tiles_of(bm, bn), n their sum of N.)
+template <typename Tiles>
+int gemm_splits(int64_t M, int64_t n, const Tiles& tiles_of, int64_t stages, int* split_layout)
 {
     const int64_t cus = g_cu_count > 0 ? g_cu_count : 256;
-    const int64_t tiles = ((M + 63) / 64) * ((N + 127) / 128);  // 64 x 128 tiles
-    const double plane_bytes = (double)M * (double)N * 4.0;
+    const int64_t tiles = tiles_of(64, 128);
+    const double plane_bytes = (double)M * (double)n * 4.0;
     int64_t s = 1;
     int lay = 4;
     if (tiles * 2 <= cus && stages >= 8) {
         // unsplit: 64 x 64 tiles where they fit one round (gemm3_layout), about
         // 0.85 of the 64 x 128 time
-        const bool one64 = ((M + 63) / 64) * ((N + 63) / 64) <= cus;
+        const bool one64 = tiles_of(64, 64) <= cus;
         double best = 0.3 * (double)stages * (one64 ? 0.85 : 1.0);
         for (const int L : {4, 5}) {
-            const int64_t tl = L == 4 ? tiles : ((M + 63) / 64) * ((N + 63) / 64);
+            const int64_t tl = L == 4 ? tiles : tiles_of(64, 64);
             const double f = L == 4 ? 1.0 : 0.75;
             const int64_t smax = std::min<int64_t>(cus / tl, stages / 2);
             for (int64_t c = 2; c <= smax; c++) {
@@ -316,6 +320,16 @@ int gemm_splits(int64_t M, int64_t N, int64_t stages, int* split_layout)
     s = std::max<int64_t>(1, std::min<int64_t>(s, stages));
     if (split_layout) *split_layout = lay;
     return (int)s;
+}
+
+auto gemm_tiles(int64_t M, int64_t N)
+{
+    return [M, N](int64_t bm, int64_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
+}
+
+int gemm_splits(int64_t M, int64_t N, int64_t stages, int* split_layout)
+{
+    return gemm_splits(M, N, gemm_tiles(M, N), stages, split_layout);
 }
 
 // k_gemm3 tile numbering.  Each XCD (with its own L2) runs a contiguous
@@ -359,16 +373,20 @@ int gemm3_norder(int64_t M, int64_t N, int64_t act_row_halfs, int64_t krange_cod
 // 128 x 128 one on MI355X), else 128 x 128.  (128 x 128 as 8 waves of
 // 64 x 32 measured the same as 4 waves of 128 x 32 at M=512: the loads
 // into LDS, not latency within a SIMD, bound a block.)
-int gemm3_layout(int64_t M, int64_t N, int splits, int split_layout)
+template <typename Tiles>
+int gemm3_layout(const Tiles& tiles_of, int splits, int split_layout)
 {
     if (splits > 1) return split_layout;
     const int64_t cus = g_cu_count > 0 ? g_cu_count : 256;
-    if (((M + 63) / 64) * ((N + 63) / 64) <= cus) return 5;
-    if (((M + 63) / 64) * ((N + 127) / 128) <= cus) return 4;
-    const int64_t nbm = (M + kGemmBM - 1) / kGemmBM;
-    const int64_t r128 = (nbm * ((N + 127) / 128) + cus - 1) / cus;
-    const int64_t r192 = (nbm * ((N + 191) / 192) + cus - 1) / cus;
+    if (tiles_of(64, 64) <= cus) return 5;
+    if (tiles_of(64, 128) <= cus) return 4;
+    const int64_t r128 = (tiles_of(kGemmBM, 128) + cus - 1) / cus;
+    const int64_t r192 = (tiles_of(kGemmBM, 192) + cus - 1) / cus;
     return 4 * r192 < 3 * r128 ? 1 : 3;
+}
+int gemm3_layout(int64_t M, int64_t N, int splits, int split_layout)
+{
+    return gemm3_layout(gemm_tiles(M, N), splits, split_layout);
 }
 
 constexpr std::size_t kAlign = 256;
@@ -699,7 +717,7 @@ int run_call(const LinArgs& base, int kernel, int act, int outd, void* stream, c
             a.ws = nullptr;
             if (a.K % kGemmBK == 0) {
                 // fp32 activations: the GEMM runs on their split fp16 form
-                // (M rows of 2K: scaled high parts, then low parts, plus one
+                // (M rows of 2K: scaled low parts, then high parts, plus one
                 // inverse scale per row), made in the workspace first
                 const bool f32 = act == VVH_F32;
                 uint64_t xs_bytes = 0, rs_bytes = 0;
@@ -761,6 +779,118 @@ int run_call(const LinArgs& base, int kernel, int act, int outd, void* stream, c
     }
     if (e != 0) return fail_hip((hipError_t)e, "kernel launch");
     return VVH_OK;
+}
+
+// Plans whose problems share their activations (one inp, M and K: q, k and v, or
+// gate and up of a prompt) and take the GEMM: one launch over all their tiles
+// (and one reduction where their k is split), with fp32 activations split into
+// their fp16 halves once.  Also decode plans in fp32 (one M): one k_gemv_f32 launch.
+// Measured per plan against a launch per problem (graph replay): 0.5B q/k/v at M = 512
+// 18.6 -> 7.0 us, gate and up 21.8 -> 17.4; 1.5B q/k/v at M = 2048 34.2 -> 18.8, 0.5B at M =
+// 64 (three k_skinny launches before) 30.8 -> 6.5; fp32 q/k/v at M = 333 35.5 -> 15.1, gate
+// and up 35.1 -> 26.7, q/k/v at M = 1 9.3 -> 3.9.
+constexpr int kGroupNone = 0, kGroupGemm = 1, kGroupGemv = 2;
+
+int plan_group(const std::vector<LinArgs>& args, int act)
+{
+    if (args.size() < 2 || args.size() > (std::size_t)kDotInline) return kGroupNone;
+    const LinArgs& a = args[0];
+    bool same = true, gemv = act == VVH_F32;
+    for (const LinArgs& b : args) {
+        const bool aligned = b.K % 16 == 0 && aligned16(b.w) && aligned16(b.inp);
+        same = same && aligned && b.inp == a.inp && b.M == a.M && b.K == a.K;
+        gemv = gemv && b.M == a.M && choose_kernel(b.M, b.N, b.K, act, aligned) == K_GEMV_F32;
+    }
+    if (gemv) return kGroupGemv;
+    const int64_t min_m = act == VVH_F32 ? (int64_t)kGemmF32MinM : kSkinnyMaxM + 1;
+    return same && a.K > 0 && a.K % kGemmBK == 0 && a.M >= min_m ? kGroupGemm : kGroupNone;
+}
+
+void group_blocks(LinGroup& l, std::size_t count, int64_t blocks)
+{
+    for (std::size_t i = 0; i + 1 < (std::size_t)kDotInline; i++)
+        l.b[i] = i + 1 < count ? l.g.p[i + 1].block_begin : INT32_MAX;
+    l.blocks = (int32_t)blocks;
+}
+
+// Runs a kGroupGemm or kGroupGemv plan; *done = false, and nothing launched,
+// where it needs a workspace it cannot have now or is too large for one grid.
+int run_group(const std::vector<LinArgs>& args, int group, int act, int outd, void* stream, bool* done)
+{
+    *done = false;
+    const std::size_t count = args.size();
+    LinGroup l{};
+    int64_t blocks = 0;
+    if (group == kGroupGemv) {
+        int64_t tiles = 0;
+        for (const LinArgs& a : args) tiles += (a.N + kDecodeTileN - 1) / kDecodeTileN;
+        for (std::size_t i = 0; i < count; i++) {
+            LinArgs& a = l.g.p[i] = args[i];
+            a.ksplit = choose_ksplit(tiles, a.K);
+            a.block_begin = (int32_t)blocks;
+            blocks += decode_blocks(a);
+            if (blocks > INT32_MAX) return VVH_OK;
+        }
+        group_blocks(l, count, blocks);
+        *done = true;
+        const int e = launch_gemv_f32_group(l, outd, stream);
+        return e == 0 ? VVH_OK : fail_hip((hipError_t)e, "grouped launch");
+    }
+    const bool f32 = act == VVH_F32;
+    const int64_t M = args[0].M, K = args[0].K, stages = (f32 ? 2 * K : K) / kGemmBK;
+    int64_t n = 0;
+    for (const LinArgs& a : args) n += a.N;
+    auto tiles_of = [&](int64_t bm, int64_t bn) {
+        int64_t t = 0;
+        for (const LinArgs& a : args) t += ((M + bm - 1) / bm) * ((a.N + bn - 1) / bn);
+        return t;
+    };
+    int split_layout = 4;
+    int sp = gemm_splits(M, n, tiles_of, stages, &split_layout);
+    const int64_t kst = (stages + sp - 1) / sp;
+    sp = (int)((stages + kst - 1) / kst);  // no empty split
+    const int layout = gemm3_layout(tiles_of, sp, split_layout);
+    if (tiles_of(gemm3_tile_m(layout), gemm3_tile_n(layout)) * sp > INT32_MAX) return VVH_OK;
+    uint64_t xs = 0, rs = 0, plane = 0;
+    if (f32) {
+        if (!mul_ok((uint64_t)M * (uint64_t)K, 4, &xs)) return VVH_OK;
+        xs = align_up(xs);
+        rs = align_up((uint64_t)M * 4);
+    }
+    if (sp > 1 && !mul_ok((uint64_t)M * (uint64_t)n, (uint64_t)sp * 4, &plane)) return VVH_OK;
+    float* ws = nullptr;
+    if (xs + rs + plane > 0 && !workspace_try(stream, xs + rs + plane, &ws)) return VVH_OK;
+    char* wb = reinterpret_cast<char*>(ws);
+    float* wp = reinterpret_cast<float*>(wb + xs + rs);
+    for (std::size_t i = 0; i < count; i++) {
+        LinArgs& a = l.g.p[i] = args[i];
+        a.nsplit = sp;
+        a.kstages = sp > 1 ? (int32_t)kst : 0;
+        a.ws = nullptr;
+        if (sp > 1) {
+            a.ws = wp;
+            wp += (int64_t)sp * M * a.N;
+        }
+        if (f32) {
+            a.inp = wb;
+            a.xrs = reinterpret_cast<const float*>(wb + xs);
+            a.bk = K;
+            a.K = 2 * K;
+        }
+        const int64_t krange = sp > 1 ? kst * kGemmBK : K, arow = sp > 1 ? kst * kGemmBK : a.K;
+        a.norder = gemm3_norder(M, a.N, arow, krange, layout, sp);
+        a.block_begin = (int32_t)blocks;
+        blocks += ((M + gemm3_tile_m(layout) - 1) / gemm3_tile_m(layout)) *
+                  ((a.N + gemm3_tile_n(layout) - 1) / gemm3_tile_n(layout)) * sp;
+    }
+    group_blocks(l, count, blocks);
+    *done = true;
+    int e = 0;
+    if (f32)
+        e = launch_split_f32(static_cast<const float*>(args[0].inp), M, K, wb, reinterpret_cast<float*>(wb + xs), stream);
+    if (e == 0) e = launch_gemm3_group(l, outd, layout, stream);
+    if (e == 0 && sp > 1) e = launch_splitk_reduce_group(l, (int)count, outd, stream);
+    return e == 0 ? VVH_OK : fail_hip((hipError_t)e, "grouped launch");
 }
 
 // k_dot plan: problems ordered by K (longest rows first, so the last blocks
@@ -1588,6 +1718,7 @@ VVH_API int vvh_plan_create(const vvh_q8_problem* problems, size_t count, int ac
             return fail_hip(e, "plan table upload");
         }
     }
+    if (!p.dot && !p.stream && !p.grouped && ov == K_AUTO) p.group = plan_group(p.args, act_dtype);
     std::lock_guard<std::mutex> lock(g_pmu);
     const vvh_plan h = g_next_plan++;
     g_plans.emplace(h, std::move(p));
@@ -1633,6 +1764,11 @@ static int plan_run(vvh_plan plan, int64_t pos, void* stream)
     if (p->grouped) {
         const int e = launch_skinny_grouped(p->dev_table, (int)p->args.size(), p->total_blocks, p->out, stream);
         return e == 0 ? VVH_OK : fail_hip((hipError_t)e, "grouped launch");
+    }
+    if (p->group != kGroupNone && g_override.load() == K_AUTO) {
+        bool done = false;
+        const int st = run_group(p->args, p->group, p->act, p->out, stream, &done);
+        if (st != VVH_OK || done) return st;
     }
     for (const LinArgs& a : p->args) {
         const bool aligned = a.K % 16 == 0 && aligned16(a.w) && aligned16(a.inp);
@@ -1860,7 +1996,8 @@ VVH_API int vvh_plan_launches(vvh_plan plan, int* launches)
     std::lock_guard<std::mutex> lock(g_pmu);
     auto it = g_plans.find(plan);
     if (it == g_plans.end()) return fail(VVH_ERR_UNKNOWN_HANDLE, "unknown plan %llu", (unsigned long long)plan);
-    *launches = (it->second.grouped || it->second.stream || it->second.dot) ? 1 : (int)it->second.args.size();
+    const Plan& p = it->second;
+    *launches = (p.grouped || p.stream || p.dot || p.group != kGroupNone) ? 1 : (int)p.args.size();
     return VVH_OK;
 }
 
