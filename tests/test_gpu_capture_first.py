@@ -1,0 +1,112 @@
+"""Calls that use the stream's workspace when they can have it and do without
+otherwise: captured on a stream that never ran them (the capture may not
+allocate), replayed between eager work, against the eager result on a stream
+that has a workspace.  Attention and dense calls whose splits need it, fp32
+linears of a few rows, and a grouped plan whose k is split.
+"""
+import ctypes
+
+import numpy as np
+import pytest
+
+from vvllm_amd import capi
+
+pytestmark = pytest.mark.gpu
+
+F16, F32 = capi.F16, capi.F32
+V = ctypes.c_void_p
+
+
+def hip():
+    lib = ctypes.CDLL("libamdhip64.so.7")
+    for name, args in {"hipStreamCreate": [ctypes.POINTER(V)], "hipStreamSynchronize": [V], "hipStreamDestroy": [V],
+                       "hipStreamBeginCapture": [V, ctypes.c_int], "hipStreamEndCapture": [V, ctypes.POINTER(V)],
+                       "hipGraphInstantiate": [ctypes.POINTER(V), V, V, V, ctypes.c_size_t],
+                       "hipGraphLaunch": [V, V], "hipGraphExecDestroy": [V], "hipGraphDestroy": [V]}.items():
+        getattr(lib, name).argtypes = args
+    return lib
+
+
+def buf(rng, shape, dt, std=1.0):
+    return capi.DevBuf.from_array(rng.normal(0, std, shape).astype(dt))
+
+
+def attention(rng, d, n_q, len0, H, KVH, D):
+    dt = np.float16 if d == F16 else np.float32
+    q, k, v = buf(rng, (n_q, H, D), dt), buf(rng, (len0 + n_q, KVH, D), dt), buf(rng, (len0 + n_q, KVH, D), dt)
+    return (q, k, v), (n_q, H * D), dt, lambda o, s: capi.call(
+        "vvh_attention", o.ptr, q.ptr, k.ptr, v.ptr, n_q, len0, H, KVH, D, float(1 / np.sqrt(D)), d, s)
+
+
+def dense(rng, d, M, N, K):
+    dt = np.float16 if d == F16 else np.float32
+    x, w = buf(rng, (M, K), dt), buf(rng, (N, K), dt, 0.05)
+    return (x, w), (M, N), dt, lambda o, s: capi.call("vvh_dense", o.ptr, x.ptr, w.ptr, d, None, None, M, N, K, d, s)
+
+
+def linear(rng, M, N, K, plan, d=F32):
+    dt = np.float16 if d == F16 else np.float32
+    x = buf(rng, (M, K), dt)
+    es = np.dtype(dt).itemsize
+    q = capi.DevBuf.from_array(rng.integers(-127, 128, (N, K)).astype(np.int8))
+    s = capi.DevBuf.from_array(rng.uniform(1e-4, 3e-4, N).astype(np.float32))
+
+    def run(o, stream):
+        if not plan:
+            return capi.call("vvh_linear_q8_dev", o.ptr, x.ptr, q.ptr, s.ptr, None, None, M, N, K, d, d, stream)
+        half = N // 2  # the two halves of the rows as a plan: its blocks of M x N / 2 outputs one after the other
+        pr = [capi.Q8Problem(out=o.addr(i * M * half * es), inp=x.ptr, residual=None, weight=q.addr(i * half * K),
+                             scales=s.addr(i * half * 4), bias=None, M=M, N=half, K=K) for i in range(2)]
+        key = o.ptr
+        if key not in plans:
+            h = ctypes.c_uint64()
+            capi.call("vvh_plan_create", (capi.Q8Problem * 2)(*pr), 2, d, d, ctypes.byref(h))
+            plans[key] = h.value
+        return capi.call("vvh_plan_run", plans[key], stream)
+    plans = {}
+    return (x, q, s, plans), (M, N), dt, run
+
+
+CASES = {
+    "attention_f16": lambda r: attention(r, F16, 7, 4000, 12, 2, 128),
+    "attention_f32": lambda r: attention(r, F32, 9, 2000, 14, 2, 64),
+    "dense_f16": lambda r: dense(r, F16, 64, 896, 4864),
+    "dense_f32": lambda r: dense(r, F32, 128, 896, 4864),
+    "linear_f32_few": lambda r: linear(r, 5, 1536, 1536, False),
+    "plan_f16": lambda r: linear(r, 40, 256, 896, True, F16),
+    "plan_f32_decode": lambda r: linear(r, 3, 256, 4864, True),
+}
+
+
+@pytest.mark.parametrize("name", CASES)
+def test_captured_without_a_workspace(gpu, name):
+    print(f"[case] captured without a workspace: {name}", flush=True)
+    lib = hip()
+    keep, shape, dt, run = CASES[name](np.random.default_rng(len(name)))
+    size = int(np.prod(shape)) * np.dtype(dt).itemsize
+    want, got = capi.DevBuf(size), capi.DevBuf(size)
+    run(want, None)
+    capi.sync()
+    ref = want.to_array(dt, shape).astype(np.float64)
+    if name.startswith("plan"):  # the plan of the captured run exists before the capture
+        run(got, None)
+        capi.sync()
+    stream, graph, ex = V(), V(), V()
+    assert lib.hipStreamCreate(ctypes.byref(stream)) == 0
+    capi.call("vvh_workspace_release", stream)
+    assert lib.hipStreamBeginCapture(stream, 1) == 0  # thread-local: an allocation would fail
+    run(got, stream)
+    assert lib.hipStreamEndCapture(stream, ctypes.byref(graph)) == 0
+    assert lib.hipGraphInstantiate(ctypes.byref(ex), graph, None, None, 0) == 0
+    zero = np.zeros(shape, dt)
+    for _ in range(3):
+        capi.call("vvh_memcpy_h2d", got.ptr, zero.ctypes.data, size)
+        run(want, None)
+        capi.sync()
+        assert lib.hipGraphLaunch(ex, stream) == 0 and lib.hipStreamSynchronize(stream) == 0
+        y = got.to_array(dt, shape).astype(np.float64)
+        # the same sums in another order: a rounding of the output, or fp32 sums of up to 5000 products
+        tol = 2.0 ** -10 if dt == np.float16 else 2e-6
+        assert np.linalg.norm(y - ref) <= tol * np.linalg.norm(ref)
+    assert lib.hipGraphExecDestroy(ex) == 0 and lib.hipGraphDestroy(graph) == 0
+    assert lib.hipStreamDestroy(stream) == 0

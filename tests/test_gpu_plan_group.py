@@ -84,12 +84,23 @@ def test_gemm_group(gpu, M, Ns, K, d):
 
 
 @pytest.mark.parametrize("M,Ns,K,same_x", [(1, (896, 128, 128), 896, True), (1, (4864, 4864), 896, False),
-                                           (3, (100, 17, 16, 33), 4864, False), (15, (896, 128), 1000 - 8, True),
+                                           (2, (100, 17, 16, 33), 4864, False), (15, (896, 128), 1000 - 8, True),
                                            (20, (64, 48), 208, True)])
 def test_gemv_f32_group(gpu, M, Ns, K, same_x):
     print(f"[case] gemv group M={M} N={Ns} K={K}", flush=True)
     plan, refs, dev = build(np.random.default_rng(M + K), M, Ns, K, F32, same_x)
     assert launches(plan) == 1
+    capi.call("vvh_plan_run", plan, None)
+    capi.sync()
+    check(refs, M, K, F32)
+    capi.call("vvh_plan_destroy", plan)
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 33, 16), (2, 896, 4864), (3, 1000, 144), (4, 17, 8960), (5, 1536, 1536),
+                                   (7, 50, 4096), (8, 9728, 896), (15, 130, 1024), (9, 260, 560), (3, 64, 4160)])
+def test_f32_few_rows(gpu, M, N, K):
+    print(f"[case] f32 few rows M={M} N={N} K={K}", flush=True)
+    plan, refs, dev = build(np.random.default_rng(M + K), M, (N, N), K, F32, same_x=False)  # one by one, or k_gemv_f32
     capi.call("vvh_plan_run", plan, None)
     capi.sync()
     check(refs, M, K, F32)

@@ -289,8 +289,8 @@ int linear_dev(void* out, const void* inp, const int8_t* w, const float* scales,
 // Launchers (linear_kernels.hip).  Return a hipError_t value as int.
 int launch_generic(const LinArgs& a, int act, int out, void* stream);
 int launch_gemv_f32(const LinArgs& a, int out, void* stream);
-// the problems of a group (one M) in one launch
-int launch_gemv_f32_group(const LinGroup& g, int out, void* stream);
+// the `count` problems of a group (one M) in one launch
+int launch_gemv_f32_group(const LinGroup& g, int count, int out, void* stream);
 int launch_skinny(const LinArgs& a, int out, void* stream);
 int launch_skinny_grouped(const LinArgs* dev_table, int count, int64_t total_blocks, int out,
                           void* stream);

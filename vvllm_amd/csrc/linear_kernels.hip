@@ -13,7 +13,7 @@
 //
 // Kernel families:
 //   k_generic   any shape/alignment; one thread per output, sequential k.
-//   k_gemv_f32  fp32 activations, M <= 8 per pass: VALU fp32 FMAs.
+//   k_gemv_f32  fp32 activations, M <= 8 per pass: VALU fp32 FMAs (gemv_kernels.hip).
 //   k_skinny    fp16 activations, M <= 16: one wave owns 16 output channels,
 //               streams their int8 rows with 16-byte loads, converts codes to
 //               fp16 in registers and accumulates with
@@ -101,103 +101,6 @@ __device__ __forceinline__ DecodeCoord decode_coord(const LinArgs& a, int64_t bl
     c.s0 = c.ks * per;
     c.s1 = c.s0 + per < steps ? c.s0 + per : steps;
     return c;
-}
-
-// ---------------------------------------------------------------------------
-// k_gemv_f32: fp32 activations.  Each lane accumulates MT rows of fp32 dot
-// products over its 16-code chunks with exact int8 -> fp32 conversion and
-// fp32 FMAs; the four lanes sharing a channel are combined with cross-lane
-// adds, then the ksplit waves through LDS.  blockIdx.y selects the group of
-// MT activation rows.
-// ---------------------------------------------------------------------------
-template <int MT, typename OT>
-__device__ __forceinline__ void gemv_f32_body(const LinArgs& a, int64_t block, int64_t mbase)
-{
-    __shared__ float red[4][MT][16];
-    const DecodeCoord c = decode_coord(a, block);
-    const int64_t n0 = c.tile * kDecodeTileN;
-    const int64_t n = n0 + (c.lane & 15);
-    const int64_t nrow = n < a.N ? n : a.N - 1;
-    const int chunk = c.lane >> 4;
-    const int8_t* wp = a.w + nrow * a.K + chunk * 16;
-    const float* x = static_cast<const float*>(a.inp);
-
-    float acc[MT];
-#pragma unroll
-    for (int m = 0; m < MT; m++) acc[m] = 0.0f;
-
-    if (n0 < a.N) {
-#pragma unroll 2
-        for (int64_t s = c.s0; s < c.s1; s++) {
-            const int64_t k = s * 64 + chunk * 16;
-            if (k < a.K) {
-                const u4 wv = ld_stream(wp + s * 64);
-                float wf[16];
-#pragma unroll
-                for (int j = 0; j < 4; j++) {
-#pragma unroll
-                    for (int b = 0; b < 4; b++)
-                        wf[4 * j + b] = (float)(int8_t)((wv[j] >> (8 * b)) & 0xff);
-                }
-#pragma unroll
-                for (int m = 0; m < MT; m++) {
-                    if (mbase + m < a.M) {
-                        const f4* xp = reinterpret_cast<const f4*>(x + (mbase + m) * a.K + k);
-                        float sum = acc[m];
-#pragma unroll
-                        for (int q = 0; q < 4; q++) {
-                            const f4 xv = xp[q];
-                            sum = __builtin_fmaf(xv[0], wf[4 * q + 0], sum);
-                            sum = __builtin_fmaf(xv[1], wf[4 * q + 1], sum);
-                            sum = __builtin_fmaf(xv[2], wf[4 * q + 2], sum);
-                            sum = __builtin_fmaf(xv[3], wf[4 * q + 3], sum);
-                        }
-                        acc[m] = sum;
-                    }
-                }
-            }
-        }
-    }
-    // combine the four 16-byte chunks of each channel (lanes l, l^16, l^32, l^48)
-#pragma unroll
-    for (int m = 0; m < MT; m++) {
-        acc[m] = sum_x32(sum_x16(acc[m]));
-    }
-    if (c.ksplit > 1) {
-        if (c.lane < 16) {
-#pragma unroll
-            for (int m = 0; m < MT; m++) red[c.wave][m][c.lane] = acc[m];
-        }
-        __syncthreads();
-        if (c.ks == 0 && c.lane < 16) {
-#pragma unroll
-            for (int m = 0; m < MT; m++) {
-                float s = red[c.wave][m][c.lane];
-                for (int j = 1; j < c.ksplit; j++) s += red[c.wave + j][m][c.lane];
-                acc[m] = s;
-            }
-        }
-    }
-    if (c.ks == 0 && c.lane < 16 && n < a.N) {
-#pragma unroll
-        for (int m = 0; m < MT; m++)
-            if (mbase + m < a.M) store_out<OT>(a, mbase + m, n, acc[m]);
-    }
-}
-
-template <int MT, typename OT>
-__global__ __launch_bounds__(256) void k_gemv_f32(LinArgs a)
-{
-    gemv_f32_body<MT, OT>(a, blockIdx.x, (int64_t)blockIdx.y * MT);
-}
-
-// The problems of a plan (q, k and v of a decode layer) in one launch.
-template <int MT, typename OT>
-__global__ __launch_bounds__(256) void k_gemv_f32_group(LinGroup l)
-{
-    const int b = blockIdx.x;
-    const LinArgs a = l.g.p[(b >= l.b[0]) + (b >= l.b[1]) + (b >= l.b[2])];
-    gemv_f32_body<MT, OT>(a, b - a.block_begin, (int64_t)blockIdx.y * MT);
 }
 
 // ---------------------------------------------------------------------------
@@ -1851,46 +1754,6 @@ int launch_generic(const LinArgs& a, int act, int out, void* stream)
     else if (act == VVH_F32) hipLaunchKernelGGL((k_generic<float, f16>), grid, block, 0, S(stream), a);
     else if (out == VVH_F32) hipLaunchKernelGGL((k_generic<f16, float>), grid, block, 0, S(stream), a);
     else hipLaunchKernelGGL((k_generic<f16, f16>), grid, block, 0, S(stream), a);
-    return (int)hipGetLastError();
-}
-
-template <int MT>
-static void gemv_f32_launch(const LinArgs& a, int out, dim3 grid, hipStream_t s)
-{
-    if (out == VVH_F32) hipLaunchKernelGGL((k_gemv_f32<MT, float>), grid, dim3(256), 0, s, a);
-    else hipLaunchKernelGGL((k_gemv_f32<MT, f16>), grid, dim3(256), 0, s, a);
-}
-
-template <int MT>
-static void gemv_f32_group_launch(const LinGroup& l, int out, dim3 grid, hipStream_t s)
-{
-    if (out == VVH_F32) hipLaunchKernelGGL((k_gemv_f32_group<MT, float>), grid, dim3(256), 0, s, l);
-    else hipLaunchKernelGGL((k_gemv_f32_group<MT, f16>), grid, dim3(256), 0, s, l);
-}
-
-int launch_gemv_f32_group(const LinGroup& l, int out, void* stream)
-{
-    const int64_t M = l.g.p[0].M, mt = M <= 1 ? 1 : M <= 2 ? 2 : M <= 4 ? 4 : 8;
-    const dim3 grid((unsigned)l.blocks, (unsigned)((M + mt - 1) / mt));
-    switch (mt) {
-        case 1: gemv_f32_group_launch<1>(l, out, grid, S(stream)); break;
-        case 2: gemv_f32_group_launch<2>(l, out, grid, S(stream)); break;
-        case 4: gemv_f32_group_launch<4>(l, out, grid, S(stream)); break;
-        default: gemv_f32_group_launch<8>(l, out, grid, S(stream)); break;
-    }
-    return (int)hipGetLastError();
-}
-
-int launch_gemv_f32(const LinArgs& a, int out, void* stream)
-{
-    const int64_t mt = a.M <= 1 ? 1 : a.M <= 2 ? 2 : a.M <= 4 ? 4 : 8;
-    const dim3 grid((unsigned)decode_blocks(a), (unsigned)((a.M + mt - 1) / mt));
-    switch (mt) {
-        case 1: gemv_f32_launch<1>(a, out, grid, S(stream)); break;
-        case 2: gemv_f32_launch<2>(a, out, grid, S(stream)); break;
-        case 4: gemv_f32_launch<4>(a, out, grid, S(stream)); break;
-        default: gemv_f32_launch<8>(a, out, grid, S(stream)); break;
-    }
     return (int)hipGetLastError();
 }
 

@@ -458,6 +458,19 @@ int dot_depth(int64_t K, int ksplit)
 // once per 8 rows (gate/up 4864 x 896, graph replay: M = 8 13.7 against
 // 14.1 us on the GEMM, M = 16 17.0 against 14.2, M = 32 23.9 against 15.1).
 constexpr std::size_t kGemmF32MinM = 16;
+// ... and from fewer on long rows and large weights (K % 64 == 0), where
+// k_gemv_f32 reads its activations per weight tile, or streams the weights twice:
+// graph replay, k_gemv_f32 / GEMM: M = 3 896 x 4864 16.5 / 10.9 us, 1536 x 8960 29 / 14.9,
+// 17920 x 1536 22.4 / 20.2, 9728 x 896 9.2 / 11.5; M = 6 1536 x 1536 10.2 / 9.5, 9728 x 896 15.7 /
+// 11.6, 896 x 896 7.9 / 8.8; M = 2 896 x 4864 8.6 / 10.7.  The error against 64 bits is the
+// smaller of the two (K = 896 1.15e-7 / 1.21e-7, 1536 1.2e-7 / 1.9e-7, 8960 1.2e-7 / 3.1e-7).
+// Such a call takes k_gemv_f32 where the GEMM's workspace cannot be had (run_call).
+bool gemm_f32_few_rows(std::size_t M, std::size_t N, std::size_t K)
+{
+    if (K % kGemmBK != 0) return false;
+    const double nk = (double)N * (double)K;
+    return (M >= 5 && ((K >= 1024 && nk >= 2.3e6) || nk >= 8e6)) || (M >= 3 && (K >= 4096 || nk >= 20e6));
+}
 
 // Small-M fp16 dispatch, from a sweep of every family forced on each shape
 // (us per call on the GPU, calls replayed from HIP graphs; the bench.py
@@ -580,7 +593,8 @@ bool dot_call_takes_x_tile(int64_t M, int64_t N, int64_t K)
 
 int natural_kernel(std::size_t M, std::size_t N, std::size_t K, int act)
 {
-    if (act == VVH_F32) return (M >= kGemmF32MinM && K % kGemmBK == 0) ? K_GEMM : K_GEMV_F32;
+    if (act == VVH_F32)
+        return (M >= kGemmF32MinM && K % kGemmBK == 0) || gemm_f32_few_rows(M, N, K) ? K_GEMM : K_GEMV_F32;
     const int64_t tiles = ((int64_t)N + kDecodeTileN - 1) / kDecodeTileN;
     const bool dot_ok = dot_fits((int64_t)N, (int64_t)K);
     if ((M <= kDotAutoMaxM || (M <= kDotAutoMfMaxM && tiles < kDotMfTiles)) && dot_ok) return K_DOT;
@@ -661,13 +675,31 @@ int validate_call(const void* out, const void* inp, const int8_t* w, const float
     return VVH_OK;
 }
 
+// Workspace of a GEMM call with K % 64 == 0: the split fp32 activations and their
+// row scales, and the k splits' planes.
+uint64_t gemm_ws_bytes(int64_t M, int64_t N, int64_t K, bool f32)
+{
+    int layout = 4;
+    const int64_t stages = (f32 ? 2 * K : K) / kGemmBK;
+    const int s = gemm_splits(M, N, stages, &layout);
+    return (f32 ? align_up((uint64_t)M * (uint64_t)K * 4) + align_up((uint64_t)M * 4) : 0) +
+           (s > 1 ? (uint64_t)s * (uint64_t)M * (uint64_t)N * 4 : 0);
+}
+
 int run_call(const LinArgs& base, int kernel, int act, int outd, void* stream, const WsSource* wsrc = nullptr)
 {
     LinArgs a = base;
     int e = 0;
+    if (kernel == K_GEMM && act == VVH_F32 && a.M < (int64_t)kGemmF32MinM && g_override.load() == K_AUTO) {
+        // few rows: without the workspace (a capture that cannot allocate, a
+        // fixed buffer too small) the kernel that needs none
+        const uint64_t bytes = gemm_ws_bytes(a.M, a.N, a.K, true);
+        float* ws = nullptr;
+        if (wsrc ? bytes > wsrc->bytes : !workspace_try(stream, bytes, &ws)) kernel = K_GEMV_F32;
+    }
     switch (kernel) {
         case K_GEMV_F32: {
-            a.ksplit = choose_ksplit((a.N + kDecodeTileN - 1) / kDecodeTileN, a.K);
+            a.ksplit = choose_ksplit((a.N + kDecodeTileN - 1) / kDecodeTileN, a.K, kDotStep);
             const int64_t mt = a.M <= 1 ? 1 : a.M <= 2 ? 2 : a.M <= 4 ? 4 : kGemvF32MaxM;
             if (decode_blocks(a) > INT32_MAX || (a.M + mt - 1) / mt > 65535)
                 return fail(VVH_ERR_UNSUPPORTED, "problem too large for the decode grid");
@@ -801,9 +833,12 @@ int plan_group(const std::vector<LinArgs>& args, int act)
         same = same && aligned && b.inp == a.inp && b.M == a.M && b.K == a.K;
         gemv = gemv && b.M == a.M && choose_kernel(b.M, b.N, b.K, act, aligned) == K_GEMV_F32;
     }
-    if (gemv) return kGroupGemv;
-    const int64_t min_m = act == VVH_F32 ? (int64_t)kGemmF32MinM : kSkinnyMaxM + 1;
-    return same && a.K > 0 && a.K % kGemmBK == 0 && a.M >= min_m ? kGroupGemm : kGroupNone;
+    std::size_t n = 0;
+    for (const LinArgs& b : args) n += (std::size_t)b.N;
+    const bool rows = act == VVH_F32 ? natural_kernel((std::size_t)a.M, n, (std::size_t)a.K, act) == K_GEMM
+                                     : a.M > kSkinnyMaxM;
+    if (same && a.K > 0 && a.K % kGemmBK == 0 && rows) return kGroupGemm;
+    return gemv ? kGroupGemv : kGroupNone;
 }
 
 void group_blocks(LinGroup& l, std::size_t count, int64_t blocks)
@@ -826,14 +861,14 @@ int run_group(const std::vector<LinArgs>& args, int group, int act, int outd, vo
         for (const LinArgs& a : args) tiles += (a.N + kDecodeTileN - 1) / kDecodeTileN;
         for (std::size_t i = 0; i < count; i++) {
             LinArgs& a = l.g.p[i] = args[i];
-            a.ksplit = choose_ksplit(tiles, a.K);
+            a.ksplit = choose_ksplit(tiles, a.K, kDotStep);
             a.block_begin = (int32_t)blocks;
             blocks += decode_blocks(a);
             if (blocks > INT32_MAX) return VVH_OK;
         }
         group_blocks(l, count, blocks);
         *done = true;
-        const int e = launch_gemv_f32_group(l, outd, stream);
+        const int e = launch_gemv_f32_group(l, (int)count, outd, stream);
         return e == 0 ? VVH_OK : fail_hip((hipError_t)e, "grouped launch");
     }
     const bool f32 = act == VVH_F32;
