@@ -30,7 +30,7 @@
 //   MFMAs of (j, slice 0) || convert (j, slice 1);
 //   MFMAs of (j, slice 1) || convert (j+1, slice 0).
 // Stage indices, fragment parity and wait thresholds are compile-time
-// constants (the loop is unrolled by D, D even).
+// constants (the loop is unrolled by whole rings, an even number of steps).
 //
 // The MFMAs compute the transposed tile (codes as the A operand, activations
 // as B): lane l then holds, for each group g of its 16 accumulator values,
@@ -38,7 +38,7 @@
 // 16-byte write.
 //
 // Epilogue: the raw fp32 sums go through LDS (32-row quarter q of the tile
-// in stage buffer q); each thread then owns one 8-wide column chunk (its 8
+// in stage buffer q; with fewer than four stages in two passes of two); each thread then owns one 8-wide column chunk (its 8
 // scales and biases loaded at kernel start), applies acc * scale + bias
 // (+ residual) in fp32 with one rounding, and stores rows with 16-byte
 // non-temporal stores (the output is not read again by this kernel; measured
@@ -156,14 +156,23 @@ __device__ __forceinline__ void gemm3_fill(f16* __restrict__ sa, int8_t* __restr
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, sb + (wave * LB + i) * 1024, 16, b_off[i], kb, 0, 0);
 }
 
-// BM = 64: blocks of half the LDS and registers, two resident per CU, so one
-// block's MFMAs run while the other waits at its barrier or for its loads.
+// BM = 64 or D < 4: blocks of at most half the LDS and registers, two resident
+// per CU, so one block's MFMAs run while the other waits at its barrier or for
+// its loads.  That gain outweighs the shorter ring of 128-row tiles (graph
+// replay, one 4-stage block per CU -> two of D stages): 128 x 128, D = 3, M=2048
+// N=8960 K=1536 82.5 -> 64.9 us, N=4864 K=896 30.4 -> 25.4, M=300 N=17920 30.3 ->
+// 25.7; 128 x 192, D = 2, N=8960 72.5 -> 68.8, N=4864 30.4 -> 27.6.
+// FOLD: fp32 activations (a.bk), whose second set of accumulators fits two
+// blocks per CU only with 64-row tiles.
 // A = LinGroup: the problems of a plan that share their activations (q, k and v,
 // or gate and up) in one launch; a block finds its problem among them.
-template <typename OT, int D, int WN, int TJ, int TI, int BM, typename A = LinArgs>
-__global__ __launch_bounds__(64 * (BM / 32 / TI) * WN, BM == 64 ? 2 : 1) void k_gemm3(A args)
+template <typename OT, bool FOLD, int D, int WN, int TJ, int TI, int BM, typename A = LinArgs>
+__global__ __launch_bounds__(64 * (BM / 32 / TI) * WN, BM == 64 || D < 4 ? 2 : 1) void k_gemm3(A args)
 {
-    static_assert(D == 4, "four stages: even (static fragment parity) and one epilogue quarter per stage");
+    static_assert(D == 4 || ((D == 2 || D == 3) && BM == 128), "an epilogue quarter per stage, or two passes of two quarters");
+    constexpr int U = D % 2 ? 2 * D : D;  // steps per loop round: whole rings, an even number (static fragment parity)
+    constexpr int NP = D == 4 ? 1 : 2;        // epilogue passes
+    constexpr int PR = BM / NP;               // rows of a pass
     static_assert(TI == 2 || TI == 4, "wave tiles of 64 or 128 rows");
     static_assert(BM == 64 || BM == 128, "block tiles of 64 or 128 rows");
     constexpr int WM = BM / 32 / TI;  // waves along the BM rows
@@ -176,7 +185,9 @@ __global__ __launch_bounds__(64 * (BM / 32 / TI) * WN, BM == 64 ? 2 : 1) void k_
     constexpr int LPS = LA + LB;  // loads per stage per thread
     using Stage = Gemm3Stage<BN, BM>;
     using Frag = Gemm3Frag<TJ, TI>;
-    __shared__ Stage st0, st1, st2, st3;
+    __shared__ Stage st0, st1;
+    __shared__ std::conditional_t<(D > 2), Stage, char> st2;
+    __shared__ std::conditional_t<D == 4, Stage, char> st3;
 
     // consecutive tiles (same n0, or same m0 with a.norder) on one XCD
     LinArgs a;
@@ -273,8 +284,8 @@ __global__ __launch_bounds__(64 * (BM / 32 / TI) * WN, BM == 64 ? 2 : 1) void k_
         constexpr int s = decltype(S)::value % D;
         if constexpr (s == 0) return st0;
         else if constexpr (s == 1) return st1;
-        else if constexpr (s == 2) return st2;
-        else return st3;
+        else if constexpr (s == 2) return reinterpret_cast<Stage&>(st2);
+        else return reinterpret_cast<Stage&>(st3);
     };
     auto issue = [&](Stage& g, int64_t kt) {
         const int64_t k0 = (kbase + kt) * kGemmBK;
@@ -286,12 +297,11 @@ __global__ __launch_bounds__(64 * (BM / 32 / TI) * WN, BM == 64 ? 2 : 1) void k_
     for (int i = 0; i < TI; i++)
 #pragma unroll
         for (int j = 0; j < TJ; j++) acc[i][j] = f16v{};
-    // fp32 activations (a.bk): every 8 stages the accumulators are added to a
+    // FOLD: every 8 stages the accumulators are added to a
     // second set, so that a sum's chain of additions is short: error against 64 bits
     // of an unsplit call of K = 896 1.6e-7 -> 1.1e-7, of K = 4864 4.0e-7 -> 1.3e-7, for 3% more time
-    constexpr bool TWO = sizeof(OT) == 4;
-    f16v sum[TWO ? TI : 1][TWO ? TJ : 1];
-    if constexpr (TWO) {
+    f16v sum[FOLD ? TI : 1][FOLD ? TJ : 1];
+    if constexpr (FOLD) {
 #pragma unroll
         for (int i = 0; i < TI; i++)
 #pragma unroll
@@ -352,19 +362,19 @@ __global__ __launch_bounds__(64 * (BM / 32 / TI) * WN, BM == 64 ? 2 : 1) void k_
     if (nk >= D) {
         prologue.template operator()<D>();
         int64_t kt0 = 0;
-        for (; kt0 + 2 * D <= nk; kt0 += D) {
-            // a full group: every step refills and waits at the steady-state depth
+        for (; kt0 + U + D <= nk; kt0 += U) {
+            // a full round: every step refills and waits at the steady-state depth
             [&]<int... J>(std::integer_sequence<int, J...>) {
                 (step.template operator()<J, true, true, (D - 2) * LPS>(kt0), ...);
-            }(std::make_integer_sequence<int, D>{});
-            if constexpr (TWO) {
-                if (a.bk && kt0 & D) fold();
+            }(std::make_integer_sequence<int, U>{});
+            if constexpr (FOLD) {
+                if (kt0 & U) fold();
             }
         }
-        const int64_t r = nk - kt0;  // D .. 2D-1
+        const int64_t r = nk - kt0;  // D .. U + D - 1
         [&]<int... R>(std::integer_sequence<int, R...>) {
             ((r == R + D ? steps.template operator()<R + D>(kt0) : void()), ...);
-        }(std::make_integer_sequence<int, D>{});
+        }(std::make_integer_sequence<int, U>{});
     } else {
         [&]<int... R>(std::integer_sequence<int, R...>) {
             ((nk == R + 1 ? [&] {
@@ -374,23 +384,24 @@ __global__ __launch_bounds__(64 * (BM / 32 / TI) * WN, BM == 64 ? 2 : 1) void k_
         }(std::make_integer_sequence<int, D - 1>{});
     }
 
-    if constexpr (TWO) {
-        if (a.bk) {
+    if constexpr (FOLD) {
 #pragma unroll
-            for (int i = 0; i < TI; i++)
+        for (int i = 0; i < TI; i++)
 #pragma unroll
-                for (int j = 0; j < TJ; j++) acc[i][j] += sum[i][j];
-        }
+            for (int j = 0; j < TJ; j++) acc[i][j] += sum[i][j];
     }
 
     // ---- epilogue ----
     __builtin_amdgcn_s_waitcnt(0);
     lds_barrier();
     constexpr int ES = BN + 4;  // fp32 row stride of an epilogue quarter
-    auto quarter = [&](int q) -> float* {
-        return reinterpret_cast<float*>(q == 0 ? &st0 : q == 1 ? &st1 : q == 2 ? &st2 : &st3);
+    auto quarter = [&](int q) -> float* {  // D < 4: quarters 2 and 3 in a second pass over stages 0 and 1
+        if constexpr (D < 4) return reinterpret_cast<float*>(q % 2 == 0 ? &st0 : &st1);
+        else return reinterpret_cast<float*>(q == 0 ? &st0 : q == 1 ? &st1 : q == 2 ? &st2 : &st3);
     };
-    constexpr int RI = (BM + RG - 1) / RG;  // rows per thread
+    constexpr int RI = (PR + RG - 1) / RG;  // rows per thread and pass
+    // whether row i of this thread lies in the pass
+    auto in_pass = [&](int i) { return i + 1 < RI || (RI - 1) * RG + erg < PR; };
     // Interior tiles (every row and column inside the problem, whole 8-wide
     // chunks, no split) take a branch-free path; its residual rows are
     // loaded here, so their latency overlaps the accumulator transpose.
@@ -399,14 +410,16 @@ __global__ __launch_bounds__(64 * (BM / 32 / TI) * WN, BM == 64 ? 2 : 1) void k_
     constexpr int RW = sizeof(OT) / 2;  // 16-byte chunks per 8 outputs
     u4 rr[RI][RW];
     const int64_t o_first = (m0 + erg) * a.N + en, o_step = RG * a.N;
-    if (interior && own && a.res) {
-        const OT* rp = static_cast<const OT*>(a.res) + o_first;
+    auto residual_rows = [&](int p) {
+        if (!(interior && own && a.res)) return;
+        const OT* rp = static_cast<const OT*>(a.res) + o_first + p * PR * a.N;
 #pragma unroll
         for (int i = 0; i < RI; i++)
-            if (i + 1 < RI || erg + i * RG < BM)
+            if (in_pass(i))
 #pragma unroll
                 for (int c = 0; c < RW; c++) rr[i][c] = reinterpret_cast<const u4*>(rp + i * o_step)[c];
-    }
+    };
+    residual_rows(0);
     if (a.xrs) {
         // split fp32 activations: each row's sums times its power-of-two scale
 #pragma unroll
@@ -417,140 +430,152 @@ __global__ __launch_bounds__(64 * (BM / 32 / TI) * WN, BM == 64 ? 2 : 1) void k_
             for (int tj = 0; tj < TJ; tj++) acc[ti][tj] *= rs;
         }
     }
+    // pass P of the tile's rows (the only one, with a stage per quarter of 32)
+    auto epilogue = [&]<int P>() {
+        if constexpr (P > 0) {
+            residual_rows(P);
+            lds_barrier();  // every thread is done with the first pass
+        }
 #pragma unroll
-    for (int ti = 0; ti < TI; ti++) {
-        float* q = quarter((row0 >> 5) + ti) + fl * ES + col0 + 4 * fh;
+        for (int ti = 0; ti < TI; ti++) {
+            if constexpr (D < 4)
+                if ((row0 + ti * 32) / PR != P) continue;
+            float* q = quarter((row0 >> 5) + ti) + fl * ES + col0 + 4 * fh;
 #pragma unroll
-        for (int tj = 0; tj < TJ; tj++)
+            for (int tj = 0; tj < TJ; tj++)
 #pragma unroll
-            for (int g = 0; g < 4; g++)
-                *reinterpret_cast<f4*>(q + tj * 32 + 8 * g) =
-                    f4{acc[ti][tj][4 * g], acc[ti][tj][4 * g + 1], acc[ti][tj][4 * g + 2], acc[ti][tj][4 * g + 3]};
-    }
-    lds_barrier();
-    if (!own) return;
-    // lanes 8-15 of a 16-lane read group take the other half of their chunk
-    // first, so the group covers distinct banks
-    const int sw = (ech >> 3) & 1;
-    if (interior) {
-        constexpr int UB = 8;  // rows whose LDS reads are in flight together
+                for (int g = 0; g < 4; g++)
+                    *reinterpret_cast<f4*>(q + tj * 32 + 8 * g) =
+                        f4{acc[ti][tj][4 * g], acc[ti][tj][4 * g + 1], acc[ti][tj][4 * g + 2], acc[ti][tj][4 * g + 3]};
+        }
+
+        lds_barrier();
+        if (!own) return;
+        // lanes 8-15 of a 16-lane read group take the other half of their chunk
+        // first, so the group covers distinct banks
+        const int sw = (ech >> 3) & 1;
+        if (interior) {
+            constexpr int UB = RI < 8 ? RI : 8;  // rows whose LDS reads are in flight together
 #pragma unroll
-        for (int i0 = 0; i0 < RI; i0 += UB) {
-            f4 p[UB], q[UB];
+            for (int i0 = 0; i0 < RI; i0 += UB) {
+                f4 p[UB], q[UB];
 #pragma unroll
-            for (int u = 0; u < UB; u++) {
-                const int i = i0 + u, row = erg + i * RG;
-                if (i < RI && (i + 1 < RI || row < BM)) {
+                for (int u = 0; u < UB; u++) {
+                    const int i = i0 + u, row = P * PR + erg + i * RG;
+                    if (i < RI && in_pass(i)) {
+                        const float* tq = quarter(row >> 5) + (row & 31) * ES + ech * 8;
+                        p[u] = *reinterpret_cast<const f4*>(tq + 4 * sw);
+                        q[u] = *reinterpret_cast<const f4*>(tq + 4 - 4 * sw);
+                    }
+                }
+#pragma unroll
+                for (int u = 0; u < UB; u++) {
+                    const int i = i0 + u;
+                    if (!(i < RI && in_pass(i))) continue;
+                    const f4 lo = sw ? q[u] : p[u], hi = sw ? p[u] : q[u];
+                    float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+#pragma unroll
+                    for (int e = 0; e < 8; e++) v[e] = v[e] * sc[e] + bi[e];
+                    OT* op = static_cast<OT*>(a.out) + o_first + P * PR * a.N + i * o_step;
+                    if constexpr (sizeof(OT) == 2) {
+                        if (a.res) {
+                            const h8 r8 = __builtin_bit_cast(h8, rr[i][0]);
+#pragma unroll
+                            for (int e = 0; e < 8; e++) v[e] += (float)r8[e];
+                        }
+                        h8 o8;
+#pragma unroll
+                        for (int e = 0; e < 8; e++) o8[e] = (f16)v[e];
+                        __builtin_nontemporal_store(o8, reinterpret_cast<h8*>(op));
+                    } else {
+                        if (a.res) {
+                            const f4 r0 = __builtin_bit_cast(f4, rr[i][0]), r1 = __builtin_bit_cast(f4, rr[i][1]);
+#pragma unroll
+                            for (int e = 0; e < 4; e++) {
+                                v[e] += r0[e];
+                                v[e + 4] += r1[e];
+                            }
+                        }
+                        __builtin_nontemporal_store(f4{v[0], v[1], v[2], v[3]}, reinterpret_cast<f4*>(op));
+                        __builtin_nontemporal_store(f4{v[4], v[5], v[6], v[7]}, reinterpret_cast<f4*>(op + 4));
+                    }
+                }
+            }
+            return;
+        }
+        if (en >= a.N) return;
+        const bool vec = (a.N % 8) == 0 && en + 8 <= a.N;
+        constexpr int UG = 4;  // rows whose LDS reads are in flight together
+#pragma unroll
+        for (int i0 = 0; i0 < RI; i0 += UG) {
+            f4 v0[UG], v1[UG];
+#pragma unroll
+            for (int u = 0; u < UG; u++) {
+                const int row = P * PR + erg + (i0 + u) * RG;
+                if (i0 + u < RI && in_pass(i0 + u)) {
                     const float* tq = quarter(row >> 5) + (row & 31) * ES + ech * 8;
-                    p[u] = *reinterpret_cast<const f4*>(tq + 4 * sw);
-                    q[u] = *reinterpret_cast<const f4*>(tq + 4 - 4 * sw);
+                    const f4 p = *reinterpret_cast<const f4*>(tq + 4 * sw);
+                    const f4 q = *reinterpret_cast<const f4*>(tq + 4 - 4 * sw);
+                    v0[u] = sw ? q : p;
+                    v1[u] = sw ? p : q;
                 }
             }
 #pragma unroll
-            for (int u = 0; u < UB; u++) {
-                const int i = i0 + u, row = erg + i * RG;
-                if (!(i < RI && (i + 1 < RI || row < BM))) continue;
-                const f4 lo = sw ? q[u] : p[u], hi = sw ? p[u] : q[u];
-                float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+            for (int u = 0; u < UG; u++) {
+                const int row = P * PR + erg + (i0 + u) * RG;
+                const int64_t mm = m0 + row;
+                if (!(i0 + u < RI && in_pass(i0 + u)) || mm >= a.M) continue;
+                float v[8] = {v0[u][0], v0[u][1], v0[u][2], v0[u][3], v1[u][0], v1[u][1], v1[u][2], v1[u][3]};
+                const int64_t o = mm * a.N + en;
+                if (split) {  // raw partial sums of this split
+                    float* wp = a.ws + ks * a.M * a.N + o;
+                    if (vec) {
+                        *reinterpret_cast<f4*>(wp) = v0[u];
+                        *reinterpret_cast<f4*>(wp + 4) = v1[u];
+                    } else {
+                        for (int e = 0; e < 8 && en + e < a.N; e++) wp[e] = v[e];
+                    }
+                    continue;
+                }
 #pragma unroll
                 for (int e = 0; e < 8; e++) v[e] = v[e] * sc[e] + bi[e];
-                OT* op = static_cast<OT*>(a.out) + o_first + i * o_step;
-                if constexpr (sizeof(OT) == 2) {
-                    if (a.res) {
-                        const h8 r8 = __builtin_bit_cast(h8, rr[i][0]);
-#pragma unroll
-                        for (int e = 0; e < 8; e++) v[e] += (float)r8[e];
-                    }
-                    h8 o8;
-#pragma unroll
-                    for (int e = 0; e < 8; e++) o8[e] = (f16)v[e];
-                    __builtin_nontemporal_store(o8, reinterpret_cast<h8*>(op));
-                } else {
-                    if (a.res) {
-                        const f4 r0 = __builtin_bit_cast(f4, rr[i][0]), r1 = __builtin_bit_cast(f4, rr[i][1]);
-#pragma unroll
-                        for (int e = 0; e < 4; e++) {
-                            v[e] += r0[e];
-                            v[e + 4] += r1[e];
-                        }
-                    }
-                    __builtin_nontemporal_store(f4{v[0], v[1], v[2], v[3]}, reinterpret_cast<f4*>(op));
-                    __builtin_nontemporal_store(f4{v[4], v[5], v[6], v[7]}, reinterpret_cast<f4*>(op + 4));
-                }
-            }
-        }
-        return;
-    }
-    if (en >= a.N) return;
-    const bool vec = (a.N % 8) == 0 && en + 8 <= a.N;
-    constexpr int U = 4;  // rows whose LDS reads are in flight together
-#pragma unroll
-    for (int i0 = 0; i0 < RI; i0 += U) {
-        f4 v0[U], v1[U];
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-            const int row = erg + (i0 + u) * RG;
-            if (i0 + u < RI && row < BM) {
-                const float* tq = quarter(row >> 5) + (row & 31) * ES + ech * 8;
-                const f4 p = *reinterpret_cast<const f4*>(tq + 4 * sw);
-                const f4 q = *reinterpret_cast<const f4*>(tq + 4 - 4 * sw);
-                v0[u] = sw ? q : p;
-                v1[u] = sw ? p : q;
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-            const int row = erg + (i0 + u) * RG;
-            const int64_t mm = m0 + row;
-            if (!(i0 + u < RI && row < BM) || mm >= a.M) continue;
-            float v[8] = {v0[u][0], v0[u][1], v0[u][2], v0[u][3], v1[u][0], v1[u][1], v1[u][2], v1[u][3]};
-            const int64_t o = mm * a.N + en;
-            if (split) {  // raw partial sums of this split
-                float* wp = a.ws + ks * a.M * a.N + o;
                 if (vec) {
-                    *reinterpret_cast<f4*>(wp) = v0[u];
-                    *reinterpret_cast<f4*>(wp + 4) = v1[u];
-                } else {
-                    for (int e = 0; e < 8 && en + e < a.N; e++) wp[e] = v[e];
-                }
-                continue;
-            }
+                    if constexpr (sizeof(OT) == 2) {
+                        if (a.res) {
+                            const h8 r8 = *reinterpret_cast<const h8*>(static_cast<const f16*>(a.res) + o);
 #pragma unroll
-            for (int e = 0; e < 8; e++) v[e] = v[e] * sc[e] + bi[e];
-            if (vec) {
-                if constexpr (sizeof(OT) == 2) {
-                    if (a.res) {
-                        const h8 r8 = *reinterpret_cast<const h8*>(static_cast<const f16*>(a.res) + o);
-#pragma unroll
-                        for (int e = 0; e < 8; e++) v[e] += (float)r8[e];
-                    }
-                    h8 o8;
-#pragma unroll
-                    for (int e = 0; e < 8; e++) o8[e] = (f16)v[e];
-                    __builtin_nontemporal_store(o8, reinterpret_cast<h8*>(static_cast<f16*>(a.out) + o));
-                } else {
-                    if (a.res) {
-                        const f4 r0 = *reinterpret_cast<const f4*>(static_cast<const float*>(a.res) + o);
-                        const f4 r1 = *reinterpret_cast<const f4*>(static_cast<const float*>(a.res) + o + 4);
-#pragma unroll
-                        for (int e = 0; e < 4; e++) {
-                            v[e] += r0[e];
-                            v[e + 4] += r1[e];
+                            for (int e = 0; e < 8; e++) v[e] += (float)r8[e];
                         }
+                        h8 o8;
+#pragma unroll
+                        for (int e = 0; e < 8; e++) o8[e] = (f16)v[e];
+                        __builtin_nontemporal_store(o8, reinterpret_cast<h8*>(static_cast<f16*>(a.out) + o));
+                    } else {
+                        if (a.res) {
+                            const f4 r0 = *reinterpret_cast<const f4*>(static_cast<const float*>(a.res) + o);
+                            const f4 r1 = *reinterpret_cast<const f4*>(static_cast<const float*>(a.res) + o + 4);
+#pragma unroll
+                            for (int e = 0; e < 4; e++) {
+                                v[e] += r0[e];
+                                v[e + 4] += r1[e];
+                            }
+                        }
+                        __builtin_nontemporal_store(f4{v[0], v[1], v[2], v[3]}, reinterpret_cast<f4*>(static_cast<float*>(a.out) + o));
+                        __builtin_nontemporal_store(f4{v[4], v[5], v[6], v[7]},
+                                                    reinterpret_cast<f4*>(static_cast<float*>(a.out) + o + 4));
                     }
-                    __builtin_nontemporal_store(f4{v[0], v[1], v[2], v[3]}, reinterpret_cast<f4*>(static_cast<float*>(a.out) + o));
-                    __builtin_nontemporal_store(f4{v[4], v[5], v[6], v[7]},
-                                                reinterpret_cast<f4*>(static_cast<float*>(a.out) + o + 4));
-                }
-            } else {
-                for (int e = 0; e < 8 && en + e < a.N; e++) {
-                    float x = v[e];
-                    if (a.res) x += ld_f(static_cast<const OT*>(a.res) + o + e);
-                    st_f(static_cast<OT*>(a.out) + o + e, x);
+                } else {
+                    for (int e = 0; e < 8 && en + e < a.N; e++) {
+                        float x = v[e];
+                        if (a.res) x += ld_f(static_cast<const OT*>(a.res) + o + e);
+                        st_f(static_cast<OT*>(a.out) + o + e, x);
+                    }
                 }
             }
         }
-    }
+    };
+    epilogue.template operator()<0>();
+    if constexpr (D < 4) epilogue.template operator()<1>();
 }
 
 // Tile shapes (layout code -> WN, TJ, TI, BM): 1 = 128 x 192 (4 waves of
@@ -558,52 +583,51 @@ __global__ __launch_bounds__(64 * (BM / 32 / TI) * WN, BM == 64 ? 2 : 1) void k_
 // fragment feeds 4 row tiles, 2.5 conversion VALU per MFMA; measured against
 // 4 waves of 64 x 64 in the same runs: M=512 gate/up 11.13 -> 10.78 us,
 // M=2048 33.7 -> 33.3 us, split-K down M=2048 32.7 -> 32.0 us), 4 = 64 x 128
-// (4 waves of 64 x 32, two blocks per CU), 5 = 64 x 64 (2 waves of 64 x 32:
+// (4 waves of 64 x 32), 5 = 64 x 64 (2 waves of 64 x 32:
 // a block fills 12 KB of LDS per stage instead of 16, for calls whose 64 x 64
 // tiles, or split tiles, fit one round over the CUs).
 int gemm3_tile_n(int layout) { return layout == 1 ? 192 : layout == 5 ? 64 : 128; }
 int gemm3_tile_m(int layout) { return (layout == 4 || layout == 5) ? 64 : 128; }
 
-template <int WN, int TJ, int TI, int BM>
-static void gemm3_go(const LinArgs& a, bool f32, hipStream_t s)
+// G = LinArgs or LinGroup; p: the call, or the group's first problem
+template <int WN, int TJ, int TI, int BM, int D, typename G>
+static void gemm3_go(const G& g, const LinArgs& p, unsigned blocks, bool f32, hipStream_t s)
 {
-    constexpr int BN = 32 * TJ * WN;
-    constexpr int NT = 64 * (BM / 32 / TI) * WN;
-    const int64_t tiles = ((a.M + BM - 1) / BM) * ((a.N + BN - 1) / BN);
-    const dim3 grid((unsigned)(tiles * (a.nsplit > 1 ? a.nsplit : 1)));
-    if (f32) hipLaunchKernelGGL((k_gemm3<float, 4, WN, TJ, TI, BM>), grid, dim3(NT), 0, s, a);
-    else hipLaunchKernelGGL((k_gemm3<f16, 4, WN, TJ, TI, BM>), grid, dim3(NT), 0, s, a);
+    const dim3 grid(blocks), block(64 * (BM / 32 / TI) * WN);
+    if constexpr (BM == 64) {
+        if (p.bk) {
+            if (f32) hipLaunchKernelGGL((k_gemm3<float, true, D, WN, TJ, TI, BM, G>), grid, block, 0, s, g);
+            else hipLaunchKernelGGL((k_gemm3<f16, true, D, WN, TJ, TI, BM, G>), grid, block, 0, s, g);
+            return;
+        }
+    }
+    if (f32) hipLaunchKernelGGL((k_gemm3<float, false, D, WN, TJ, TI, BM, G>), grid, block, 0, s, g);
+    else hipLaunchKernelGGL((k_gemm3<f16, false, D, WN, TJ, TI, BM, G>), grid, block, 0, s, g);
 }
 
-template <int WN, int TJ, int TI, int BM>
-static void gemm3_group_go(const LinGroup& g, bool f32, hipStream_t s)
+template <typename G>
+static int gemm3_launch(const G& g, const LinArgs& p, int64_t blocks, int out, int layout, void* stream)
 {
-    constexpr int NT = 64 * (BM / 32 / TI) * WN;
-    const dim3 grid((unsigned)g.blocks);
-    if (f32) hipLaunchKernelGGL((k_gemm3<float, 4, WN, TJ, TI, BM, LinGroup>), grid, dim3(NT), 0, s, g);
-    else hipLaunchKernelGGL((k_gemm3<f16, 4, WN, TJ, TI, BM, LinGroup>), grid, dim3(NT), 0, s, g);
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    const bool f32 = out == VVH_F32;
+    if (p.bk && gemm3_tile_m(layout) != 64) return (int)hipErrorInvalidValue;  // no such instantiation
+    if (layout == 3) gemm3_go<4, 1, 4, 128, 3>(g, p, (unsigned)blocks, f32, s);
+    else if (layout == 4) gemm3_go<4, 1, 2, 64, 4>(g, p, (unsigned)blocks, f32, s);
+    else if (layout == 5) gemm3_go<2, 1, 2, 64, 4>(g, p, (unsigned)blocks, f32, s);
+    else gemm3_go<2, 3, 2, 128, 2>(g, p, (unsigned)blocks, f32, s);
+    return (int)hipGetLastError();
 }
 
 int launch_gemm3_group(const LinGroup& g, int out, int layout, void* stream)
 {
-    hipStream_t s = static_cast<hipStream_t>(stream);
-    const bool f32 = out == VVH_F32;
-    if (layout == 3) gemm3_group_go<4, 1, 4, 128>(g, f32, s);
-    else if (layout == 4) gemm3_group_go<4, 1, 2, 64>(g, f32, s);
-    else if (layout == 5) gemm3_group_go<2, 1, 2, 64>(g, f32, s);
-    else gemm3_group_go<2, 3, 2, 128>(g, f32, s);
-    return (int)hipGetLastError();
+    return gemm3_launch(g, g.g.p[0], g.blocks, out, layout, stream);
 }
 
 int launch_gemm3(const LinArgs& a, int out, int layout, void* stream)
 {
-    hipStream_t s = static_cast<hipStream_t>(stream);
-    const bool f32 = out == VVH_F32;
-    if (layout == 3) gemm3_go<4, 1, 4, 128>(a, f32, s);
-    else if (layout == 4) gemm3_go<4, 1, 2, 64>(a, f32, s);
-    else if (layout == 5) gemm3_go<2, 1, 2, 64>(a, f32, s);
-    else gemm3_go<2, 3, 2, 128>(a, f32, s);
-    return (int)hipGetLastError();
+    const int64_t bm = gemm3_tile_m(layout), bn = gemm3_tile_n(layout);
+    const int64_t tiles = ((a.M + bm - 1) / bm) * ((a.N + bn - 1) / bn);
+    return gemm3_launch(a, a, tiles * (a.nsplit > 1 ? a.nsplit : 1), out, layout, stream);
 }
 
 }  // namespace vvh

@@ -366,27 +366,25 @@ int gemm3_norder(int64_t M, int64_t N, int64_t act_row_halfs, int64_t krange_cod
 // then), else 64 x 128 when those tiles give every block a CU of its
 // own (then more CUs work than with 128-row tiles, each on half a tile:
 // gate/up N=4864 K=896 at M=128 and 256, 10.5 -> 8.2 us; q/k/v N=1152 at
-// M=512, 10.3 -> 8.0 us; with more 64-row tiles than CUs, two share a CU
-// and the time rises: M=512 gate/up 10.7 -> 11.8 us); else 128 x 192 when
-// it takes fewer rounds of blocks over the CUs than 128 x 128 by a margin
-// that pays for its longer tiles (a 128 x 192 tile takes 1.33x as long as a
-// 128 x 128 one on MI355X), else 128 x 128.  (128 x 128 as 8 waves of
-// 64 x 32 measured the same as 4 waves of 128 x 32 at M=512: the loads
-// into LDS, not latency within a SIMD, bound a block.)
+// M=512, 10.3 -> 8.0 us), or where the activations are fp32 (their second set
+// of accumulators leaves one 128-row block per CU: 128 x 128 against 64 x 128,
+// M=300 N=17920 K=1536 64.4 -> 55.0 us, M=700 N=K=1536 32.4 -> 24.2, M=1000
+// N=4864 K=896 46 -> 38); else 128 x 192 when it takes fewer rounds of blocks
+// over the CUs than 128 x 128 by a margin that pays for its longer tiles, and at
+// most two, which its two blocks per CU make one (M=2048 N=4864 K=896: 27.6 us,
+// 128 x 128 26.6); else 128 x 128, whose longer ring is ahead from there (128 x
+// 192 against it, M=2048 K=1536: N=8960 68.8 -> 66.8 us, N=17920 132.1 -> 128.0;
+// M=1500 N=12000 K=512 40.0 -> 34.3).
 template <typename Tiles>
-int gemm3_layout(const Tiles& tiles_of, int splits, int split_layout)
+int gemm3_layout(const Tiles& tiles_of, int splits, int split_layout, bool act_f32)
 {
     if (splits > 1) return split_layout;
     const int64_t cus = g_cu_count > 0 ? g_cu_count : 256;
     if (tiles_of(64, 64) <= cus) return 5;
-    if (tiles_of(64, 128) <= cus) return 4;
+    if (tiles_of(64, 128) <= cus || act_f32) return 4;
     const int64_t r128 = (tiles_of(kGemmBM, 128) + cus - 1) / cus;
     const int64_t r192 = (tiles_of(kGemmBM, 192) + cus - 1) / cus;
-    return 4 * r192 < 3 * r128 ? 1 : 3;
-}
-int gemm3_layout(int64_t M, int64_t N, int splits, int split_layout)
-{
-    return gemm3_layout(gemm_tiles(M, N), splits, split_layout);
+    return 4 * r192 < 3 * r128 && r192 <= 2 ? 1 : 3;
 }
 
 constexpr std::size_t kAlign = 256;
@@ -790,7 +788,7 @@ int run_call(const LinArgs& base, int kernel, int act, int outd, void* stream, c
                     if (a.nsplit > 1) a.ws = reinterpret_cast<float*>(wb + xs_bytes + rs_bytes);
                 }
                 {
-                    const int layout = gemm3_layout(a.M, a.N, a.nsplit, split_layout);
+                    const int layout = gemm3_layout(gemm_tiles(a.M, a.N), a.nsplit, split_layout, f32);
                     const int64_t krange = a.nsplit > 1 ? (int64_t)a.kstages * kGemmBK : (a.bk ? a.bk : a.K);
                     const int64_t arow = a.nsplit > 1 ? (int64_t)a.kstages * kGemmBK : a.K;
                     a.norder = gemm3_norder(a.M, a.N, arow, krange, layout, a.nsplit);
@@ -884,7 +882,7 @@ int run_group(const std::vector<LinArgs>& args, int group, int act, int outd, vo
     int sp = gemm_splits(M, n, tiles_of, stages, &split_layout);
     const int64_t kst = (stages + sp - 1) / sp;
     sp = (int)((stages + kst - 1) / kst);  // no empty split
-    const int layout = gemm3_layout(tiles_of, sp, split_layout);
+    const int layout = gemm3_layout(tiles_of, sp, split_layout, f32);
     if (tiles_of(gemm3_tile_m(layout), gemm3_tile_n(layout)) * sp > INT32_MAX) return VVH_OK;
     uint64_t xs = 0, rs = 0, plane = 0;
     if (f32) {
@@ -2101,7 +2099,7 @@ VVH_API int vvh_gemm_variant(size_t M, size_t N, size_t K, int* tile_n, int* spl
             const int64_t kst = (stages + s - 1) / s;
             s = (int)((stages + kst - 1) / kst);
         }
-        const int layout = gemm3_layout((int64_t)M, (int64_t)N, s, split_layout);
+        const int layout = gemm3_layout(gemm_tiles((int64_t)M, (int64_t)N), s, split_layout, false);
         v = gemm3_tile_m(layout) == 64 ? 4 : 3;
         tn = gemm3_tile_n(layout);
     }
