@@ -358,32 +358,28 @@ int launch_attention_prefill(const AttnPrefillPlan& p, void* out, const void* q,
                              int64_t n_q, int64_t len0, int64_t H, int64_t KVH, int64_t D, float scale, int dtype,
                              float* ws, void* stream);
 // n_q = 1 fast path: grouped heads, split over the sequence into nb blocks
-// per kv head.  mfma: the fp16 matrix-core kernel (head_dim 64 or 128), which
-// merges the blocks in the same launch and, with nb > 1, needs a zeroed
-// arrival counter per kv head (cnt, kAttnCounters of them per stream); else
-// the lane kernel, followed by a merge launch when nb > 1.  ws holds
+// per kv head.  mfma: the fp16 matrix-core kernels (head_dim 64 or 128), else
+// the lane kernel; a merge launch follows when nb > 1.  ws holds
 // attention_decode_ws_floats() floats (none when nb == 1).
 struct AttnDecodePlan {
     bool mfma;
-    int waves;          // waves per block of the mfma kernel (4 or 8)
+    int waves;          // waves per block of the mfma kernels (1: k_attention_parts; 4 or 8)
     int64_t per_block;  // keys per block
     int64_t nb;         // blocks per kv head
 };
-constexpr int64_t kAttnCounters = 16384;
 bool attention_decode_ok(const void* k, const void* v, int64_t len, int64_t H, int64_t KVH, int64_t D);
 int64_t attention_decode_max_len();
-AttnDecodePlan attention_decode_plan(const void* q, int64_t len, int64_t H, int64_t KVH, int64_t D, int dtype);
+AttnDecodePlan attention_decode_plan(const void* q, int64_t len, int64_t H, int64_t KVH, int64_t D, int dtype,
+                                     bool coarse);
 int64_t attention_decode_ws_floats(const AttnDecodePlan& p, int64_t H, int64_t D);
-inline bool attention_decode_counted(const AttnDecodePlan& p) { return p.mfma && p.nb > 1; }
 int launch_attention_decode(const AttnDecodePlan& p, void* out, const void* q, const void* k, const void* v,
-                            int64_t len, int64_t H, int64_t KVH, int64_t D, float scale, float* ws, unsigned* cnt,
-                            int dtype, void* stream);
+                            int64_t len, int64_t H, int64_t KVH, int64_t D, float scale, float* ws, int dtype,
+                            void* stream);
 // Per-wave parts of the decode attention (k_attention_parts) for spans the
 // matrix-core kernel takes in one block (mfma and nb == 1 in the plan);
 // nparts = that block's waves.  parts: nparts * H rows of D + 4 floats.
 int launch_attention_parts(float* parts, const void* q, const void* k, const void* v, int64_t len, int64_t H,
                            int64_t KVH, int64_t D, float scale, int nparts, void* stream);
-int launch_zero_u32(unsigned* p, int64_t n, void* stream);
 int launch_copy2(void* d0, const void* s0, void* d1, const void* s1, int64_t bytes, void* stream);
 int launch_dense(void* out, const void* x, const void* w, int wdtype, const float* bias, const void* res, int64_t M,
                  int64_t N, int64_t K, int dtype, void* stream);

@@ -781,22 +781,24 @@ __global__ __launch_bounds__(256) void k_attention_decode(T* __restrict__ out, c
 // Block per head, one pass over the partials: thread (s, d) merges the
 // blocks c = s, s + S, ... (S = blockDim.x / D) into a running maximum and sums
 // rescaled to it (the online-softmax merge); the S groups then merge the
-// same way through LDS.
-template <typename T>
+// same way through LDS.  A partial's row: m, l, o of the lane kernel; PARTS: o,
+// m, l (m in log2 units) and two unused floats of the matrix-core kernels.
+template <typename T, bool PARTS>
 __global__ __launch_bounds__(1024) void k_attention_combine(T* __restrict__ out, const float* __restrict__ ws,
                                                             int32_t blocks, int32_t H, int32_t D)
 {
     __shared__ float sm[1024], sn[1024], sd[1024];
+    auto ex = [](float x) { return PARTS ? exp2f(x) : expf(x); };
     const int h = blockIdx.x, tid = threadIdx.x;
     const int S = (int)blockDim.x / D, s = tid / D, d = tid - s * D;
     float M = -INFINITY, num = 0.0f, den = 0.0f;
     if (s < S) {
 #pragma unroll 4
         for (int c = s; c < blocks; c += S) {
-            const float* w = ws + ((int64_t)c * H + h) * (D + 2);
-            const float m = w[0], l = w[1], o = w[2 + d];
+            const float* w = ws + ((int64_t)c * H + h) * (PARTS ? D + 4 : D + 2);
+            const float m = w[PARTS ? D : 0], l = w[PARTS ? D + 1 : 1], o = w[PARTS ? d : 2 + d];
             const float mn = fmaxf(M, m);          // m is finite: every block has a key
-            const float a = expf(M - mn), b = expf(m - mn);  // a = 0 on the first block
+            const float a = ex(M - mn), b = ex(m - mn);  // a = 0 on the first block
             num = num * a + o * b;
             den = den * a + l * b;
             M = mn;
@@ -811,7 +813,7 @@ __global__ __launch_bounds__(1024) void k_attention_combine(T* __restrict__ out,
         for (int g = 0; g < S; g++) mt = fmaxf(mt, sm[g * D + tid]);
         float a = 0.0f, b = 0.0f;
         for (int g = 0; g < S; g++) {
-            const float f = expf(sm[g * D + tid] - mt);  // 0 for a group without blocks
+            const float f = ex(sm[g * D + tid] - mt);  // 0 for a group without blocks
             a += sn[g * D + tid] * f;
             b += sd[g * D + tid] * f;
         }
@@ -847,11 +849,15 @@ __global__ __launch_bounds__(1024) void k_attention_combine(T* __restrict__ out,
 // assignment of dims (or keys) to a lane's 8 slots that A and B share gives
 // the same sums.  The W waves merge their (max, sum, O) through LDS.  With one
 // block per kv head the block writes the output; otherwise each block writes
-// its partial (max, sum, O) to ws, and the last block of the kv head to arrive
-// (a per-kv-head counter in cnt, left at zero again for the next call) merges
-// the nb partials and writes the output: one launch either way.
+// its partial (O, max, sum) to ws and k_attention_combine merges the nb of them
+// in a second launch.  (Merging in the last block to arrive instead cost each
+// block a device-wide release, and that block a serial chain over all partials:
+// graph replay, per call, 12 heads / 2 kv heads of 128, 2000 keys 12.0 -> 8.8 us,
+// 4096 16.0 -> 9.1, 30000 41.8 -> 14.3; with a block per chunk, k_attention_parts,
+// 7.3 and 8.3 at 2000 and 4096.)
 // ---------------------------------------------------------------------------
 constexpr int kDecChunk = 64;  // keys per wave and chunk
+constexpr int kDecParts = 64;  // most chunks of a kv head that are a block each (attention_decode_plan)
 
 typedef _Float16 h4v __attribute__((ext_vector_type(4)));
 
@@ -986,7 +992,7 @@ __global__ __launch_bounds__(64 * kDecWaves) void k_attention_decode_mfma(const 
                                                                const f16* __restrict__ k, const f16* __restrict__ v,
                                                                int64_t len, int64_t per_block, int32_t KVH, int32_t G,
                                                                float scale_log2, f16* __restrict__ out,
-                                                               float* __restrict__ ws, unsigned* __restrict__ cnt)
+                                                               float* __restrict__ ws)
 {
     constexpr int DE = D / 16;              // 16-dim tiles of O^T
     constexpr int VP = D + 4;               // V row pitch in LDS (halves)
@@ -994,7 +1000,6 @@ __global__ __launch_bounds__(64 * kDecWaves) void k_attention_decode_mfma(const 
     static_assert(kDecWaves * kDecChunk * VP * 2 >= kDecWaves * 16 * OP * 4, "O aliases the V regions");
     __shared__ __align__(16) _Float16 vs[kDecWaves * kDecChunk * VP];
     __shared__ float wm[kDecWaves][16], wl[kDecWaves][16];
-    __shared__ int last_s;
     const int g = blockIdx.x, tid = threadIdx.x, w = tid >> 6, lane = tid & 63, r = lane & 15, gr = lane >> 4;
     const int H = G * KVH;
     const int64_t kvs = (int64_t)KVH * D;
@@ -1033,43 +1038,17 @@ __global__ __launch_bounds__(64 * kDecWaves) void k_attention_decode_mfma(const 
         if (!split) {
             out[((int64_t)g * G + h) * D + d] = (f16)(num / den);
         } else {
-            float* pw = ws + ((int64_t)blockIdx.y * H + (int64_t)g * G + h) * (D + 2);
-            pw[2 + d] = num;
+            float* pw = ws + ((int64_t)blockIdx.y * H + (int64_t)g * G + h) * (D + 4);
+            pw[d] = num;
             if (d == 0) {
-                pw[0] = M;
-                pw[1] = den;
+                pw[D] = M;
+                pw[D + 1] = den;
             }
         }
     }
-    if (!split) return;
-    // the partials visible device-wide before the block counts itself in
-    __threadfence();
-    __syncthreads();
-    if (tid == 0) last_s = atomicAdd(cnt + g, 1u) == gridDim.y - 1;
-    __syncthreads();
-    if (!last_s) return;
-    __threadfence();  // the other blocks' partials, not stale cached lines
-    const int nb = (int)gridDim.y;
-    for (int idx = tid; idx < G * D; idx += 64 * kDecWaves) {
-        const int h = idx / D, d = idx - h * D;
-        const float* pw = ws + ((int64_t)g * G + h) * (D + 2);
-        const int64_t step = (int64_t)H * (D + 2);
-        float M = -INFINITY, num = 0.0f, den = 0.0f;
-#pragma unroll 4
-        for (int b = 0; b < nb; b++) {
-            const float mb = pw[b * step], lb = pw[b * step + 1], ob = pw[b * step + 2 + d];
-            const float mx = fmaxf(M, mb);  // mb is finite: every block has a key
-            const float a = exp2f(M - mx), c = exp2f(mb - mx);
-            num = num * a + ob * c;
-            den = den * a + lb * c;
-            M = mx;
-        }
-        out[((int64_t)g * G + h) * D + d] = (f16)(num / den);
-    }
-    if (tid == 0) cnt[g] = 0u;  // ready for the next call on this stream
 }
 
-// Decode attention as per-wave parts, for spans that k_attention_decode_mfma
+// Decode attention as per-wave parts.  For spans that k_attention_decode_mfma
 // takes in one block of W waves (nb == 1): block (g, w) is one wave doing
 // what wave w of that block does (the chunks w, w + W, ... of kv head g, the
 // same wave body) and writes, for each query head h = g G + r of the kv
@@ -1078,7 +1057,8 @@ __global__ __launch_bounds__(64 * kDecWaves) void k_attention_decode_mfma(const 
 // head in part order (attn_merge_add, then num / den) repeats the block's
 // merge of its waves, so the output has the bits of the one-launch kernel;
 // the merge runs in the consumer (k_dot input stage 3).  One wave per block
-// spreads a kv head's K/V rows over W CUs instead of one.
+// spreads a kv head's K/V rows over W CUs instead of one.  Longer spans take it
+// with W = their chunks, merged by k_attention_combine.
 template <int D>
 __global__ __launch_bounds__(64) void k_attention_parts(const f16* __restrict__ q, const f16* __restrict__ k,
                                                         const f16* __restrict__ v, int64_t len, int32_t KVH,
@@ -1105,12 +1085,6 @@ __global__ __launch_bounds__(64) void k_attention_parts(const f16* __restrict__ 
             pr[D + 1] = l;
         }
     }
-}
-
-__global__ void k_zero_u32(unsigned* __restrict__ p, int64_t n)
-{
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = 0u;
 }
 
 // Two copies of n bytes in one launch (the K and V rows of a cache append):
@@ -1142,14 +1116,6 @@ int launch_copy2(void* d0, const void* s0, void* d1, const void* s1, int64_t byt
     return (int)hipGetLastError();
 }
 
-int launch_zero_u32(unsigned* p, int64_t n, void* stream)
-{
-    if (n <= 0) return 0;
-    hipLaunchKernelGGL(k_zero_u32, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, static_cast<hipStream_t>(stream),
-                       p, n);
-    return (int)hipGetLastError();
-}
-
 bool attention_decode_ok(const void* k, const void* v, int64_t len, int64_t H, int64_t KVH, int64_t D)
 {
     return D % 8 == 0 && D <= kAttnMaxD && H / KVH <= kAttnMaxG && reinterpret_cast<uintptr_t>(k) % 16 == 0 &&
@@ -1172,21 +1138,30 @@ static int64_t attn_per_block(int64_t len, int64_t KVH, int64_t D)
 
 // The matrix-core kernel takes spans of up to 8 chunks of 64 keys in one
 // block per kv head, one chunk per wave (4 waves up to 4 chunks, else 8), with
-// no cross-block merge.  Longer spans take 4-wave blocks, one chunk per wave
-// while that keeps at most 64 blocks per kv head and ~256 blocks in all,
-// several beyond.  (Graph-replayed, Qwen2.5-0.5B shapes: a wave's second
-// chunk costs ~2 us, the cross-block merge ~3.4 us, so 8 waves in one block
-// win at 512 keys and 4-wave blocks at 1024 and beyond.)
-AttnDecodePlan attention_decode_plan(const void* q, int64_t len, int64_t H, int64_t KVH, int64_t D, int dtype)
+// no cross-block merge.  Longer spans of up to kDecParts chunks take one-wave
+// blocks of a chunk each (k_attention_parts) while they fit one round over the
+// CUs (256): 14 / 2 heads of 64, 1023 keys, 6.3 us against 6.6 in 4-wave blocks
+// and 7.8 with those merged by the last to arrive; 12 / 2 heads of 128, 700 keys
+// 7.3 against 8.9 and 11.5; two rounds of them lose (32 / 8 heads of 128, 4000
+// keys 9.6 against 9.2), and so do more partials (12 / 2, 8191 keys 10.4
+// against 9.7, 30000 23.1 against 14.3: the merge grows).  The rest take 4-wave
+// blocks, one chunk per wave while that keeps at most 64 blocks per kv head and
+// ~256 blocks in all, several beyond.  coarse: no one-wave blocks, whose
+// partials take up to 4 times the workspace.
+AttnDecodePlan attention_decode_plan(const void* q, int64_t len, int64_t H, int64_t KVH, int64_t D, int dtype,
+                                     bool coarse)
 {
     AttnDecodePlan p{};
-    p.mfma = dtype == VVH_F16 && (D == 64 || D == 128) && H / KVH <= 16 && KVH <= kAttnCounters &&
+    p.mfma = dtype == VVH_F16 && (D == 64 || D == 128) && H / KVH <= 16 &&
              reinterpret_cast<uintptr_t>(q) % 16 == 0;
     if (p.mfma) {
         const int64_t chunks = (len + kDecChunk - 1) / kDecChunk;
         if (chunks <= 8) {
             p.waves = chunks <= 4 ? 4 : 8;
             p.per_block = p.waves * kDecChunk;
+        } else if (!coarse && chunks <= kDecParts && chunks * KVH <= 256) {
+            p.waves = 1;
+            p.per_block = kDecChunk;
         } else {
             p.waves = 4;
             const int64_t nb_cap = std::min<int64_t>(64, std::max<int64_t>(1, 256 / KVH));
@@ -1217,7 +1192,7 @@ int launch_attention_parts(float* parts, const void* q, const void* k, const voi
 
 int64_t attention_decode_ws_floats(const AttnDecodePlan& p, int64_t H, int64_t D)
 {
-    return p.nb > 1 ? p.nb * H * (D + 2) : 0;
+    return p.nb > 1 ? p.nb * H * (p.mfma ? D + 4 : D + 2) : 0;
 }
 
 // Combine block: D x S threads, S (a power of two, 1 <= S <= 1024 / D) the
@@ -1231,8 +1206,8 @@ static unsigned combine_threads(int64_t nb, int64_t D)
 }
 
 int launch_attention_decode(const AttnDecodePlan& p, void* out, const void* q, const void* k, const void* v,
-                            int64_t len, int64_t H, int64_t KVH, int64_t D, float scale, float* ws, unsigned* cnt,
-                            int dtype, void* stream)
+                            int64_t len, int64_t H, int64_t KVH, int64_t D, float scale, float* ws, int dtype,
+                            void* stream)
 {
     const int64_t per = p.per_block, nb = p.nb;
     const dim3 grid((unsigned)KVH, (unsigned)nb);
@@ -1241,12 +1216,18 @@ int launch_attention_decode(const AttnDecodePlan& p, void* out, const void* q, c
         const float sl = (float)((double)scale * 1.4426950408889634);  // scores in log2 units
         auto go = [&](auto kern) {
             hipLaunchKernelGGL(kern, grid, dim3(64 * p.waves), 0, s, (const f16*)q, (const f16*)k, (const f16*)v,
-                               len, per, (int32_t)KVH, (int32_t)(H / KVH), sl, (f16*)out, ws, cnt);
+                               len, per, (int32_t)KVH, (int32_t)(H / KVH), sl, (f16*)out, ws);
         };
-        if (D == 64)
+        if (p.waves == 1) {
+            const int st = launch_attention_parts(ws, q, k, v, len, H, KVH, D, scale, (int)nb, stream);
+            if (st != 0) return st;
+        } else if (D == 64)
             p.waves == 8 ? go(k_attention_decode_mfma<64, 8>) : go(k_attention_decode_mfma<64, 4>);
         else
             p.waves == 8 ? go(k_attention_decode_mfma<128, 8>) : go(k_attention_decode_mfma<128, 4>);
+        if (nb > 1)
+            hipLaunchKernelGGL((k_attention_combine<f16, true>), dim3((unsigned)H), dim3(combine_threads(nb, D)), 0, s,
+                               (f16*)out, ws, (int32_t)nb, (int32_t)H, (int32_t)D);
         return (int)hipGetLastError();
     }
     const bool one = per <= 256 / attn_lanes((int)D);  // one sub-chunk per block
@@ -1258,8 +1239,8 @@ int launch_attention_decode(const AttnDecodePlan& p, void* out, const void* q, c
             hipLaunchKernelGGL((k_attention_decode<f16, false>), grid, dim3(256), 0, s, (f16*)out, (const f16*)q,
                                (const f16*)k, (const f16*)v, len, (int32_t)H, (int32_t)KVH, (int32_t)D, scale, per, ws);
         if (nb > 1)
-            hipLaunchKernelGGL(k_attention_combine<f16>, dim3((unsigned)H), dim3(combine_threads(nb, D)), 0, s, (f16*)out, ws,
-                               (int32_t)nb, (int32_t)H, (int32_t)D);
+            hipLaunchKernelGGL((k_attention_combine<f16, false>), dim3((unsigned)H), dim3(combine_threads(nb, D)), 0, s,
+                               (f16*)out, ws, (int32_t)nb, (int32_t)H, (int32_t)D);
     } else {
         if (one)
             hipLaunchKernelGGL((k_attention_decode<float, true>), grid, dim3(256), 0, s, (float*)out,
@@ -1270,8 +1251,8 @@ int launch_attention_decode(const AttnDecodePlan& p, void* out, const void* q, c
                                (const float*)q, (const float*)k, (const float*)v, len, (int32_t)H, (int32_t)KVH,
                                (int32_t)D, scale, per, ws);
         if (nb > 1)
-            hipLaunchKernelGGL(k_attention_combine<float>, dim3((unsigned)H), dim3(combine_threads(nb, D)), 0, s, (float*)out, ws,
-                               (int32_t)nb, (int32_t)H, (int32_t)D);
+            hipLaunchKernelGGL((k_attention_combine<float, false>), dim3((unsigned)H), dim3(combine_threads(nb, D)), 0, s,
+                               (float*)out, ws, (int32_t)nb, (int32_t)H, (int32_t)D);
     }
     return (int)hipGetLastError();
 }

@@ -131,7 +131,6 @@ struct Workspace {
     void* p = nullptr;
     std::size_t bytes = 0;
     std::vector<void*> retired;
-    unsigned* cnt = nullptr;  // kAttnCounters arrival counters of the decode attention, zero between calls
 };
 std::mutex g_wsmu;
 std::unordered_map<void*, Workspace> g_ws;
@@ -153,48 +152,6 @@ int workspace_for(void* stream, std::size_t bytes, float** out)
         w.bytes = nb;
     }
     *out = static_cast<float*>(w.p);
-    return VVH_OK;
-}
-
-// The stream's decode-attention counters: allocated on first use and zeroed
-// before this returns, by a kernel on a private non-blocking stream that the
-// host waits for.  So they are zero for the first direct call and for the
-// first replay alike, also when the first use happens inside a capture of
-// `stream` (the private stream is not captured; no memset node is recorded);
-// every call leaves them at zero again.
-hipStream_t g_zero_stream[64] = {};
-
-int counters_for(void* stream, unsigned** out)
-{
-    std::lock_guard<std::mutex> lock(g_wsmu);
-    Workspace& w = g_ws[stream];
-    if (!w.cnt) {
-        if (g_device < 0 || g_device >= 64) return fail(VVH_ERR_UNSUPPORTED, "device %d out of range", g_device);
-        hipStream_t& zs = g_zero_stream[g_device];
-        if (!zs) {
-            const hipError_t e = hipStreamCreateWithFlags(&zs, hipStreamNonBlocking);
-            if (e != hipSuccess) {
-                (void)hipGetLastError();
-                zs = nullptr;
-                return fail_hip(e, "attention counters: private stream");
-            }
-        }
-        void* p = nullptr;
-        hipError_t e = hipMalloc(&p, (std::size_t)kAttnCounters * sizeof(unsigned));
-        if (e != hipSuccess) {
-            (void)hipGetLastError();
-            return fail_hip(e, "attention counters hipMalloc");
-        }
-        int st = launch_zero_u32(static_cast<unsigned*>(p), kAttnCounters, zs);
-        if (st == 0) st = (int)hipStreamSynchronize(zs);
-        if (st != 0) {
-            (void)hipGetLastError();
-            (void)hipFree(p);
-            return fail_hip((hipError_t)st, "attention counters zero launch");
-        }
-        w.cnt = static_cast<unsigned*>(p);
-    }
-    *out = w.cnt;
     return VVH_OK;
 }
 
@@ -1563,7 +1520,6 @@ VVH_API int vvh_workspace_release(void* stream)
     if (e != hipSuccess) return fail_hip(e, "workspace release: synchronize");
     for (void* p : it->second.retired) (void)hipFree(p);
     if (it->second.p) (void)hipFree(it->second.p);
-    if (it->second.cnt) (void)hipFree(it->second.cnt);
     g_ws.erase(it);
     return VVH_OK;
 }
@@ -2225,22 +2181,21 @@ VVH_API int vvh_attention(void* out, const void* q, const void* k, const void* v
         return fail(VVH_ERR_UNSUPPORTED, "attention span %zu > %lld", len0 + n_q - 1, (long long)attention_max_len());
     REQUIRE_INIT();
     if (decode) {
-        const AttnDecodePlan p = attention_decode_plan(q, (int64_t)len0, (int64_t)num_heads, (int64_t)num_kv_heads,
-                                                       (int64_t)head_dim, dtype);
+        AttnDecodePlan p = attention_decode_plan(q, (int64_t)len0, (int64_t)num_heads, (int64_t)num_kv_heads,
+                                                 (int64_t)head_dim, dtype, false);
         float* ws = nullptr;
-        unsigned* cnt = nullptr;
-        const int64_t wsf = attention_decode_ws_floats(p, (int64_t)num_heads, (int64_t)head_dim);
-        if (wsf > 0) {
+        int64_t wsf = attention_decode_ws_floats(p, (int64_t)num_heads, (int64_t)head_dim);
+        if (p.mfma && wsf > 0 && !workspace_try(stream, (std::size_t)wsf * 4, &ws)) {
+            p = attention_decode_plan(q, (int64_t)len0, (int64_t)num_heads, (int64_t)num_kv_heads, (int64_t)head_dim,
+                                      dtype, true);
+            wsf = attention_decode_ws_floats(p, (int64_t)num_heads, (int64_t)head_dim);
+        }
+        if (wsf > 0 && !ws) {
             const int st = workspace_for(stream, (std::size_t)wsf * 4, &ws);
             if (st != VVH_OK) return st;
         }
-        if (attention_decode_counted(p)) {
-            const int st = counters_for(stream, &cnt);
-            if (st != VVH_OK) return st;
-        }
         return ret_launch(launch_attention_decode(p, out, q, k, v, (int64_t)len0, (int64_t)num_heads,
-                                                  (int64_t)num_kv_heads, (int64_t)head_dim, scale, ws, cnt, dtype,
-                                                  stream),
+                                                  (int64_t)num_kv_heads, (int64_t)head_dim, scale, ws, dtype, stream),
                           "attention launch");
     }
     if (attention_prefill_ok(out, q, k, v, (int64_t)n_q, (int64_t)len0, (int64_t)num_heads, (int64_t)num_kv_heads,
@@ -2278,7 +2233,7 @@ VVH_API int vvh_attention_parts(float* parts, size_t parts_floats, size_t* npart
         return fail(VVH_ERR_UNSUPPORTED, "attention parts need fp16, head_dim 64 or 128, num_heads / num_kv_heads "
                     "<= 16 and 16-byte aligned q, k, v and parts");
     const AttnDecodePlan p = attention_decode_plan(q, (int64_t)len0, (int64_t)num_heads, (int64_t)num_kv_heads,
-                                                   (int64_t)head_dim, dtype);
+                                                   (int64_t)head_dim, dtype, false);
     if (!p.mfma || p.nb != 1)
         return fail(VVH_ERR_UNSUPPORTED, "a span of %zu positions is not one block per kv head (at most 512)", len0);
     const std::size_t need = (std::size_t)p.waves * num_heads * (head_dim + 4);
