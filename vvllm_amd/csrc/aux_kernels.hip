@@ -89,19 +89,43 @@ __global__ __launch_bounds__(256) void k_convert(DT* __restrict__ d, const ST* _
         d[i] = (DT)(float)s[i];
 }
 
-int launch_convert(void* dst, int dst_dtype, const void* src, int src_dtype, int64_t n, void* stream)
+// The same, 8 elements a thread in 16-byte accesses, for 32-byte aligned rows; the
+// block after the whole chunks takes the remainder.
+template <typename DT, typename ST>
+__global__ __launch_bounds__(256) void k_convert_vec(DT* __restrict__ d, const ST* __restrict__ s, int64_t n)
+{
+    typedef DT d8 __attribute__((ext_vector_type(8)));
+    typedef ST s8 __attribute__((ext_vector_type(8)));
+    const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 8;
+    if (i + 8 <= n) {
+        const s8 v = *reinterpret_cast<const s8*>(s + i);
+        d8 o;
+#pragma unroll
+        for (int e = 0; e < 8; e++) o[e] = (DT)(float)v[e];
+        *reinterpret_cast<d8*>(d + i) = o;
+    } else {
+        for (int64_t e = i; e < n; e++) d[e] = (DT)(float)s[e];
+    }
+}
+
+template <typename DT, typename ST>
+static void convert_go(DT* d, const ST* src, int64_t n, hipStream_t s)
 {
     const int64_t want = (n + 255) / 256;
-    const dim3 grid((unsigned)(want < 16384 ? (want > 0 ? want : 1) : 16384));
-    hipStream_t s = static_cast<hipStream_t>(stream);
-    if (dst_dtype == VVH_F16 && src_dtype == VVH_F32)
-        hipLaunchKernelGGL((k_convert<f16, float>), grid, dim3(256), 0, s, (f16*)dst, (const float*)src, n);
-    else if (dst_dtype == VVH_F32 && src_dtype == VVH_F16)
-        hipLaunchKernelGGL((k_convert<float, f16>), grid, dim3(256), 0, s, (float*)dst, (const f16*)src, n);
-    else if (dst_dtype == VVH_F32)
-        hipLaunchKernelGGL((k_convert<float, float>), grid, dim3(256), 0, s, (float*)dst, (const float*)src, n);
+    if (((reinterpret_cast<uintptr_t>(d) | reinterpret_cast<uintptr_t>(src)) & 31) == 0 && (n + 2047) / 2048 <= (1 << 22))
+        hipLaunchKernelGGL((k_convert_vec<DT, ST>), dim3((unsigned)(n > 0 ? (n + 2047) / 2048 : 1)), dim3(256), 0, s, d, src, n);
     else
-        hipLaunchKernelGGL((k_convert<f16, f16>), grid, dim3(256), 0, s, (f16*)dst, (const f16*)src, n);
+        hipLaunchKernelGGL((k_convert<DT, ST>), dim3((unsigned)(want < 16384 ? (want > 0 ? want : 1) : 16384)), dim3(256), 0,
+                           s, d, src, n);
+}
+
+int launch_convert(void* dst, int dst_dtype, const void* src, int src_dtype, int64_t n, void* stream)
+{
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    if (dst_dtype == VVH_F16 && src_dtype == VVH_F32) convert_go((f16*)dst, (const float*)src, n, s);
+    else if (dst_dtype == VVH_F32 && src_dtype == VVH_F16) convert_go((float*)dst, (const f16*)src, n, s);
+    else if (dst_dtype == VVH_F32) convert_go((float*)dst, (const float*)src, n, s);
+    else convert_go((f16*)dst, (const f16*)src, n, s);
     return (int)hipGetLastError();
 }
 
