@@ -291,7 +291,11 @@ VVH_API int vvh_linear_q8_dev_in(void* out, const void* inp, const int8_t* dev_w
  * (act_dtype, out_dtype) pair, resolved once (kernel choice, tile
  * decomposition, device-resident descriptor table) and launched with
  * vvh_plan_run as a single kernel when every problem takes the decode path
- * (M <= 16), else as one launch per problem.  It is the counterpart of the
+ * (M <= 16), or when its problems read the same activations and take the
+ * GEMM, or are fp32 of few rows (a GEMM of fp32 activations or of split k adds
+ * its split and reduction launches, and without their workspace, as in a
+ * capture that cannot allocate, the problems run one by one); else as one
+ * launch per problem.  It is the counterpart of the
  * reference IR's pre-resolved op list (src/ir/executable.cc:192-354) for the
  * int8 linears that share an input (q/k/v, transformer.h:139-144) or are
  * otherwise independent.  Problems must not write memory another problem of
