@@ -86,3 +86,28 @@ def test_prefill_unseen_rows(gpu, n_q, len0, H, KVH, D, d, bad):
     assert (np.abs(got - ref)[early] <= ULP[d] * np.abs(ref)[early] + 1e-5 * np.abs(clean_v).max()).all()
     if not np.isfinite(bad):
         assert not np.isfinite(got[n_q - 3:, H - 1, 5]).any()
+
+
+@pytest.mark.parametrize("n_q,len0,H,KVH,D", [(40, 1, 14, 2, 64), (700, 1, 12, 2, 128), (33, 3000, 12, 2, 128)])
+@pytest.mark.parametrize("d", [F32, F16])
+@pytest.mark.parametrize("gap", [12, 18, 22, 26])
+def test_prefill_small_weights(gpu, n_q, len0, H, KVH, D, d, gap):
+    """The keys a row attends to under a few with 2^gap times their weight and
+    values of 0 (an attention sink) make up its whole output, so each weight
+    has to keep its bits however far below the largest it is.  A key group of
+    the tiles takes 32 keys at a time: one such key in each.  Per element, next
+    to the output's rounding: scores of up to 26 in log2 units, summed in fp32
+    (2e-5 of the value), and for fp16, weights in steps of 2^-34 of the largest
+    (half of one for each key).
+    """
+    print(f"[case] small weights n_q={n_q} len0={len0} D={D} dtype={d} gap={gap}", flush=True)
+    rng = np.random.default_rng(gap)
+    T, scale = len0 + n_q - 1, float(1 / np.sqrt(D))
+    q, k, v = np.zeros((n_q, H, D)), np.zeros((T, KVH, D)), rng.uniform(500, 1500, (T, KVH, D))
+    q[..., 0] = 8.0
+    sinks = [t for t in (0, 32, 64, 96) if t < T]
+    k[sinks, :, 0], v[sinks] = gap / (8.0 * scale * np.log2(np.e)), 0.0
+    q, k, v = (a.astype(npd(d)) for a in (q, k, v))
+    got, ref = run(q, k, v, len0, scale, d), reference(q, k, v, len0, scale)
+    tol = (ULP[d] + 2e-5) * np.abs(ref) + (2.0 ** -25 + T * 2.0 ** -35 * 1500.0 if d == F16 else 0.0)
+    assert (np.abs(got - ref) <= tol).all()

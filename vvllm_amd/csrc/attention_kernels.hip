@@ -83,14 +83,22 @@ __device__ void attn_row_general(const T* __restrict__ qr, const T* __restrict__
 //   S^T = K q^T    v_mfma_f32_32x32x16_f16, A = K rows, B = the 32 query rows
 //                  (kept in registers): lane l gets row l % 32's scores of 16
 //                  keys, 8 (i / 4) + 4 (l / 32) + i % 4 for i < 16;
-//   softmax        p = exp2(score scale log2 e - m), m the row's running
-//                  maximum in log2 units, moved (and O, l rescaled) only when
-//                  a score exceeds it by more than 8: p stays below 2^8;
+//   softmax        p = exp2(score scale log2 e - b), b the row's running
+//                  maximum in log2 units less 10, moved (and O, l rescaled) only
+//                  when a score exceeds that maximum by more than 5: p stays
+//                  below 2^15, and the largest is 2^10 or more;
 //   O^T += V^T p   A = V^T by LDS transpose reads, B = the lane's own p: the
 //                  order of keys inside an MFMA is free as long as A and B
 //                  share it, so p needs no shuffles.  p goes in as fp16 high
-//                  and low parts (two products), about 22 bits.
-// The groups' (m, l, O) are merged through LDS at the end; blocks that share a
+//                  and low parts (two products): about 22 bits, and steps of
+//                  2^-24, fp16's smallest, 2^-34 of the largest weight.  (With
+//                  weights from 2^0 to 2^8 those of 2^-25 of the largest were
+//                  lost while l counted them: 4000 keys under one of 2^22 times
+//                  their weight whose V is 0, 3e-2 off.  2^13 to 2^15 would
+//                  keep three bits more, but moves b, and with it O, in nearly
+//                  every stage: 500 queries after 3500 positions 32.2 us with
+//                  2^0 or 2^7 .. 2^15, 31.4 to 33.3 here, 35.4 with 2^13.)
+// The groups' (b, l, O) are merged through LDS at the end; blocks that share a
 // row block's keys (gridDim.y of them) leave theirs to k_attention_prefill_merge.
 //
 // A stage costs about 3400 clocks with one wave per SIMD or two (8 waves): the
@@ -115,6 +123,7 @@ __global__ __launch_bounds__(256 * RG) void k_attention_prefill(
     constexpr int RPP = 64 / CPR;         // rows per 1 KB load
     constexpr int LP = KS / RPP / NW;     // loads of K (and of V) per wave and stage
     constexpr int DT = D / 16, DE = D / 32;
+    constexpr float kTopLog2 = 10.0f;     // log2 of a row's largest weight when b moves
     static_assert(KS / RPP % NW == 0, "whole loads per wave");
     constexpr int kStage = 2 * KS * D;    // halves: K rows, then V rows
     static_assert(kStage * 2 >= NW / 2 * 32 * D * 4, "half of the waves' O in each stage");
@@ -176,7 +185,7 @@ __global__ __launch_bounds__(256 * RG) void k_attention_prefill(
     h8 qf[DT];
 #pragma unroll
     for (int d = 0; d < DT; d++) qf[d] = *reinterpret_cast<const h8*>(q + q_off + 16 * d + 8 * hb);
-    float m = -1e30f, l = 0.0f;
+    float b = -1e30f, l = 0.0f;
     f16v o[DE];
 #pragma unroll
     for (int e = 0; e < DE; e++) o[e] = f16v{};
@@ -204,10 +213,10 @@ __global__ __launch_bounds__(256 * RG) void k_attention_prefill(
 #pragma unroll
         for (int i = 1; i < 16; i++) mx = fmaxf(mx, s[i]);
         mx = max_x32(mx) * scale_log2;
-        const bool up = mx > m + 8.0f;
+        const bool up = mx > b + (kTopLog2 + 5.0f);
         if (__any(up)) {
-            const float mn = up ? mx : m, corr = __builtin_amdgcn_exp2f(m - mn);
-            m = mn;
+            const float bn = fmaxf(mx - kTopLog2, b), corr = __builtin_amdgcn_exp2f(b - bn);
+            b = bn;
             l *= corr;
 #pragma unroll
             for (int e = 0; e < DE; e++) o[e] *= corr;
@@ -220,7 +229,7 @@ __global__ __launch_bounds__(256 * RG) void k_attention_prefill(
                 float p[2];
 #pragma unroll
                 for (int w = 0; w < 2; w++) {
-                    p[w] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[8 * u + j + w], scale_log2, -m));
+                    p[w] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[8 * u + j + w], scale_log2, -b));
                     l += p[w];
                 }
                 const h2 hi = __builtin_convertvector(f2{p[0], p[1]}, h2);
@@ -265,7 +274,7 @@ __global__ __launch_bounds__(256 * RG) void k_attention_prefill(
         return reinterpret_cast<f4*>((w < NW / 2 ? sm0 : sm1) + w % (NW / 2) * 64 * D) + r * (D / 4) + (c ^ (r & 15));
     };
     if (hb == 0) {
-        wm[wave][ln] = m;
+        wm[wave][ln] = b;
         wl[wave][ln] = l;
     }
     if (tid < ROWS) bad[tid] = 0;
