@@ -25,12 +25,16 @@ def npd(d):
     return np.float32 if d == F32 else np.float16
 
 
-def build(rng, M, Ns, K, d, same_x=True):
+def build(rng, M, Ns, K, d, same_x=True, outlier=0.0):
     dev, probs, refs = [], [], []
     x = rng.normal(0, 1, (M, K)).astype(npd(d))
+    if outlier:
+        x[:, K // 2] = outlier
     dx = capi.DevBuf.from_array(x)
     for i, N in enumerate(Ns):
         q = rng.integers(-127, 128, (N, K)).astype(np.int8)
+        if outlier:
+            q[:, K // 2] = 0
         s = rng.uniform(1e-4, 3e-4, N).astype(np.float32)
         b = rng.normal(0, 1, N).astype(np.float32) if i % 2 == 0 else None
         r = rng.normal(0, 1, (M, N)).astype(npd(d)) if i == 1 else None
@@ -105,6 +109,21 @@ def test_f32_few_rows(gpu, M, N, K):
     capi.sync()
     check(refs, M, K, F32)
     capi.call("vvh_plan_destroy", plan)
+
+
+@pytest.mark.parametrize("M,Ns,K", [(3, (896, 128), 4864), (5, (1536, 256, 256), 1536), (6, (4864, 4864), 896),
+                                    (15, (896, 128, 128), 4096), (8, (130,), 8960), (4, (9000, 9000), 1152)])
+def test_f32_few_rows_keep_small_activations(gpu, M, Ns, K):
+    """Fewer than 16 fp32 rows are used as they are: an activation 2^36 times
+    the others, under codes of 0, costs the others no bits."""
+    print(f"[case] f32 few rows, one large activation M={M} N={Ns} K={K}", flush=True)
+    plan, refs, dev = build(np.random.default_rng(M + K), M, Ns, K, F32, outlier=2.0 ** 36)
+    capi.call("vvh_plan_run", plan, None)
+    capi.sync()
+    check(refs, M, K, F32)
+    capi.call("vvh_plan_destroy", plan)
+    for N in Ns:
+        assert capi.kernel_choice(M, N, K, F32, F32) == "gemv_f32"
 
 
 def test_different_inputs_run_one_by_one(gpu):

@@ -412,20 +412,11 @@ int dot_depth(int64_t K, int ksplit)
 // rows on, when K % 64 == 0; below it k_gemv_f32, which streams the weights
 // once per 8 rows (gate/up 4864 x 896, graph replay: M = 8 13.7 against
 // 14.1 us on the GEMM, M = 16 17.0 against 14.2, M = 32 23.9 against 15.1).
+// Fewer rows stay there where the GEMM would be faster as well (M = 3 896 x 4864
+// 16.5 against 10.9 us, M = 6 9728 x 896 15.7 against 11.6): they are used as
+// they are, and an activation far below its row's largest would lose bits in
+// the split form.
 constexpr std::size_t kGemmF32MinM = 16;
-// ... and from fewer on long rows and large weights (K % 64 == 0), where
-// k_gemv_f32 reads its activations per weight tile, or streams the weights twice:
-// graph replay, k_gemv_f32 / GEMM: M = 3 896 x 4864 16.5 / 10.9 us, 1536 x 8960 29 / 14.9,
-// 17920 x 1536 22.4 / 20.2, 9728 x 896 9.2 / 11.5; M = 6 1536 x 1536 10.2 / 9.5, 9728 x 896 15.7 /
-// 11.6, 896 x 896 7.9 / 8.8; M = 2 896 x 4864 8.6 / 10.7.  The error against 64 bits is the
-// smaller of the two (K = 896 1.15e-7 / 1.21e-7, 1536 1.2e-7 / 1.9e-7, 8960 1.2e-7 / 3.1e-7).
-// Such a call takes k_gemv_f32 where the GEMM's workspace cannot be had (run_call).
-bool gemm_f32_few_rows(std::size_t M, std::size_t N, std::size_t K)
-{
-    if (K % kGemmBK != 0) return false;
-    const double nk = (double)N * (double)K;
-    return (M >= 5 && ((K >= 1024 && nk >= 2.3e6) || nk >= 8e6)) || (M >= 3 && (K >= 4096 || nk >= 20e6));
-}
 
 // Small-M fp16 dispatch, from a sweep of every family forced on each shape
 // (us per call on the GPU, calls replayed from HIP graphs; the bench.py
@@ -549,7 +540,7 @@ bool dot_call_takes_x_tile(int64_t M, int64_t N, int64_t K)
 int natural_kernel(std::size_t M, std::size_t N, std::size_t K, int act)
 {
     if (act == VVH_F32)
-        return (M >= kGemmF32MinM && K % kGemmBK == 0) || gemm_f32_few_rows(M, N, K) ? K_GEMM : K_GEMV_F32;
+        return M >= kGemmF32MinM && K % kGemmBK == 0 ? K_GEMM : K_GEMV_F32;
     const int64_t tiles = ((int64_t)N + kDecodeTileN - 1) / kDecodeTileN;
     const bool dot_ok = dot_fits((int64_t)N, (int64_t)K);
     if ((M <= kDotAutoMaxM || (M <= kDotAutoMfMaxM && tiles < kDotMfTiles)) && dot_ok) return K_DOT;
@@ -630,28 +621,10 @@ int validate_call(const void* out, const void* inp, const int8_t* w, const float
     return VVH_OK;
 }
 
-// Workspace of a GEMM call with K % 64 == 0: the split fp32 activations and their
-// row scales, and the k splits' planes.
-uint64_t gemm_ws_bytes(int64_t M, int64_t N, int64_t K, bool f32)
-{
-    int layout = 4;
-    const int64_t stages = (f32 ? 2 * K : K) / kGemmBK;
-    const int s = gemm_splits(M, N, stages, &layout);
-    return (f32 ? align_up((uint64_t)M * (uint64_t)K * 4) + align_up((uint64_t)M * 4) : 0) +
-           (s > 1 ? (uint64_t)s * (uint64_t)M * (uint64_t)N * 4 : 0);
-}
-
 int run_call(const LinArgs& base, int kernel, int act, int outd, void* stream, const WsSource* wsrc = nullptr)
 {
     LinArgs a = base;
     int e = 0;
-    if (kernel == K_GEMM && act == VVH_F32 && a.M < (int64_t)kGemmF32MinM && g_override.load() == K_AUTO) {
-        // few rows: without the workspace (a capture that cannot allocate, a
-        // fixed buffer too small) the kernel that needs none
-        const uint64_t bytes = gemm_ws_bytes(a.M, a.N, a.K, true);
-        float* ws = nullptr;
-        if (wsrc ? bytes > wsrc->bytes : !workspace_try(stream, bytes, &ws)) kernel = K_GEMV_F32;
-    }
     switch (kernel) {
         case K_GEMV_F32: {
             a.ksplit = choose_ksplit((a.N + kDecodeTileN - 1) / kDecodeTileN, a.K, kDotStep);
@@ -788,10 +761,7 @@ int plan_group(const std::vector<LinArgs>& args, int act)
         same = same && aligned && b.inp == a.inp && b.M == a.M && b.K == a.K;
         gemv = gemv && b.M == a.M && choose_kernel(b.M, b.N, b.K, act, aligned) == K_GEMV_F32;
     }
-    std::size_t n = 0;
-    for (const LinArgs& b : args) n += (std::size_t)b.N;
-    const bool rows = act == VVH_F32 ? natural_kernel((std::size_t)a.M, n, (std::size_t)a.K, act) == K_GEMM
-                                     : a.M > kSkinnyMaxM;
+    const bool rows = act == VVH_F32 ? a.M >= (int64_t)kGemmF32MinM : a.M > kSkinnyMaxM;
     if (same && a.K > 0 && a.K % kGemmBK == 0 && rows) return kGroupGemm;
     return gemv ? kGroupGemv : kGroupNone;
 }
