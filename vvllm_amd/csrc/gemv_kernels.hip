@@ -184,13 +184,32 @@ __device__ __forceinline__ void gemv_f32_body(const int8_t* __restrict__ w, cons
     }
 }
 
-// What the first loads depend on comes first (14 dwords, preloaded into
+// The grid row's pass of up to MT activation rows.  The rows past M of the last
+// one would cost what the others do, so it runs a body of 1, 2, 4, 6 or 8 rows
+// (graph replay, us, all passes of 8 -> these: M = 9 9728 x 896 23.6 -> 14.6, 17920 x
+// 1536 58.6 -> 42.4; M = 5 17920 x 1536 37.3 -> 29.7).
+template <int MT, typename OT, int D>
+__device__ __forceinline__ void gemv_f32_pass(const int8_t* __restrict__ w, const float* __restrict__ x, int64_t N,
+                                              int64_t K, int32_t ksplit, int64_t M, const LinArgs& a, int64_t block)
+{
+    const int64_t mbase = (int64_t)blockIdx.y * MT;
+    if constexpr (MT == 8) {
+        const int64_t rows = M - mbase;
+        if (rows == 1) return gemv_f32_body<1, OT, D>(w, x, N, K, ksplit, M, a, block, mbase);
+        if (rows == 2) return gemv_f32_body<2, OT, D>(w, x, N, K, ksplit, M, a, block, mbase);
+        if (rows <= 4) return gemv_f32_body<4, OT, D>(w, x, N, K, ksplit, M, a, block, mbase);
+        if (rows <= 6) return gemv_f32_body<6, OT, D>(w, x, N, K, ksplit, M, a, block, mbase);
+    }
+    gemv_f32_body<MT, OT, D>(w, x, N, K, ksplit, M, a, block, mbase);
+}
+
+// What the first loads depend on comes first (10 dwords, preloaded into
 // registers at dispatch).
 template <int MT, typename OT, int D>
 __global__ __launch_bounds__(256) void k_gemv_f32(const int8_t* __restrict__ w, const float* __restrict__ x, int64_t N,
                                                   int64_t K, int32_t ksplit, int32_t M, LinArgs a)
 {
-    gemv_f32_body<MT, OT, D>(w, x, N, K, ksplit, M, a, blockIdx.x, (int64_t)blockIdx.y * MT);
+    gemv_f32_pass<MT, OT, D>(w, x, N, K, ksplit, M, a, blockIdx.x);
 }
 
 // The problems of a plan (q, k and v of a decode layer) in one launch.
@@ -199,11 +218,13 @@ __global__ __launch_bounds__(256) void k_gemv_f32_group(LinGroup l)
 {
     const int b = blockIdx.x;
     const LinArgs a = l.g.p[(b >= l.b[0]) + (b >= l.b[1]) + (b >= l.b[2])];
-    gemv_f32_body<MT, OT, D>(a.w, static_cast<const float*>(a.inp), a.N, a.K, a.ksplit, a.M, a, b - a.block_begin,
-                             (int64_t)blockIdx.y * MT);
+    gemv_f32_pass<MT, OT, D>(a.w, static_cast<const float*>(a.inp), a.N, a.K, a.ksplit, a.M, a, b - a.block_begin);
 }
 
 namespace {
+
+// Rows of a pass: the fewest that take the call's, up to 8.
+int gemv_rows(int64_t M) { return M <= 2 ? (int)std::max<int64_t>(M, 1) : M <= 4 ? 4 : M <= 6 ? 6 : 8; }
 
 // Steps in flight: the wave's whole range where it is short (2, or 5 to 7 steps),
 // else 4 (see dot_depth).
@@ -239,13 +260,14 @@ void gemv_group_go(const LinGroup& l, int d, hipStream_t s)
 int launch_gemv_f32(const LinArgs& a, int out, void* stream)
 {
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const int mt = a.M <= 1 ? 1 : a.M <= 2 ? 2 : a.M <= 4 ? 4 : 8;
+    const int mt = gemv_rows(a.M);
     const int d = gemv_depth(a.K, a.ksplit, mt);
     auto go = [&]<typename OT>(OT*) {
         switch (mt) {
             case 1: gemv_go<1, OT>(a, d, s); break;
             case 2: gemv_go<2, OT>(a, d, s); break;
             case 4: gemv_go<4, OT>(a, d, s); break;
+            case 6: gemv_go<6, OT>(a, d, s); break;
             default: gemv_go<8, OT>(a, d, s); break;
         }
     };
@@ -258,7 +280,7 @@ int launch_gemv_f32_group(const LinGroup& l, int count, int out, void* stream)
 {
     hipStream_t s = static_cast<hipStream_t>(stream);
     const int64_t M = l.g.p[0].M;
-    const int mt = M <= 1 ? 1 : M <= 2 ? 2 : M <= 4 ? 4 : 8;
+    const int mt = gemv_rows(M);
     int d = 2;
     for (int i = 0; i < count; i++) d = std::max(d, gemv_depth(l.g.p[i].K, l.g.p[i].ksplit, 2));
     auto go = [&]<typename OT>(OT*) {
@@ -266,6 +288,7 @@ int launch_gemv_f32_group(const LinGroup& l, int count, int out, void* stream)
             case 1: gemv_group_go<1, OT>(l, d, s); break;
             case 2: gemv_group_go<2, OT>(l, d, s); break;
             case 4: gemv_group_go<4, OT>(l, d, s); break;
+            case 6: gemv_group_go<6, OT>(l, d, s); break;
             default: gemv_group_go<8, OT>(l, d, s); break;
         }
     };
