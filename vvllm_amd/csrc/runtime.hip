@@ -782,6 +782,7 @@ int run_group(const std::vector<LinArgs>& args, int group, int act, int outd, vo
     LinGroup l{};
     int64_t blocks = 0;
     if (group == kGroupGemv) {
+        if ((args[0].M + kGemvF32MaxM - 1) / kGemvF32MaxM > 65535) return VVH_OK;  // run_call refuses it
         int64_t tiles = 0;
         for (const LinArgs& a : args) tiles += (a.N + kDecodeTileN - 1) / kDecodeTileN;
         for (std::size_t i = 0; i < count; i++) {
