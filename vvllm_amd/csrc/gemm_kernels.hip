@@ -297,9 +297,13 @@ __global__ __launch_bounds__(64 * (BM / 32 / TI) * WN, BM == 64 || D < 4 ? 2 : 1
     for (int i = 0; i < TI; i++)
 #pragma unroll
         for (int j = 0; j < TJ; j++) acc[i][j] = f16v{};
-    // FOLD: every 8 stages the accumulators are added to a
-    // second set, so that a sum's chain of additions is short: error against 64 bits
-    // of an unsplit call of K = 896 1.6e-7 -> 1.1e-7, of K = 4864 4.0e-7 -> 1.3e-7, for 3% more time
+    // FOLD: every 2 stages the accumulators are added to a second set, so that a
+    // sum's chain of additions is short, also in a split of few stages.  Error against
+    // 64 bits, no folds / every 8 / every 2: M = 333, N = 4864, K = 896 3.1e-7 / 1.1e-7 /
+    // 0.9e-7, M = 500, N = 1536, K = 8960 5.7e-7 / 1.4e-7 / 1.7e-7; k and v of a prompt's
+    // plan (M = 100, 128 columns each, K = 896), which on their own are split over k more
+    // than the plan is (0.94e-7), 1.18e-7 every 8, 0.99e-7 every 4, 0.92e-7 here.  The times
+    // are alike (M = 333, 2 x 4864 x 896 25.3 us every 8, 25.2 every 2, 26.6 every stage).
     f16v sum[FOLD ? TI : 1][FOLD ? TJ : 1];
     if constexpr (FOLD) {
 #pragma unroll
@@ -338,6 +342,7 @@ __global__ __launch_bounds__(64 * (BM / 32 / TI) * WN, BM == 64 || D < 4 ? 2 : 1
         gemm3_slice<TJ, TI>(f.a[0], fb[0], acc, f.b[1], fb[1]);
         if constexpr (NEXT) gemm3_slice<TJ, TI>(f.a[1], fb[1], acc, frag(jn).b[0], fb[0]);
         else gemm3_slice_last<TJ, TI>(f.a[1], fb[1], acc);
+        if constexpr (FOLD && J % 2 == 1) fold();
     };
     // R steps from kt0 (kt0 % D == 0) with the problem's stage count kt0 + R
     auto steps = [&]<int R>(int64_t kt0) {
@@ -367,9 +372,6 @@ __global__ __launch_bounds__(64 * (BM / 32 / TI) * WN, BM == 64 || D < 4 ? 2 : 1
             [&]<int... J>(std::integer_sequence<int, J...>) {
                 (step.template operator()<J, true, true, (D - 2) * LPS>(kt0), ...);
             }(std::make_integer_sequence<int, U>{});
-            if constexpr (FOLD) {
-                if (kt0 & U) fold();
-            }
         }
         const int64_t r = nk - kt0;  // D .. U + D - 1
         [&]<int... R>(std::integer_sequence<int, R...>) {
