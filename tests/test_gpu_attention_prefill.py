@@ -88,6 +88,22 @@ def test_prefill_unseen_rows(gpu, n_q, len0, H, KVH, D, d, bad):
         assert not np.isfinite(got[n_q - 3:, H - 1, 5]).any()
 
 
+@pytest.mark.parametrize("n_q,len0,H,KVH,D,bound", [(333, 1, 14, 2, 64, 3.5e-7), (300, 67, 8, 8, 64, 4.2e-7),
+                                                    (500, 1, 12, 2, 128, 5.5e-7), (126, 20, 8, 1, 128, 4.6e-7)])
+def test_prefill_f32_error(gpu, n_q, len0, H, KVH, D, bound):
+    """fp32 attention is closer to 64 bits (2-norm) than one block per head and
+    query with a chain of head_dim products per score.  At these sizes 4.26e-7,
+    5.14e-7, 6.45e-7 and 5.76e-7 in one chain per score and per lane's weights
+    (that form: 0 to 3% less), 2.79e-7, 3.31e-7, 4.01e-7 and 3.52e-7 in two
+    chains and with the weights summed by stages."""
+    print(f"[case] fp32 error n_q={n_q} len0={len0} H={H} D={D}", flush=True)
+    q, k, v, scale = draw(n_q, len0, H, KVH, D, F32)
+    got, ref = run(q, k, v, len0, scale, F32), reference(q, k, v, len0, scale)
+    e = np.linalg.norm(got - ref) / np.linalg.norm(ref)
+    print(f"error {e:.3e}")
+    assert e <= bound
+
+
 @pytest.mark.parametrize("n_q,len0,H,KVH,D", [(40, 1, 14, 2, 64), (700, 1, 12, 2, 128), (33, 3000, 12, 2, 128)])
 @pytest.mark.parametrize("d", [F32, F16])
 @pytest.mark.parametrize("gap", [12, 18, 22, 26])
