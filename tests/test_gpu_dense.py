@@ -68,3 +68,21 @@ def test_dense_rows_nonfinite(gpu, d):
     capi.sync()
     fin = np.isfinite(do.to_array(npd(d), (M, N)))
     assert not fin[M - 1].any() and not fin[:, N - 1].any() and fin[:M - 1, :N - 1].all()
+
+
+@pytest.mark.parametrize("M,N,K,bound", [(200, 256, 256, 7.95e-8), (306, 1536, 432, 8.4e-8), (64, 512, 512, 8.4e-8),
+                                         (128, 1000, 896, 8.7e-8)])
+def test_dense_f32_error(gpu, M, N, K, bound):
+    """Closer to 64 bits (2-norm) than a wave per weight row with 64 lanes and
+    a butterfly: at these sizes 8.16e-8, 8.68e-8, 8.64e-8 and 8.93e-8 with the
+    waves' sums added in 32 bits (the butterfly 1 to 2% less up to K = 512),
+    7.63e-8, 8.20e-8, 8.17e-8 and 8.45e-8 in 64."""
+    rng = np.random.default_rng(M + K)
+    x, w = rng.normal(0, 1, (M, K)).astype(np.float32), rng.normal(0, 0.1, (N, K)).astype(np.float32)
+    dx, dw, do = capi.DevBuf.from_array(x), capi.DevBuf.from_array(w), capi.DevBuf(M * N * 4)
+    capi.call("vvh_dense", do.ptr, dx.ptr, dw.ptr, F32, None, None, M, N, K, F32, None)
+    capi.sync()
+    y = x.astype(np.float64) @ w.astype(np.float64).T
+    e = np.linalg.norm(do.to_array(np.float32, (M, N)) - y) / np.linalg.norm(y)
+    print(f"error {e:.3e}")
+    assert e <= bound

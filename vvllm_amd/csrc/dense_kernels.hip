@@ -86,10 +86,12 @@ __device__ __forceinline__ void dense_store4(T* out, const T* res, const float* 
 //
 // fp32: v_mfma_f32_32x32x2_f32, exact products, fp32 sums.  Four accumulators
 // take turns, and every 4 stages they are added to a fifth, so a chain runs over
-// 4 products' additions and then K / 128: with the four waves' sums that is closer to
-// 64 bits than the vector form's 64 lanes and their butterfly (relative error,
-// 2-norm: K = 896 9.3e-8 against 9.8e-8, 1536 9.4e-8 against 1.1e-7, 4864 1.1e-7
-// against 1.7e-7; two accumulators, folded every 4 or 2 stages, 1.0e-7 at K = 896).
+// 4 products' additions and then K / 128; the four waves' sums are added in 64
+// bits.  That is closer to 64 bits than the vector form's 64 lanes and their
+// butterfly at every K (relative error, 2-norm: K = 256 7.7e-8 against 8.1e-8, 512
+// 8.2e-8 against 8.5e-8, 896 8.9e-8 against 9.8e-8, 4864 1.0e-7 against 1.7e-7; with
+// the waves' sums added in 32 bits 8.2e-8 and 8.7e-8 at K = 256 and 512, in the
+// same time; two accumulators, folded every 4 or 2 stages, 1.0e-7 at K = 896).
 // Bound by the fp32 matrix rate (256 flop per clock and CU) where the tiles fill
 // the chip.
 // fp16: v_mfma_f32_32x32x16_f16; bound by the fill of LDS.
@@ -269,7 +271,11 @@ __global__ __launch_bounds__(256, 2) void k_dense_mfma(const T* __restrict__ x, 
     lds_barrier();
     for (int idx = tid; idx < BM * BN / 4; idx += 256) {
         const int m = idx / (BN / 4), q = idx % (BN / 4);
-        store(m0 + m, n0 + 4 * q, (*at(0, m, q) + *at(1, m, q)) + (*at(2, m, q) + *at(3, m, q)));
+        const f4 y0 = *at(0, m, q), y1 = *at(1, m, q), y2 = *at(2, m, q), y3 = *at(3, m, q);
+        f4 y;
+#pragma unroll
+        for (int e = 0; e < 4; e++) y[e] = (float)(((double)y0[e] + y1[e]) + ((double)y2[e] + y3[e]));
+        store(m0 + m, n0 + 4 * q, y);
     }
 }
 
