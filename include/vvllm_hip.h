@@ -291,7 +291,7 @@ VVH_API int vvh_linear_q8_dev_in(void* out, const void* inp, const int8_t* dev_w
  * decomposition, device-resident descriptor table) and launched with
  * vvh_plan_run as a single kernel when every problem takes the decode path
  * (M <= 16), or when its problems read the same activations and take the
- * GEMM, or are fp32 of few rows (a GEMM of fp32 activations or of split k adds
+ * GEMM (not from fp16 to fp32), or are fp32 of few rows (a GEMM of fp32 activations or of split k adds
  * its split and reduction launches, and without their workspace, as in a
  * capture that cannot allocate, the problems run one by one); else as one
  * launch per problem.  It is the counterpart of the

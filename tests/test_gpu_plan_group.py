@@ -145,6 +145,30 @@ def test_f32_group_error(gpu, M, Ns, K):
     capi.call("vvh_plan_destroy", plan)
 
 
+@pytest.mark.parametrize("M,Ns,K", [(59, (1600, 64, 384), 960), (847, (448, 256, 64), 1728), (41, (1362, 1362), 512)])
+def test_fp16_to_fp32_runs_one_by_one(gpu, M, Ns, K):
+    """fp16 activations with fp32 outputs keep the sums, and the bits, of a
+    problem alone: a group's fewer k splits would show in 32 bits."""
+    print(f"[case] fp16 to fp32 M={M} N={Ns} K={K}", flush=True)
+    rng = np.random.default_rng(M)
+    dx = capi.DevBuf.from_array(rng.normal(0, 1, (M, K)).astype(np.float16))
+    dev = [(capi.DevBuf.from_array(rng.integers(-127, 128, (N, K)).astype(np.int8)),
+            capi.DevBuf.from_array(rng.uniform(1e-4, 3e-4, N).astype(np.float32)), capi.DevBuf(M * N * 4), capi.DevBuf(M * N * 4))
+           for N in Ns]
+    probs = [capi.Q8Problem(out=o.ptr, inp=dx.ptr, residual=None, weight=q.ptr, scales=s.ptr, bias=None, M=M, N=N, K=K)
+             for (q, s, o, _), N in zip(dev, Ns)]
+    h = ctypes.c_uint64()
+    capi.call("vvh_plan_create", (capi.Q8Problem * len(Ns))(*probs), len(Ns), F16, F32, ctypes.byref(h))
+    assert launches(h.value) == len(Ns)
+    capi.call("vvh_plan_run", h.value, None)
+    for (q, s, _, o), N in zip(dev, Ns):
+        capi.linear_q8_dev(o, dx, q, s, None, None, M, N, K, F16, F32)
+    capi.sync()
+    capi.call("vvh_plan_destroy", h.value)
+    for (_, _, a, b), N in zip(dev, Ns):
+        assert np.array_equal(a.to_array(np.float32, (M, N)), b.to_array(np.float32, (M, N)))
+
+
 def test_different_inputs_run_one_by_one(gpu):
     plan, refs, dev = build(np.random.default_rng(9), 100, (128, 192), 512, F16, same_x=False)
     assert launches(plan) == 2

@@ -749,11 +749,15 @@ int run_call(const LinArgs& base, int kernel, int act, int outd, void* stream, c
 // 18.6 -> 7.0 us, gate and up 21.8 -> 17.4; 1.5B q/k/v at M = 2048 34.2 -> 18.8, 0.5B at M =
 // 64 (three k_skinny launches before) 30.8 -> 6.5; fp32 q/k/v at M = 333 35.5 -> 15.1, gate
 // and up 35.1 -> 26.7, q/k/v at M = 1 9.3 -> 3.9.
+// fp16 activations with fp32 outputs stay one by one: a group's k is split less
+// than a problem's on its own, and their sums are not folded (error against 64
+// bits of M = 59, 1600 + 64 + 384 columns of K = 960 7.7e-8 one by one, 1.56e-7 in a
+// group, 7.9e-8 in one of folded sums).
 constexpr int kGroupNone = 0, kGroupGemm = 1, kGroupGemv = 2;
 
-int plan_group(const std::vector<LinArgs>& args, int act)
+int plan_group(const std::vector<LinArgs>& args, int act, int outd)
 {
-    if (args.size() < 2 || args.size() > (std::size_t)kDotInline) return kGroupNone;
+    if (args.size() < 2 || args.size() > (std::size_t)kDotInline || (act == VVH_F16 && outd == VVH_F32)) return kGroupNone;
     const LinArgs& a = args[0];
     bool same = true, gemv = act == VVH_F32;
     for (const LinArgs& b : args) {
@@ -1678,7 +1682,7 @@ VVH_API int vvh_plan_create(const vvh_q8_problem* problems, size_t count, int ac
             return fail_hip(e, "plan table upload");
         }
     }
-    if (!p.dot && !p.stream && !p.grouped && ov == K_AUTO) p.group = plan_group(p.args, act_dtype);
+    if (!p.dot && !p.stream && !p.grouped && ov == K_AUTO) p.group = plan_group(p.args, act_dtype, out_dtype);
     std::lock_guard<std::mutex> lock(g_pmu);
     const vvh_plan h = g_next_plan++;
     g_plans.emplace(h, std::move(p));
