@@ -32,7 +32,7 @@ def reference(x, w, b, r):
 
 
 CASES = [(5, 64, 8), (9, 64, 8), (6, 70, 2052 * 4), (31, 63, 64), (32, 65, 72), (33, 130, 896), (64, 896, 4864), (65, 200, 2056), (128, 128, 32),
-         (129, 1000, 1000), (300, 9728, 136), (512, 8200, 896), (7, 40, 4864), (100, 33, 8960)]
+         (129, 1000, 1000), (5, 512, 512), (7, 1100, 896), (10, 1024, 1024), (300, 9728, 136), (512, 8200, 896), (7, 40, 4864), (100, 33, 8960)]
 
 
 @pytest.mark.parametrize("d", [F32, F16])

@@ -302,13 +302,26 @@ __global__ __launch_bounds__(256) void k_dense_reduce(const float* __restrict__ 
 
 // Calls the MFMA form takes: both types alike, 5 rows or more, rows of whole
 // 16-byte chunks, aligned, and sizes in 31 bits (rows and byte offsets within a
-// tile of 64 rows).  fp32 calls of 5 to 8 rows over short rows keep the vector
-// form, two passes over the weights (graph replay: 5 x 4864 x 896 9.2 us against
-// 10.8, 8 x 896 x 896 7.6 against 8.3).
+// tile of 64 rows).  Few rows over short ones keep the vector form, two or
+// three passes over the weights, where that is faster (graph replay, us, against
+// this form): fp32 calls of 5 to 8 rows over up to 2048 values (5 x 4864 x 896 9.2
+// against 10.8, 8 x 896 x 896 7.6 against 8.3) and of 9 and 10 over small weights (9
+// x 512 x 512 6.2 against 6.9, 9 / 10 x 896 x 896 7.4 / 7.8 against 7.9; 9 x 1200 x 1024
+// 8.0 against 7.5) or of 11 over about 512 (11 x 1000 x 512 6.8 against 7.0); fp16
+// calls of 5 to 8 rows over 769 to 1024 values (5 / 8 x 896 x 896 5.7 / 6.9 against 7.2, 6
+// x 3000 x 1024 6.9 against 7.8, 8 x 2000 x 1000 7.4 against 7.8; 8 x 2400 x 896 7.6
+// against 7.2), and over small weights of 5 and 6 rows from 512 on (5 x 512 x 512 4.8
+// against 5.3) and of 5 up to 1536 (512 x 1536 6.5 against 6.8).
 bool dense_mfma_ok(const void* x, const void* w, int wdtype, int64_t M, int64_t N, int64_t K, int dtype)
 {
     const int64_t es = dtype == VVH_F16 ? 2 : 4;
-    if (dtype == VVH_F32 && M <= 8 && K <= 2048) return false;
+    const int64_t nk = N * K;
+    if (dtype == VVH_F32 && ((M <= 8 && K <= 2048) || (M <= 10 && K <= 1024 && nk <= 900000) ||
+                             (M <= 11 && K > 384 && K <= 512 && nk <= 600000)))
+        return false;
+    if (dtype == VVH_F16 && ((M <= 8 && K > 768 && K <= 1024 && nk <= (M <= 6 ? 3300000 : M == 7 ? 3100000 : 2100000)) ||
+                             (M <= 6 && K >= 512 && K <= (M == 5 ? 1536 : 768) && nk <= (1 << 20))))
+        return false;
     return dtype == wdtype && M > 4 && K > 0 && K % (16 / es) == 0 &&
            ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w)) & 15) == 0 && M <= (1 << 30) &&
            N <= (1 << 30) && K * es * 64 < ((int64_t)1 << 31) && (M + 31) / 32 * ((N + 63) / 64) <= (1 << 30);
