@@ -20,15 +20,23 @@
  *     Launches are asynchronous on it; errors of the launch itself are
  *     reported, errors of the kernel's execution surface at the next
  *     synchronising call.
- *   - Split-K GEMMs, fp32-activation GEMMs (M * K * 4 + M * 4 bytes for the
- *     split activations), multi-chunk decode attention and multi-block
- *     sampling use a per-stream workspace that grows on demand (hipMalloc, to at
- *     least twice its size, never below 1 MiB).  Under HIP graph capture it
- *     cannot grow: run the same calls once on that stream before capturing
- *     (decode attention needs at most 512 * (num_heads / num_kv_heads) *
- *     (head_dim + 2) * 4 bytes, 4.3 MB, at any span).  A buffer the
- *     workspace outgrows is kept, not freed, so graphs captured before the
- *     growth stay valid; vvh_workspace_release frees them all.
+ *   - A per-stream workspace that grows on demand (hipMalloc, to at least
+ *     twice its size, never below 1 MiB) serves split-K GEMMs and
+ *     fp32-activation GEMMs (M * K * 4 + M * 4 bytes for the split activations),
+ *     single or in plans, multi-chunk decode attention, multi-block sampling,
+ *     and outside of captures vvh_dense of more than 4 rows and vvh_attention
+ *     of several queries, where they split k or the keys.  Under HIP graph
+ *     capture it cannot grow: run the same calls once on that stream before
+ *     capturing (decode attention needs at most 512 * (num_heads /
+ *     num_kv_heads) * (head_dim + 2) * 4 bytes, 4.3 MB, at any span).  A buffer
+ *     the workspace outgrows is kept, not freed, so graphs captured before the
+ *     growth stay valid; vvh_workspace_release frees them all.  A graph of
+ *     calls that use the workspace holds it: replay it on the capturing stream,
+ *     or while that stream runs no such call, and not after
+ *     vvh_workspace_release.  vvh_dense and vvh_attention of several queries
+ *     leave it alone while the stream is being captured (they do not split:
+ *     other sums, so other last bits, and slower where they would), so their
+ *     graphs may be replayed anywhere.
  *   - All calls may be made from one host thread at a time per device
  *     (as the reference, which is single-threaded, README.md:282); the
  *     allocator and registries are internally locked.
@@ -447,9 +455,10 @@ VVH_API int vvh_embedding(void* out, const float* dev_table, size_t token_id, si
  * 16-byte aligned attends to up to 2^30 positions.  A single query over a
  * span long enough to split across blocks uses the stream's workspace, which
  * a call may have to allocate: make one of that size before capturing graphs on
- * the stream.  Several queries use the workspace to split the keys over more
- * blocks where that fills the device, and do without it where it cannot grow
- * (during a capture). */
+ * the stream (a smaller workspace gives fewer, longer blocks, and so other
+ * last bits, where it is large enough for those).  Several queries use the
+ * workspace to split the keys over more blocks where that fills the device,
+ * and do not split in a capture or where it cannot grow. */
 VVH_API int vvh_attention(void* out, const void* q, const void* k, const void* v, size_t n_q, size_t len0,
                           size_t num_heads, size_t num_kv_heads, size_t head_dim, float scale, int dtype,
                           void* stream);
@@ -479,7 +488,9 @@ VVH_API int vvh_linear_q8_dev_attn(void* out, const float* parts, size_t nparts,
                                    const void* residual, size_t N, size_t K, int out_dtype, void* stream);
 /* Dense linear with fp32 or fp16 weights (wdtype): out[M,N] = x[M,K] . W[N,K]^T
  * + bias[N] (+ residual[M,N], may alias out) -- Backend::linear / linear_add
- * (:139-156, :302-320); the fp32 model path and the tied LM head. */
+ * (:139-156, :302-320); the fp32 model path and the tied LM head.  More than 4
+ * rows may split k, with the partial sums in the stream's workspace, outside of
+ * captures and where it can grow. */
 VVH_API int vvh_dense(void* out, const void* x, const void* dev_weight, int wdtype, const float* dev_bias,
                       const void* residual, size_t M, size_t N, size_t K, int dtype, void* stream);
 /* out[M,N] = A[M,K] . B[K,N], B fp32 row-major (:25-42). */

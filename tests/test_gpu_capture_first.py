@@ -21,6 +21,7 @@ def hip():
     lib = ctypes.CDLL("libamdhip64.so.7")
     for name, args in {"hipStreamCreate": [ctypes.POINTER(V)], "hipStreamSynchronize": [V], "hipStreamDestroy": [V],
                        "hipStreamBeginCapture": [V, ctypes.c_int], "hipStreamEndCapture": [V, ctypes.POINTER(V)],
+                       "hipGraphGetNodes": [V, V, ctypes.POINTER(ctypes.c_size_t)],
                        "hipGraphInstantiate": [ctypes.POINTER(V), V, V, V, ctypes.c_size_t],
                        "hipGraphLaunch": [V, V], "hipGraphExecDestroy": [V], "hipGraphDestroy": [V]}.items():
         getattr(lib, name).argtypes = args
@@ -110,3 +111,46 @@ def test_captured_without_a_workspace(gpu, name):
         assert np.linalg.norm(y - ref) <= tol * np.linalg.norm(ref)
     assert lib.hipGraphExecDestroy(ex) == 0 and lib.hipGraphDestroy(graph) == 0
     assert lib.hipStreamDestroy(stream) == 0
+
+
+@pytest.mark.parametrize("name", ["attention_f16", "attention_f32", "dense_f16", "dense_f32", "dense_few_f32", "attention_short_f32"])
+def test_graph_holds_no_workspace(gpu, name):
+    """A captured vvh_dense, or vvh_attention of several queries, is one kernel
+    off the stream's workspace, also where the stream has one: its graph may be
+    replayed on another stream while the capturing one runs the same call, and
+    after vvh_workspace_release."""
+    print(f"[case] graph without workspace: {name}", flush=True)
+    lib = hip()
+    more = {"dense_few_f32": lambda r: dense(r, F32, 12, 896, 4864),  # these keep the forms without splits
+            "attention_short_f32": lambda r: attention(r, F32, 8, 400, 12, 2, 128)}
+    keep, shape, dt, run = {**CASES, **more}[name](np.random.default_rng(len(name)))
+    size = int(np.prod(shape)) * np.dtype(dt).itemsize
+    want, got = capi.DevBuf(size), capi.DevBuf(size)
+    first, other, graph, ex = V(), V(), V(), V()
+    assert lib.hipStreamCreate(ctypes.byref(first)) == 0 and lib.hipStreamCreate(ctypes.byref(other)) == 0
+    run(want, first)  # the stream has a workspace of the call's size
+    capi.sync()
+    ref = want.to_array(dt, shape).astype(np.float64)
+    assert lib.hipStreamBeginCapture(first, 1) == 0
+    run(got, first)
+    assert lib.hipStreamEndCapture(first, ctypes.byref(graph)) == 0
+    n = ctypes.c_size_t()
+    assert lib.hipGraphGetNodes(graph, None, ctypes.byref(n)) == 0
+    assert n.value == 1  # a split call is two
+    assert lib.hipGraphInstantiate(ctypes.byref(ex), graph, None, None, 0) == 0
+    zero = np.zeros(shape, dt)
+    for released in (False, False, True, True):
+        if released:
+            capi.call("vvh_workspace_release", first)
+        capi.call("vvh_memcpy_h2d", got.ptr, zero.ctypes.data, size)
+        assert lib.hipGraphLaunch(ex, other) == 0
+        if not released:
+            run(want, first)
+        assert lib.hipStreamSynchronize(other) == 0
+        capi.sync()
+        # the same sums in another order, as in test_captured_without_a_workspace
+        tol = 2.0 ** -10 if dt == np.float16 else 2e-6
+        assert np.linalg.norm(got.to_array(dt, shape).astype(np.float64) - ref) <= tol * np.linalg.norm(ref)
+        assert np.array_equal(want.to_array(dt, shape).astype(np.float64), ref)
+    assert lib.hipGraphExecDestroy(ex) == 0 and lib.hipGraphDestroy(graph) == 0
+    assert lib.hipStreamDestroy(first) == 0 and lib.hipStreamDestroy(other) == 0

@@ -657,6 +657,20 @@ AttnPrefillPlan attention_prefill_plan(int64_t n_q, int64_t len0, int64_t H, int
     return best;
 }
 
+// Whether a call that would split its keys and has no workspace for the partials
+// gives each row block all its keys, or takes k_attention.  fp32 tiles of few rows
+// over short spans lose (graph replay, us, k_attention / unsplit: 8 queries after 400
+// positions, 12 heads of 128, 29.3 / 40.9, after 1500 98.8 / 121.6, after 2500 335 / 197, 8 on
+// 8 of 128 163 / 191; 100 queries 62.5 / 46.7, after 100 25.0 / 27.5; 8, 14 of 64, after 250
+// 12.4 / 13.6, after 400 16.7 / 16.8); fp16 tiles do not (4 after 1000, 12 of 128, 60.4 / 14.7).
+bool attention_prefill_unsplit_pays(int64_t n_q, int64_t len0, int64_t H, int64_t KVH, int64_t D, int dtype)
+{
+    if (dtype != VVH_F32) return true;
+    const int64_t span = len0 + n_q - 1, blocks = n_q * H;
+    if (D == 64) return blocks > 512 || span > 300;
+    return blocks > 512 ? blocks > 1300 || span > 200 : span > (H == KVH ? 3000 : 2048);
+}
+
 int64_t attention_prefill_ws_floats(const AttnPrefillPlan& p, int64_t n_q, int64_t H, int64_t D)
 {
     return p.splits > 1 ? p.splits * n_q * H * (D + 2) : 0;

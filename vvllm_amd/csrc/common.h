@@ -353,6 +353,7 @@ struct AttnPrefillPlan {
 };
 AttnPrefillPlan attention_prefill_plan(int64_t n_q, int64_t len0, int64_t H, int64_t KVH, int64_t D, int dtype,
                                        int64_t cus);
+bool attention_prefill_unsplit_pays(int64_t n_q, int64_t len0, int64_t H, int64_t KVH, int64_t D, int dtype);
 int64_t attention_prefill_ws_floats(const AttnPrefillPlan& p, int64_t n_q, int64_t H, int64_t D);
 int launch_attention_prefill(const AttnPrefillPlan& p, void* out, const void* q, const void* k, const void* v,
                              int64_t n_q, int64_t len0, int64_t H, int64_t KVH, int64_t D, float scale, int dtype,
@@ -392,6 +393,7 @@ struct DensePlan {
 };
 bool dense_mfma_ok(const void* x, const void* w, int wdtype, int64_t M, int64_t N, int64_t K, int dtype);
 DensePlan dense_plan(int64_t M, int64_t N, int64_t K, int dtype, int64_t cus);
+bool dense_unsplit_pays(const DensePlan& p, int64_t M, int64_t N, int64_t K, int dtype, int64_t cus);
 int64_t dense_ws_floats(const DensePlan& p, int64_t M, int64_t N);
 int launch_dense_mfma(const DensePlan& p, void* out, const void* x, const void* w, const float* bias, const void* res,
                       int64_t M, int64_t N, int64_t K, int dtype, float* ws, void* stream);

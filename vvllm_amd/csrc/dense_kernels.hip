@@ -353,6 +353,21 @@ DensePlan dense_plan(int64_t M, int64_t N, int64_t K, int dtype, int64_t cus)
     return p;
 }
 
+// Whether a call that would split k and has no workspace for the planes takes a
+// tile's whole k in one block, or the vector form: its passes over the weights
+// (2.5 us and 0.42 ns per row and value, on 2200 weight rows and more in
+// proportion) against the chain of stages.  Graph replay, us, vector / unsplit:
+// fp32 896 x 4864, 5 rows 16.6 / 70, 24 47.7 / 70.6, 32 67 / 70.6; fp16 5 13.4 / 26.0, 10 23.0 /
+// 25.9, 12 27 / 26; 4864 x 896 fp32 12 rows 13.3 / 15.5.
+bool dense_unsplit_pays(const DensePlan& p, int64_t M, int64_t N, int64_t K, int dtype, int64_t cus)
+{
+    const bool f16 = dtype == VVH_F16;
+    const int64_t stages = (K + (f16 ? 63 : 31)) / (f16 ? 64 : 32), t = (M + p.bm - 1) / p.bm * ((N + 63) / 64);
+    const double b = (double)((t + cus - 1) / cus);
+    return (double)stages * (0.1 + (f16 ? 0.24 : 0.39) * b) <=
+           2.5 + 4.2e-4 * (double)M * (double)K * std::max(1.0, (double)N / 2200.0);
+}
+
 int64_t dense_ws_floats(const DensePlan& p, int64_t M, int64_t N) { return p.splits > 1 ? p.splits * M * N : 0; }
 
 template <typename T, int BM>

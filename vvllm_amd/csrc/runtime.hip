@@ -120,8 +120,8 @@ std::unordered_map<vvh_plan, Plan> g_plans;
 vvh_plan g_next_plan = 1;
 
 // ---- split-K workspace ------------------------------------------------------
-// fp32 partial sums of split GEMMs and the partials of multi-block decode
-// attention and sampling, one buffer per stream (calls on one stream run in
+// fp32 partial sums of split GEMMs and dense linears, split fp32 activations
+// and the partials of attention and sampling over many blocks, one buffer per stream (calls on one stream run in
 // order, so they can share it; calls on different streams never do).  Grown
 // on demand to at least twice its size; a buffer it outgrows is retired, not
 // freed, because a HIP graph captured earlier on the stream still holds its
@@ -156,22 +156,25 @@ int workspace_for(void* stream, std::size_t bytes, float** out)
 }
 
 // The stream's workspace of `bytes`, for calls that can do without: false
-// where it would have to grow while the stream is being captured, or cannot.
-bool workspace_try(void* stream, std::size_t bytes, float** ws)
+// where it cannot grow, and while the stream is being captured.  A graph that
+// holds no workspace may be replayed on any stream, next to the capturing
+// stream's own calls and after vvh_workspace_release.  captured: calls whose
+// graphs do hold it, like those of workspace_for, take it in a capture as well if
+// it is large enough.
+bool workspace_try(void* stream, std::size_t bytes, float** ws, bool captured = false)
 {
-    bool have;
-    {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(static_cast<hipStream_t>(stream), &st) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    if (st != hipStreamCaptureStatusNone) {
+        if (!captured) return false;
         std::lock_guard<std::mutex> lock(g_wsmu);
         const auto it = g_ws.find(stream);
-        have = it != g_ws.end() && it->second.bytes >= bytes;
-    }
-    if (!have) {
-        hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing(static_cast<hipStream_t>(stream), &st) != hipSuccess) {
-            (void)hipGetLastError();
-            return false;
-        }
-        if (st != hipStreamCaptureStatusNone) return false;
+        if (it == g_ws.end() || it->second.bytes < bytes) return false;
+        *ws = static_cast<float*>(it->second.p);
+        return true;
     }
     return workspace_for(stream, bytes, ws) == VVH_OK;
 }
@@ -824,7 +827,7 @@ int run_group(const std::vector<LinArgs>& args, int group, int act, int outd, vo
     }
     if (sp > 1 && !mul_ok((uint64_t)M * (uint64_t)n, (uint64_t)sp * 4, &plane)) return VVH_OK;
     float* ws = nullptr;
-    if (xs + rs + plane > 0 && !workspace_try(stream, xs + rs + plane, &ws)) return VVH_OK;
+    if (xs + rs + plane > 0 && !workspace_try(stream, xs + rs + plane, &ws, true)) return VVH_OK;
     char* wb = reinterpret_cast<char*>(ws);
     float* wp = reinterpret_cast<float*>(wb + xs + rs);
     for (std::size_t i = 0; i < count; i++) {
@@ -2160,7 +2163,7 @@ VVH_API int vvh_attention(void* out, const void* q, const void* k, const void* v
                                                  (int64_t)head_dim, dtype, false);
         float* ws = nullptr;
         int64_t wsf = attention_decode_ws_floats(p, (int64_t)num_heads, (int64_t)head_dim);
-        if (p.mfma && wsf > 0 && !workspace_try(stream, (std::size_t)wsf * 4, &ws)) {
+        if (p.mfma && wsf > 0 && !workspace_try(stream, (std::size_t)wsf * 4, &ws, true)) {
             p = attention_decode_plan(q, (int64_t)len0, (int64_t)num_heads, (int64_t)num_kv_heads, (int64_t)head_dim,
                                       dtype, true);
             wsf = attention_decode_ws_floats(p, (int64_t)num_heads, (int64_t)head_dim);
@@ -2178,14 +2181,18 @@ VVH_API int vvh_attention(void* out, const void* q, const void* k, const void* v
         AttnPrefillPlan p = attention_prefill_plan((int64_t)n_q, (int64_t)len0, (int64_t)num_heads,
                                                    (int64_t)num_kv_heads, (int64_t)head_dim, dtype,
                                                    g_cu_count > 0 ? g_cu_count : 256);
-        // splits need the stream's workspace; without it (a capture that
-        // cannot allocate, no memory) each block takes all its keys
+        // splits need the stream's workspace; without it (a capture, no memory)
+        // each block takes all its keys
         float* ws = nullptr;
         const int64_t wsf = attention_prefill_ws_floats(p, (int64_t)n_q, (int64_t)num_heads, (int64_t)head_dim);
-        if (wsf > 0 && !workspace_try(stream, (std::size_t)wsf * 4, &ws)) p.splits = 1;
-        return ret_launch(launch_attention_prefill(p, out, q, k, v, (int64_t)n_q, (int64_t)len0, (int64_t)num_heads,
-                                                   (int64_t)num_kv_heads, (int64_t)head_dim, scale, dtype, ws, stream),
-                          "attention launch");
+        const bool lacks = wsf > 0 && !workspace_try(stream, (std::size_t)wsf * 4, &ws);
+        if (lacks) p.splits = 1;
+        if (!lacks || attention_prefill_unsplit_pays((int64_t)n_q, (int64_t)len0, (int64_t)num_heads,
+                                                     (int64_t)num_kv_heads, (int64_t)head_dim, dtype))
+            return ret_launch(launch_attention_prefill(p, out, q, k, v, (int64_t)n_q, (int64_t)len0,
+                                                       (int64_t)num_heads, (int64_t)num_kv_heads, (int64_t)head_dim,
+                                                       scale, dtype, ws, stream),
+                              "attention launch");
     }
     return ret_launch(launch_attention(out, q, k, v, (int64_t)n_q, (int64_t)len0, (int64_t)num_heads,
                                        (int64_t)num_kv_heads, (int64_t)head_dim, scale, dtype, stream),
@@ -2233,14 +2240,18 @@ VVH_API int vvh_dense(void* out, const void* x, const void* dev_weight, int wdty
     if ((N + 3) / 4 > INT32_MAX) return fail(VVH_ERR_UNSUPPORTED, "N too large");
     REQUIRE_INIT();
     if (dense_mfma_ok(x, dev_weight, wdtype, (int64_t)M, (int64_t)N, (int64_t)K, dtype)) {
-        DensePlan p = dense_plan((int64_t)M, (int64_t)N, (int64_t)K, dtype, g_cu_count > 0 ? g_cu_count : 256);
-        // k splits need the stream's workspace; without it one block takes all of a tile's k
+        const int64_t cus = g_cu_count > 0 ? g_cu_count : 256;
+        DensePlan p = dense_plan((int64_t)M, (int64_t)N, (int64_t)K, dtype, cus);
+        // k splits need the stream's workspace; without it (a capture, no memory)
+        // one block takes all of a tile's k
         float* ws = nullptr;
         const int64_t wsf = dense_ws_floats(p, (int64_t)M, (int64_t)N);
-        if (wsf > 0 && !workspace_try(stream, (std::size_t)wsf * 4, &ws)) p.splits = 1;
-        return ret_launch(launch_dense_mfma(p, out, x, dev_weight, dev_bias, residual, (int64_t)M, (int64_t)N, (int64_t)K,
-                                            dtype, ws, stream),
-                          "dense launch");
+        const bool lacks = wsf > 0 && !workspace_try(stream, (std::size_t)wsf * 4, &ws);
+        if (lacks) p.splits = 1;
+        if (!lacks || dense_unsplit_pays(p, (int64_t)M, (int64_t)N, (int64_t)K, dtype, cus))
+            return ret_launch(launch_dense_mfma(p, out, x, dev_weight, dev_bias, residual, (int64_t)M, (int64_t)N,
+                                                (int64_t)K, dtype, ws, stream),
+                              "dense launch");
     }
     return ret_launch(launch_dense(out, x, dev_weight, wdtype, dev_bias, residual, (int64_t)M, (int64_t)N, (int64_t)K,
                                    dtype, stream),
