@@ -299,9 +299,11 @@ VVH_API int vvh_linear_q8_dev_in(void* out, const void* inp, const int8_t* dev_w
  * decomposition, device-resident descriptor table) and launched with
  * vvh_plan_run as a single kernel when every problem takes the decode path
  * (M <= 16), or when its problems read the same activations and take the
- * GEMM (not from fp16 to fp32), or are fp32 of few rows (a GEMM of fp32 activations or of split k adds
- * its split and reduction launches, and without their workspace, as in a
- * capture that cannot allocate, the problems run one by one); else as one
+ * GEMM (not from fp16 to fp32), or are fp32 of few rows (a GEMM of fp32
+ * activations or of split k adds its split and reduction launches; fp16 plans
+ * without a workspace, or captured where no problem alone would use it, do not
+ * split k, fp32 ones on the GEMM have to have run on the stream before they
+ * are captured there, like single fp32 calls of 16 rows or more); else as one
  * launch per problem.  It is the counterpart of the
  * reference IR's pre-resolved op list (src/ir/executable.cc:192-354) for the
  * int8 linears that share an input (q/k/v, transformer.h:139-144) or are

@@ -2,7 +2,7 @@
 otherwise: captured on a stream that never ran them (the capture may not
 allocate), replayed between eager work, against the eager result on a stream
 that has a workspace.  Attention and dense calls whose splits need it, fp32
-linears of a few rows, and a grouped plan whose k is split.
+linears of a few rows, and grouped plans whose k is split.
 """
 import ctypes
 
@@ -75,6 +75,7 @@ CASES = {
     "dense_f32": lambda r: dense(r, F32, 128, 896, 4864),
     "linear_f32_few": lambda r: linear(r, 5, 1536, 1536, False),
     "plan_f16": lambda r: linear(r, 40, 256, 896, True, F16),
+    "plan_f16_split": lambda r: linear(r, 128, 2048, 1536, True, F16),  # one by one its problems would split k too
     "plan_f32_decode": lambda r: linear(r, 3, 256, 4864, True),
 }
 
@@ -154,3 +155,39 @@ def test_graph_holds_no_workspace(gpu, name):
         assert np.array_equal(want.to_array(dt, shape).astype(np.float64), ref)
     assert lib.hipGraphExecDestroy(ex) == 0 and lib.hipGraphDestroy(graph) == 0
     assert lib.hipStreamDestroy(first) == 0 and lib.hipStreamDestroy(other) == 0
+
+
+@pytest.mark.parametrize("M,N,K,nodes", [(40, 256, 896, 1), (128, 2048, 1536, 2)])
+def test_split_plan_in_a_graph(gpu, M, N, K, nodes):
+    """A grouped fp16 plan whose k is split, captured on a stream that has the
+    workspace: without it where its problems alone run on k_skinny, with it
+    (GEMM and reduction, the eager bits) where they would split k as well."""
+    print(f"[case] split plan in a graph M={M} N={N} K={K}", flush=True)
+    lib = hip()
+    keep, shape, dt, run = linear(np.random.default_rng(M), M, N, K, True, F16)
+    size = int(np.prod(shape)) * 2
+    want, got = capi.DevBuf(size), capi.DevBuf(size)
+    stream, graph, ex = V(), V(), V()
+    assert lib.hipStreamCreate(ctypes.byref(stream)) == 0
+    run(want, stream)
+    run(got, stream)
+    capi.sync()
+    ref = want.to_array(dt, shape)
+    assert lib.hipStreamBeginCapture(stream, 1) == 0
+    run(got, stream)
+    assert lib.hipStreamEndCapture(stream, ctypes.byref(graph)) == 0
+    n = ctypes.c_size_t()
+    assert lib.hipGraphGetNodes(graph, None, ctypes.byref(n)) == 0
+    assert n.value == nodes
+    assert lib.hipGraphInstantiate(ctypes.byref(ex), graph, None, None, 0) == 0
+    for _ in range(3):
+        capi.call("vvh_memcpy_h2d", got.ptr, np.zeros(shape, dt).ctypes.data, size)
+        run(want, stream)
+        assert lib.hipGraphLaunch(ex, stream) == 0
+        capi.sync()
+        y = got.to_array(dt, shape)
+        if nodes == 2:
+            assert np.array_equal(y, ref)
+        assert np.linalg.norm(y.astype(np.float64) - ref) <= 2.0 ** -10 * np.linalg.norm(ref.astype(np.float64))
+    assert lib.hipGraphExecDestroy(ex) == 0 and lib.hipGraphDestroy(graph) == 0
+    assert lib.hipStreamDestroy(stream) == 0

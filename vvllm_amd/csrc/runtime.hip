@@ -121,9 +121,9 @@ vvh_plan g_next_plan = 1;
 
 // ---- split-K workspace ------------------------------------------------------
 // fp32 partial sums of split GEMMs and dense linears, split fp32 activations
-// and the partials of attention and sampling over many blocks, one buffer per stream (calls on one stream run in
-// order, so they can share it; calls on different streams never do).  Grown
-// on demand to at least twice its size; a buffer it outgrows is retired, not
+// and the partials of attention and sampling over many blocks, one buffer per
+// stream (calls on one stream run in order, so they can share it; calls on
+// different streams never do).  Grown on demand to at least twice its size; a buffer it outgrows is retired, not
 // freed, because a HIP graph captured earlier on the stream still holds its
 // address in its kernel nodes (a replay must not touch freed memory).
 // Retired buffers are freed by vvh_workspace_release or at process end.
@@ -781,7 +781,10 @@ void group_blocks(LinGroup& l, std::size_t count, int64_t blocks)
 }
 
 // Runs a kGroupGemm or kGroupGemv plan; *done = false, and nothing launched,
-// where it needs a workspace it cannot have now or is too large for one grid.
+// where fp32 activations lack the workspace for their split form or the plan is
+// too large for one grid.  fp16 activations without a workspace, or in a
+// capture that would hold none with a launch per problem (k_skinny, or GEMMs
+// of unsplit k), run unsplit.
 int run_group(const std::vector<LinArgs>& args, int group, int act, int outd, void* stream, bool* done)
 {
     *done = false;
@@ -815,10 +818,8 @@ int run_group(const std::vector<LinArgs>& args, int group, int act, int outd, vo
     };
     int split_layout = 4;
     int sp = gemm_splits(M, n, tiles_of, stages, &split_layout);
-    const int64_t kst = (stages + sp - 1) / sp;
+    int64_t kst = (stages + sp - 1) / sp;
     sp = (int)((stages + kst - 1) / kst);  // no empty split
-    const int layout = gemm3_layout(tiles_of, sp, split_layout, f32);
-    if (tiles_of(gemm3_tile_m(layout), gemm3_tile_n(layout)) * sp > INT32_MAX) return VVH_OK;
     uint64_t xs = 0, rs = 0, plane = 0;
     if (f32) {
         if (!mul_ok((uint64_t)M * (uint64_t)K, 4, &xs)) return VVH_OK;
@@ -827,7 +828,21 @@ int run_group(const std::vector<LinArgs>& args, int group, int act, int outd, vo
     }
     if (sp > 1 && !mul_ok((uint64_t)M * (uint64_t)n, (uint64_t)sp * 4, &plane)) return VVH_OK;
     float* ws = nullptr;
-    if (xs + rs + plane > 0 && !workspace_try(stream, xs + rs + plane, &ws, true)) return VVH_OK;
+    const uint64_t bytes = xs + rs + plane;
+    if (bytes > 0 && !workspace_try(stream, bytes, &ws)) {
+        auto alone = [&](const LinArgs& a) {
+            int l = 4;
+            return choose_kernel((std::size_t)a.M, (std::size_t)a.N, (std::size_t)a.K, act, true) == K_GEMM &&
+                   gemm_splits(a.M, a.N, stages, &l) > 1;
+        };
+        if (!((f32 || std::any_of(args.begin(), args.end(), alone)) && workspace_try(stream, bytes, &ws, true))) {
+            if (f32) return VVH_OK;
+            sp = 1;
+            kst = stages;
+        }
+    }
+    const int layout = gemm3_layout(tiles_of, sp, split_layout, f32);
+    if (tiles_of(gemm3_tile_m(layout), gemm3_tile_n(layout)) * sp > INT32_MAX) return VVH_OK;
     char* wb = reinterpret_cast<char*>(ws);
     float* wp = reinterpret_cast<float*>(wb + xs + rs);
     for (std::size_t i = 0; i < count; i++) {
