@@ -191,3 +191,28 @@ def test_split_plan_in_a_graph(gpu, M, N, K, nodes):
         assert np.linalg.norm(y.astype(np.float64) - ref) <= 2.0 ** -10 * np.linalg.norm(ref.astype(np.float64))
     assert lib.hipGraphExecDestroy(ex) == 0 and lib.hipGraphDestroy(graph) == 0
     assert lib.hipStreamDestroy(stream) == 0
+
+
+@pytest.mark.parametrize("name", ["dense_f16", "attention_f16", "plan_f16"])
+def test_eager_call_next_to_a_global_capture(gpu, name):
+    """A call whose first workspace is allocated while another stream is being
+    captured in the global mode leaves that capture whole."""
+    print(f"[case] eager next to a capture: {name}", flush=True)
+    lib = hip()
+    keep, shape, dt, run = CASES[name](np.random.default_rng(len(name)))
+    size = int(np.prod(shape)) * np.dtype(dt).itemsize
+    want, got, small = capi.DevBuf(size), capi.DevBuf(size), capi.DevBuf(4096)
+    captured, eager, graph = V(), V(), V()
+    assert lib.hipStreamCreate(ctypes.byref(captured)) == 0 and lib.hipStreamCreate(ctypes.byref(eager)) == 0
+    run(want, eager)
+    run(got, eager)  # a plan of `got` exists before the capture
+    capi.sync()
+    capi.call("vvh_workspace_release", eager)
+    assert lib.hipStreamBeginCapture(captured, 0) == 0
+    capi.call("vvh_eltwise", capi.OP_ADD, small.ptr, small.ptr, small.ptr, 1024, F32, captured)
+    run(got, eager)
+    assert lib.hipStreamEndCapture(captured, ctypes.byref(graph)) == 0
+    capi.sync()
+    assert np.array_equal(got.to_array(dt, shape), want.to_array(dt, shape))
+    assert lib.hipGraphDestroy(graph) == 0
+    assert lib.hipStreamDestroy(captured) == 0 and lib.hipStreamDestroy(eager) == 0

@@ -123,10 +123,11 @@ vvh_plan g_next_plan = 1;
 // fp32 partial sums of split GEMMs and dense linears, split fp32 activations
 // and the partials of attention and sampling over many blocks, one buffer per
 // stream (calls on one stream run in order, so they can share it; calls on
-// different streams never do).  Grown on demand to at least twice its size; a buffer it outgrows is retired, not
-// freed, because a HIP graph captured earlier on the stream still holds its
-// address in its kernel nodes (a replay must not touch freed memory).
-// Retired buffers are freed by vvh_workspace_release or at process end.
+// different streams never do).  Grown on demand to at least twice its size; a
+// buffer it outgrows is retired, not freed, because a HIP graph captured earlier
+// on the stream still holds its address in its kernel nodes (a replay must not
+// touch freed memory).  Retired buffers are freed by vvh_workspace_release or at
+// process end.
 struct Workspace {
     void* p = nullptr;
     std::size_t bytes = 0;
@@ -135,14 +136,20 @@ struct Workspace {
 std::mutex g_wsmu;
 std::unordered_map<void*, Workspace> g_ws;
 
-int workspace_for(void* stream, std::size_t bytes, float** out)
+// relaxed: allocate also while another stream is being captured in the global
+// mode, which forbids hipMalloc to every thread but those in the relaxed mode and
+// fails the capture where one is made (calls that needed no workspace once).
+int workspace_for(void* stream, std::size_t bytes, float** out, bool relaxed = false)
 {
     std::lock_guard<std::mutex> lock(g_wsmu);
     Workspace& w = g_ws[stream];
     if (w.bytes < bytes) {
         const std::size_t nb = std::max({bytes, 2 * w.bytes, std::size_t(1) << 20});
         void* p = nullptr;
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        relaxed = relaxed && hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
         hipError_t e = hipMalloc(&p, nb);
+        if (relaxed) (void)hipThreadExchangeStreamCaptureMode(&mode);
         if (e != hipSuccess) {
             (void)hipGetLastError();
             return fail_hip(e, "workspace hipMalloc");
@@ -176,7 +183,7 @@ bool workspace_try(void* stream, std::size_t bytes, float** ws, bool captured = 
         *ws = static_cast<float*>(it->second.p);
         return true;
     }
-    return workspace_for(stream, bytes, ws) == VVH_OK;
+    return workspace_for(stream, bytes, ws, true) == VVH_OK;
 }
 
 // ---- fixed scratch of vvh_linear_q8_dev_noalloc ------------------------------
