@@ -8,6 +8,8 @@ value), plus the scores' fp32 sums (|score| up to about 8, so 2e-6 of each
 weight) and the weights' 22 bits or more, together below 1e-5 of the largest
 |v|.
 """
+import time
+
 import numpy as np
 import pytest
 
@@ -127,3 +129,62 @@ def test_prefill_small_weights(gpu, n_q, len0, H, KVH, D, d, gap):
     got, ref = run(q, k, v, len0, scale, d), reference(q, k, v, len0, scale)
     tol = (ULP[d] + 2e-5) * np.abs(ref) + (2.0 ** -25 + T * 2.0 ** -35 * 1500.0 if d == F16 else 0.0)
     assert (np.abs(got - ref) <= tol).all()
+
+
+NONFINITE = [(40, 3, 6, 2, 64), (90, 30, 12, 2, 128), (7, 700, 12, 2, 128), (500, 1, 14, 2, 64)]
+
+
+@pytest.mark.parametrize("n_q,len0,H,KVH,D", NONFINITE)
+@pytest.mark.parametrize("d", [F32, F16])
+@pytest.mark.parametrize("where", ["v inf", "v nan", "k inf", "k nan", "v -inf and inf"])
+@pytest.mark.parametrize("in_place", [False, True])
+def test_prefill_nonfinite_rows(gpu, n_q, len0, H, KVH, D, d, where, in_place):
+    """Queries that see a key or value that is not finite get what the sums
+    give, infinities, NaN and the finite rest alike, also where out is q."""
+    print(f"[case] nonfinite n_q={n_q} len0={len0} D={D} dtype={d} {where} in_place={in_place}", flush=True)
+    q, k, v, scale = draw(n_q, len0, H, KVH, D, d)
+    t = len0 // 2 + n_q // 3  # the queries from here on see it
+    if where.startswith("v"):
+        v[t, KVH - 1, 5] = {"inf": np.inf, "nan": np.nan, "-inf": -np.inf}[where.split()[1]]
+        if "and" in where:
+            v[t + 1, KVH - 1, 5], v[t, 0, 1] = np.inf, -np.inf
+    else:
+        k[t, KVH - 1] = np.inf if where == "k inf" else np.nan
+        k[t, KVH - 1, 1:] = 0 if where == "k inf" else 1
+    with np.errstate(invalid="ignore", over="ignore"):
+        ref = reference(q, k, np.where(np.isfinite(v), v, 0), len0, scale)
+        for s in range(n_q):  # dim 5 of kv head KVH - 1 (and dim 1 of kv head 0): sums of its values
+            for kvh, dim in ((KVH - 1, 5), (0, 1)):
+                seen = v[:len0 + s, kvh, dim].astype(np.float64)
+                if not np.isfinite(seen).all():
+                    ref[s, kvh * (H // KVH):(kvh + 1) * (H // KVH), dim] = seen[~np.isfinite(seen)].sum()
+    if in_place:
+        b = [capi.DevBuf.from_array(a) for a in (q, k, v)]
+        capi.call("vvh_attention", b[0].ptr, b[0].ptr, b[1].ptr, b[2].ptr, n_q, len0, H, KVH, D, scale, d, None)
+        capi.sync()
+        got = b[0].to_array(npd(d), (n_q, H, D)).astype(np.float64)
+    else:
+        got = run(q, k, v, len0, scale, d)
+    fin = np.isfinite(ref)
+    assert fin.any() and not fin.all()
+    assert np.array_equal(got[~fin], ref[~fin], equal_nan=True)
+    vmax = np.abs(v[np.isfinite(v)]).max()
+    assert (np.abs(got[fin] - ref[fin]) <= ULP[d] * np.abs(ref[fin]) + 1e-5 * vmax).all()
+
+
+@pytest.mark.parametrize("d", [F32, F16])
+@pytest.mark.parametrize("n_q,len0,H,KVH,D,ms", [(512, 1, 14, 2, 64, 0.6), (7, 4000, 12, 2, 128, 1.2)])
+def test_prefill_nonfinite_time(gpu, n_q, len0, H, KVH, D, d, ms):
+    """An infinity that every query sees does not leave the rows to one wave
+    each (2.4 ms and more at these sizes; 0.07 to 0.5 with a block per row)."""
+    q, k, v, scale = draw(n_q, len0, H, KVH, D, d)
+    v[0] = np.inf
+    b = [capi.DevBuf.from_array(a) for a in (q, k, v)] + [capi.DevBuf(q.nbytes)]
+    best = np.inf
+    for _ in range(5):
+        t0 = time.perf_counter()
+        capi.call("vvh_attention", b[3].ptr, b[0].ptr, b[1].ptr, b[2].ptr, n_q, len0, H, KVH, D, scale, d, None)
+        capi.sync()
+        best = min(best, time.perf_counter() - t0)
+    print(f"error {best * 1e3:.3f} ms")
+    assert best * 1e3 < ms

@@ -33,38 +33,116 @@ __device__ __forceinline__ int attn_swz(int r)
     return D == 128 ? ((r & 3) << 2) | ((r >> 2) & 3) : (((r >> 1) & 1) << 2) | ((r >> 2) & 3);
 }
 
-// One row of the general kernel's arithmetic in one wave: scores, maximum,
-// exponentials and sum over the `len` visible keys only.  For rows whose
-// result from the tiles is not finite: a key past a row's last visible one
-// has weight 0 in the tiles, and 0 times an infinity or NaN of its V row
-// would reach the sums.
+// One row of the general kernel's arithmetic by a wave, over the `len` visible
+// keys only: scores, their maximum and the sum of the exponentials, then the
+// scores again and the weighted values.  For rows whose result from the tiles is
+// not finite: a key past a row's last visible one has weight 0 in the tiles, and
+// 0 times an infinity or NaN of its V row would reach the sums, as would an
+// infinity times the 0 of a weight's low part.  A key row is shared by L lanes of
+// 16 bytes, U keys of each group of lanes in flight.  M and den: the maximum (in
+// log2 units, or a little less) and the sum of the weights under it that the tiles
+// found, which no V row reaches; where they are not finite, or no weight is left,
+// they are worked out as the general kernel does.  With an infinity in a V row
+// that every query sees, us, one block per head and query (k_attention) / a wave
+// per row and one key at a time / here: 512 queries, 14 heads of 64, 72 / 2390 /
+// 93, fp32 92 / 2390 / 159; 2048, 12 of 128, 1820 / 9960 / 895, fp32 2030 / 20200 / 2390; 7
+// after 4000 242 / 2540 / 206; a NaN or infinite key 73 / 2390 / 13 at 512 (attn_redo).
 template <typename T, int D>
 __device__ void attn_row_general(const T* __restrict__ qr, const T* __restrict__ kh, const T* __restrict__ vh,
-                                 int64_t kvs, int len, float scale, T* __restrict__ orow, int lane)
+                                 int64_t kvs, int len, float scale, float M, float den, T* __restrict__ orow, int lane)
 {
-    constexpr int E = D / 64;
-    float qv[E], o[E];
+    constexpr int E = 16 / (int)sizeof(T), L = D / E, G = 64 / L, U = (int)sizeof(T) * 2;
+    typedef T te __attribute__((ext_vector_type(E)));
+    const int c = lane % L, g = lane / L;
+    const te qv = *reinterpret_cast<const te*>(qr + c * E);
+    auto load = [&](const T* base, int t0, te (&r)[U]) {
 #pragma unroll
-    for (int e = 0; e < E; e++) {
-        qv[e] = (float)qr[lane * E + e];
-        o[e] = 0.0f;
-    }
-    auto score = [&](int t) {
+        for (int u = 0; u < U; u++) {
+            const int t = t0 + u * G < len ? t0 + u * G : len - 1;
+            r[u] = *reinterpret_cast<const te*>(base + t * kvs + c * E);
+        }
+    };
+    auto score = [&](const te k) {
         float d = 0.0f;
 #pragma unroll
-        for (int e = 0; e < E; e++) d += qv[e] * (float)kh[t * kvs + lane * E + e];
-        return wave_sum_xor(d) * scale;
+        for (int e = 0; e < E; e++) d = __builtin_fmaf((float)qv[e], (float)k[e], d);
+        return group_sum(d, L);
     };
-    float mx = -INFINITY, sum = 0.0f;
-    for (int t = 0; t < len; t++) mx = fmaxf(mx, score(t));
-    for (int t = 0; t < len; t++) sum += expf(score(t) - mx);
-    for (int t = 0; t < len; t++) {
-        const float p = expf(score(t) - mx) / sum;
+    const bool known = __builtin_fabsf(M) < 1.0e30f && den > 0.0f && den < INFINITY;
+    float m = -INFINITY, l = 0.0f;  // a key at -inf adds nothing, unless all are
+    for (int t0 = g; !known && t0 < len; t0 += U * G) {
+        te k[U];
+        load(kh, t0, k);
 #pragma unroll
-        for (int e = 0; e < E; e++) o[e] += p * (float)vh[t * kvs + lane * E + e];
+        for (int u = 0; u < U; u++) {
+            const float s = score(k[u]) * scale;
+            if (t0 + u * G >= len || s == -INFINITY) continue;
+            if (s > m) {
+                l = l * expf(m - s) + 1.0f;
+                m = s;
+            } else {
+                l += expf(s - m);
+            }
+        }
     }
+    for (int off = L; off < 64; off <<= 1) {
+        const float m2 = __shfl_xor(m, off), l2 = __shfl_xor(l, off), mx = fmaxf(m, m2);
+        l = mx == -INFINITY ? l + l2 : l * expf(m - mx) + l2 * expf(m2 - mx);
+        m = mx;
+    }
+    if (known) {
+        m = M;
+        l = den;
+    } else if (!(__builtin_fabsf(m) < INFINITY)) {
+        l = __builtin_nanf("");  // exp(inf - inf)
+    }
+    // exp2(score sl + score slo - m) / l, or exp(score scale - m) / l
+    const double sd = known ? (double)scale * 1.4426950408889634 : 0.0;
+    const float sl = (float)sd, slo = (float)(sd - (double)sl), rl = 1.0f / l;
+    float o[E];
 #pragma unroll
-    for (int e = 0; e < E; e++) orow[lane * E + e] = (T)o[e];
+    for (int e = 0; e < E; e++) o[e] = l == l ? 0.0f : l;
+    if (l == l) {
+        for (int t0 = g; t0 < len; t0 += U * G) {
+            te k[U], v[U];
+            load(kh, t0, k);
+            load(vh, t0, v);
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const float s = score(k[u]);
+                if (t0 + u * G >= len) continue;
+                float p;
+                if (known) {
+                    const float x = __builtin_fmaf(s, sl, -m);
+                    p = __builtin_amdgcn_exp2f(s > -INFINITY ? __builtin_fmaf(s, slo, x) : x) * rl;
+                } else {
+                    p = expf(s * scale - m) / l;
+                }
+#pragma unroll
+                for (int e = 0; e < E; e++) o[e] = __builtin_fmaf(p, (float)v[u][e], o[e]);
+            }
+        }
+    }
+    T y[E];
+#pragma unroll
+    for (int e = 0; e < E; e++) {
+        for (int off = L; off < 64; off <<= 1) o[e] += __shfl_xor(o[e], off);
+        y[e] = (T)o[e];
+    }
+    if (g == 0)
+#pragma unroll
+        for (int e = 0; e < E; e++) orow[c * E + e] = y[e];
+}
+
+// Whether a row of numerators and denominator den under the maximum M is to be
+// done again by attn_row_general: some quotient is not finite, but not because a
+// visible score is NaN, which makes the whole row NaN there too.
+__device__ __forceinline__ bool attn_redo(const f4 y, float den, float M)
+{
+    bool nf = false;
+#pragma unroll
+    for (int j = 0; j < 4; j++) nf = nf || !(__builtin_fabsf(y[j]) <= 3.0e38f);
+    return nf && !(den != den && __builtin_fabsf(M) < INFINITY);
 }
 
 }  // namespace
@@ -289,17 +367,15 @@ __global__ __launch_bounds__(256 * RG) void k_attention_prefill(
         const int s_ = r / G;
         return ((int64_t)s_ * H + (int64_t)kvh * G + (r - s_ * G)) * D;
     };
-    auto finish = [&](int rr, int d, f4 num, float den) {
-        h4v w;
-        bool nf = false;
+    // the maximum and the sum of the weights of row rr, over its key groups
+    auto row_sums = [&](int rr, float& M, float& den) {
+        const int w0 = rr / 32, ri = rr & 31;  // wave of key group g: w0 + g RG
+        M = wm[w0][ri];
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const float y = num[j] / den;
-            nf = nf || !(__builtin_fabsf(y) <= 3.0e38f);
-            w[j] = (f16)y;
-        }
-        if (nf) bad[rr] = 1;
-        *reinterpret_cast<h4v*>(out + row_off(r0 + rr) + d) = w;
+        for (int g = 1; g < KG; g++) M = fmaxf(M, wm[w0 + g * RG][ri]);
+        den = 0.0f;
+#pragma unroll
+        for (int g = 0; g < KG; g++) den += __builtin_amdgcn_exp2f(wm[w0 + g * RG][ri] - M) * wl[w0 + g * RG][ri];
     };
     // partials of split z of row r: D floats at row z KVH R + kvh R + r, and (m, l) after all rows
     const int64_t pr0 = ((int64_t)blockIdx.y * KVH + kvh) * R + r0;
@@ -321,7 +397,11 @@ __global__ __launch_bounds__(256 * RG) void k_attention_prefill(
             den += f * wl[w0 + g * RG][ri];
         }
         if (ns == 1) {
-            finish(rr, 4 * c, num, den);
+            const f4 y = num / den;
+            // the row's D / 4 lanes agree before any stores (out may be q, which a redone row reads)
+            const uint64_t redo = __ballot(attn_redo(y, den, M)) >> (lane & (64 - D / 4)) & (((uint64_t)1 << (D / 4)) - 1);
+            if (redo) bad[rr] = 1;
+            else *reinterpret_cast<h4v*>(out + row_off(r0 + rr) + 4 * c) = __builtin_convertvector(y, h4v);
         } else {
             wo[(pr0 + rr) * (D / 4) + c] = num;
             if (c == 0) wml[pr0 + rr] = make_float2(M, den);
@@ -329,11 +409,15 @@ __global__ __launch_bounds__(256 * RG) void k_attention_prefill(
     }
     if (ns > 1) return;  // k_attention_prefill_merge finishes the rows
     __syncthreads();
-    for (int rr = wave; rr < ROWS; rr += NW) {
-        if (r0 + rr >= R) break;
-        if (!__builtin_amdgcn_readfirstlane(bad[rr])) continue;  // always, with finite inputs
+    // rows to be done again, a wave each: none, with finite inputs
+    int turn = 0;
+    for (uint64_t rows = __ballot(lane < ROWS && bad[lane % ROWS]); rows; rows &= rows - 1) {
+        if (turn++ % NW != wave) continue;
+        const int rr = __builtin_ctzll(rows);
         const int64_t off = row_off(r0 + rr);
-        attn_row_general<f16, D>(q + off, kh, vh, kvs, len0 + (r0 + rr) / G, scale, out + off, lane);
+        float M, den;
+        row_sums(rr, M, den);
+        attn_row_general<f16, D>(q + off, kh, vh, kvs, len0 + (r0 + rr) / G, scale, M, den, out + off, lane);
     }
 }
 
@@ -516,6 +600,16 @@ __global__ __launch_bounds__(256) void k_attention_prefill_f32(
         const int s_ = r / G;
         return ((int64_t)s_ * H + (int64_t)kvh * G + (r - s_ * G)) * D;
     };
+    // the maximum and the sum of the weights of row rr, over its key groups
+    auto row_sums = [&](int rr, float& M, float& den) {
+        const int w0 = rr / 32, ri = rr & 31;  // wave of key group g: w0 + g RG
+        M = wm[w0][ri];
+#pragma unroll
+        for (int g = 1; g < KG; g++) M = fmaxf(M, wm[w0 + g * RG][ri]);
+        den = 0.0f;
+#pragma unroll
+        for (int g = 0; g < KG; g++) den += __builtin_amdgcn_exp2f(wm[w0 + g * RG][ri] - M) * wl[w0 + g * RG][ri];
+    };
     const int64_t pr0 = ((int64_t)blockIdx.y * KVH + kvh) * R + r0;
     f4* wo = reinterpret_cast<f4*>(ws);
     float2* wml = reinterpret_cast<float2*>(ws + (int64_t)ns * KVH * R * D);
@@ -535,15 +629,11 @@ __global__ __launch_bounds__(256) void k_attention_prefill_f32(
             den += f * wl[w0 + g * RG][ri];
         }
         if (ns == 1) {
-            f4 y;
-            bool nf = false;
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                y[j] = num[j] / den;
-                nf = nf || !(__builtin_fabsf(y[j]) <= 3.4e38f);
-            }
-            if (nf) bad[rr] = 1;
-            *reinterpret_cast<f4*>(out + row_off(r0 + rr) + 4 * c) = y;
+            const f4 y = num / den;
+            // the row's D / 4 lanes agree before any stores (out may be q, which a redone row reads)
+            const uint64_t redo = __ballot(attn_redo(y, den, M)) >> (lane & (64 - D / 4)) & (((uint64_t)1 << (D / 4)) - 1);
+            if (redo) bad[rr] = 1;
+            else *reinterpret_cast<f4*>(out + row_off(r0 + rr) + 4 * c) = y;
         } else {
             wo[(pr0 + rr) * (D / 4) + c] = num;
             if (c == 0) wml[pr0 + rr] = make_float2(M, den);
@@ -551,11 +641,15 @@ __global__ __launch_bounds__(256) void k_attention_prefill_f32(
     }
     if (ns > 1) return;  // k_attention_prefill_merge finishes the rows
     __syncthreads();
-    for (int rr = wave; rr < ROWS; rr += 4) {
-        if (r0 + rr >= R) break;
-        if (!__builtin_amdgcn_readfirstlane(bad[rr])) continue;  // always, with finite inputs
+    // rows to be done again, a wave each: none, with finite inputs
+    int turn = 0;
+    for (uint64_t rows = __ballot(lane < ROWS && bad[lane % ROWS]); rows; rows &= rows - 1) {
+        if (turn++ % 4 != wave) continue;
+        const int rr = __builtin_ctzll(rows);
         const int64_t off = row_off(r0 + rr);
-        attn_row_general<float, D>(q + off, kh, vh, kvs, len0 + (r0 + rr) / G, scale, out + off, lane);
+        float M, den;
+        row_sums(rr, M, den);
+        attn_row_general<float, D>(q + off, kh, vh, kvs, len0 + (r0 + rr) / G, scale, M, den, out + off, lane);
     }
 }
 
@@ -587,16 +681,16 @@ __global__ __launch_bounds__(256) void k_attention_prefill_merge(const T* __rest
         den += f * ml.y;
     }
     const int64_t off = ((int64_t)s * G * KVH + (int64_t)kvh * G + (r - s * G)) * D;
-    bool nf = false;
+    f4 y = f4{};
 #pragma unroll
-    for (int e = 0; e < E; e++) {
-        const float y = num[e] / den;
-        nf = nf || !(__builtin_fabsf(y) <= 3.0e38f);
-        out[off + lane * E + e] = (T)y;
-    }
-    if (__any(nf))  // not with finite inputs
+    for (int e = 0; e < E; e++) y[e] = num[e] / den;
+    if (__any(attn_redo(y, den, M))) {  // not with finite inputs
         attn_row_general<T, D>(q + off, k + (int64_t)kvh * D, v + (int64_t)kvh * D, (int64_t)KVH * D, len0 + s, scale,
-                            out + off, lane);
+                               M, den, out + off, lane);
+        return;
+    }
+#pragma unroll
+    for (int e = 0; e < E; e++) out[off + lane * E + e] = (T)y[e];
 }
 
 // The tile kernels' calls: head_dim 64 or 128, 16-byte aligned q, K and V and
