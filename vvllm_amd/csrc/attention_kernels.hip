@@ -700,12 +700,23 @@ __global__ __launch_bounds__(256) void k_attention_prefill_merge(const T* __rest
 // fp32 calls over fewer than 128 positions keep k_attention while its blocks,
 // one per head and query, fit the chip at once: a single stage here costs more
 // (graph replay: 38 queries, 12 heads of 128, 7.2 us against 13.6; 15, 24 of 64, 4.9
-// against 8.2; 7 queries after 360 positions, 14 of 64, 15.3 against 13.3).
+// against 8.2; 7 queries after 360 positions, 14 of 64, 15.3 against 13.3).  So do
+// those a little past the first stage with fewer blocks (32 queries after 100, 14 of
+// 64, 8.8 against 10.6, 12 of 128, 13.7 against 14.7; 8 after 150 / 250, 14 of 64, 8.7 / 12.4
+// against 10.7 / 13.4; 24 after 150 / 250, 32 heads, 11.6 / 17.1 against 10.8 / 13.7; 64 after
+// 150 / 200, 12 of 128, 22.6 / 28.9 against 26.8 / 31.7, 48 after 300 34.7 against 36.5), and
+// fp16 calls of a few queries over up to 40 positions at head_dim 128 (8 after 20, 12
+// heads, 6.3 against 7.4; 24 after 20 7.2 against 7.2).
 bool attention_prefill_ok(const void* out, const void* q, const void* k, const void* v, int64_t n_q, int64_t len0,
                           int64_t H, int64_t KVH, int64_t D, float scale, int dtype)
 {
     const int64_t es = dtype == VVH_F16 ? 2 : 4;
-    if (dtype == VVH_F32 && len0 + n_q - 1 < 128 && n_q * H <= 2048) return false;
+    const int64_t span = len0 + n_q - 1, rows = n_q * H;
+    if (dtype == VVH_F32 && ((span < 128 && rows <= 2048) || (span <= 152 && rows <= 512) ||
+                             (D == 64 && span <= 270 && rows <= 256) ||
+                             (D == 128 && span <= 270 && rows > 512 && rows <= 800)))
+        return false;
+    if (dtype == VVH_F16 && D == 128 && span <= 40 && rows <= 256) return false;
     return (D == 64 || D == 128) && scale > 0.0f && scale < INFINITY &&
            ((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k) | reinterpret_cast<uintptr_t>(v)) & 15) == 0 &&
            (reinterpret_cast<uintptr_t>(out) & (uintptr_t)(4 * es - 1)) == 0 && n_q * (H / KVH) <= (1 << 30) &&
