@@ -1,6 +1,6 @@
 """vvh_convert in 8-element chunks (remainders, aligned and not) and sampling at
-the edges of its blocks: one block up to 2048 logits, then blocks of 512, at most
-1024 of them.  Conversions are exact or one rounding; the first index of the
+the edges of its blocks: one block up to 2048 logits, then blocks of 512, from
+2^18 logits on of 2048 and more, at most 1024 of them.  Conversions are exact or one rounding; the first index of the
 maximum is exact.
 """
 import numpy as np
@@ -29,7 +29,7 @@ def test_convert(gpu, n, off, src, dst):
 
 
 @pytest.mark.parametrize("d", [F16, F32])
-@pytest.mark.parametrize("n", [1, 2048, 2049, 2560, 2561, 151936, 512 * 1024, 512 * 1024 + 1])
+@pytest.mark.parametrize("n", [1, 2048, 2049, 2560, 2561, 151936, 1 << 18, (1 << 18) + 1, 512 * 1024 + 1, (1 << 21) + 1])
 def test_argmax_first_index(gpu, n, d):
     x = np.random.default_rng(n).integers(-100, 50, n).astype(DT[d])
     for at in ([0], [n - 1], [n // 3, n - 1], [min(n - 1, 511), min(n - 1, 512)]):

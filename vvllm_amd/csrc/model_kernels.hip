@@ -272,14 +272,19 @@ __global__ __launch_bounds__(256) void k_rms_norm_rows(T* __restrict__ out, cons
 }
 
 // Rows from which a wave per row pays (graph replay, fp16: 512 rows of 896 3.2 ->
-// 3.0 us, 2048 of 1536 7.5 -> 4.6; 256 of 896 2.7 -> 2.9).
-constexpr int64_t kRmsRowsMin = 512;
+// 3.0 us, 2048 of 1536 7.5 -> 4.6; 256 of 896 2.7 -> 2.9; fp32: 512 rows of 896 3.4 ->
+// 3.4, of 1536 3.6 -> 3.9, 600 of 2048 4.1 -> 4.4, 1024 of 1536 4.6 -> 4.5, 2048 6.7 ->
+// 6.2).
+static bool rms_rows_pay(int64_t rows, int64_t n, int dtype)
+{
+    return rows >= (dtype == VVH_F32 && n > 1024 ? 1024 : 512);
+}
 
 int launch_rms_norm(void* out, const void* x, const float* w, int64_t rows, int64_t n, float eps, int dtype,
                     void* stream)
 {
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if (rows >= kRmsRowsMin && n % 8 == 0 && n <= 2048 &&
+    if (rms_rows_pay(rows, n, dtype) && n % 8 == 0 && n <= 2048 &&
         ((reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w)) & 15) == 0) {
         const dim3 grid((unsigned)((rows + 3) / 4));
         if (dtype == VVH_F16)
@@ -432,13 +437,15 @@ __global__ __launch_bounds__(256) void k_rope_rows(T* __restrict__ q, T* __restr
 // Whether the form above serves a call: its shapes, and enough pairs that
 // sharing a position's angles over the heads pays for the blocks it leaves
 // unused (graph replay, 0.5B heads, 256 / 512 positions: 4.0 / 5.4 us with a
-// thread per pair, 4.1 / 4.2 here; 2048 positions of the 1.5B heads 24.1 -> 6.4).
-constexpr int64_t kRopeRowsMin = 200000;
+// thread per pair, 4.1 / 4.2 here; 2048 positions of the 1.5B heads 24.1 -> 6.4), and
+// positions enough for some blocks (100 positions of 40 heads of 128 in fp32 5.75 us
+// against 6.1, 200 8.8 against 6.6).
+constexpr int64_t kRopeRowsMin = 200000, kRopeRowsMinS = 128;
 static bool rope_rows_ok(const void* q, const void* k, const void* v, const void* kc, const void* vc, int64_t S,
                          int64_t H, int64_t KVH, int64_t D)
 {
-    return S * (H + KVH) * (D / 2) >= kRopeRowsMin && D >= 16 && D <= 512 && (D & (D - 1)) == 0 && H + KVH <= 65535 &&
-           S <= (int64_t)INT32_MAX && ((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k) |
+    return S >= kRopeRowsMinS && S * (H + KVH) * (D / 2) >= kRopeRowsMin && D >= 16 && D <= 512 && (D & (D - 1)) == 0 &&
+           H + KVH <= 65535 && S <= (int64_t)INT32_MAX && ((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k) |
              reinterpret_cast<uintptr_t>(v) | reinterpret_cast<uintptr_t>(kc) | reinterpret_cast<uintptr_t>(vc)) & 15) == 0;
 }
 
@@ -1695,11 +1702,15 @@ constexpr int64_t kArgmaxOne = 2048;  // up to this many elements one block, wit
 // else elements per block: two serial logarithm chains a thread instead of the eight of 2048 (with
 // k_convert_vec before it: a token's fp16 LM head over 151936 logits, converted and sampled, 49.8 -> 47.9 us)
 constexpr int64_t kArgmaxPer = 512;
+// and blocks of kArgmaxOne again from here on, whose partials the one block of the second launch reads sooner
+// (500000 fp32 logits, argmax / sampled, 977 against 245 blocks 7.0 / 7.7 -> 6.2 / 6.9 us)
+constexpr int64_t kArgmaxLarge = 1 << 18;
 constexpr int64_t kArgmaxMaxBlocks = 1024;
 
 static int64_t argmax_per(int64_t n)
 {
-    return n <= kArgmaxOne ? kArgmaxOne : std::max(kArgmaxPer, (n + kArgmaxMaxBlocks - 1) / kArgmaxMaxBlocks);
+    return n <= kArgmaxOne || n > kArgmaxLarge ? std::max(kArgmaxOne, (n + kArgmaxMaxBlocks - 1) / kArgmaxMaxBlocks)
+                                               : kArgmaxPer;
 }
 
 int64_t argmax_ws_bytes(int64_t n)
