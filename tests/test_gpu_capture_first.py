@@ -157,15 +157,16 @@ def test_graph_holds_no_workspace(gpu, name):
     assert lib.hipStreamDestroy(first) == 0 and lib.hipStreamDestroy(other) == 0
 
 
-@pytest.mark.parametrize("M,N,K,nodes", [(40, 256, 896, 1), (128, 2048, 1536, 2)])
-def test_split_plan_in_a_graph(gpu, M, N, K, nodes):
-    """A grouped fp16 plan whose k is split, captured on a stream that has the
-    workspace: without it where its problems alone run on k_skinny, with it
-    (GEMM and reduction, the eager bits) where they would split k as well."""
-    print(f"[case] split plan in a graph M={M} N={N} K={K}", flush=True)
+@pytest.mark.parametrize("d,M,N,K,nodes", [(F16, 40, 256, 896, 1), (F16, 128, 2048, 1536, 2), (F32, 64, 1024, 896, 3)])
+def test_split_plan_in_a_graph(gpu, d, M, N, K, nodes):
+    """A grouped plan whose k is split, captured on a stream that has the
+    workspace: without it where its problems alone run on k_skinny (one kernel),
+    with it (the split of fp32 activations, GEMM and reduction, the eager bits)
+    where they would use it as well.  One by one they are twice as many."""
+    print(f"[case] split plan in a graph dtype={d} M={M} N={N} K={K}", flush=True)
     lib = hip()
-    keep, shape, dt, run = linear(np.random.default_rng(M), M, N, K, True, F16)
-    size = int(np.prod(shape)) * 2
+    keep, shape, dt, run = linear(np.random.default_rng(M), M, N, K, True, d)
+    size = int(np.prod(shape)) * np.dtype(dt).itemsize
     want, got = capi.DevBuf(size), capi.DevBuf(size)
     stream, graph, ex = V(), V(), V()
     assert lib.hipStreamCreate(ctypes.byref(stream)) == 0
@@ -186,7 +187,7 @@ def test_split_plan_in_a_graph(gpu, M, N, K, nodes):
         assert lib.hipGraphLaunch(ex, stream) == 0
         capi.sync()
         y = got.to_array(dt, shape)
-        if nodes == 2:
+        if nodes > 1:
             assert np.array_equal(y, ref)
         assert np.linalg.norm(y.astype(np.float64) - ref) <= 2.0 ** -10 * np.linalg.norm(ref.astype(np.float64))
     assert lib.hipGraphExecDestroy(ex) == 0 and lib.hipGraphDestroy(graph) == 0
@@ -216,3 +217,44 @@ def test_eager_call_next_to_a_global_capture(gpu, name):
     assert np.array_equal(got.to_array(dt, shape), want.to_array(dt, shape))
     assert lib.hipGraphDestroy(graph) == 0
     assert lib.hipStreamDestroy(captured) == 0 and lib.hipStreamDestroy(eager) == 0
+
+
+def test_decode_attention_in_a_smaller_workspace(gpu):
+    """One query over 64 chunks of 64 keys takes a block per chunk, 2.2 MB of
+    partials; captured on a stream whose workspace is the smallest (1 MiB), four
+    chunks per block.  Against 64 bits: the output's rounding, scores summed in
+    fp32 and weights of 11 bits or more."""
+    lib = hip()
+    H, KVH, D, n = 64, 4, 128, 4096
+    rng = np.random.default_rng(4)
+    q, k, v = (rng.normal(0, 1, s).astype(np.float16) for s in ((H, D), (n, KVH, D), (n, KVH, D)))
+    dq, dk, dv = (capi.DevBuf.from_array(a) for a in (q, k, v))
+    outs = [capi.DevBuf(H * D * 2) for _ in range(2)]
+    x = capi.DevBuf.from_array(rng.normal(0, 1, 5000).astype(np.float32))
+    i = capi.DevBuf(4)
+    stream, graph, ex = V(), V(), V()
+    run = lambda o, s: capi.call("vvh_attention", o.ptr, dq.ptr, dk.ptr, dv.ptr, 1, n, H, KVH, D, float(1 / np.sqrt(D)), F16, s)
+    run(outs[0], None)
+    assert lib.hipStreamCreate(ctypes.byref(stream)) == 0
+    capi.call("vvh_argmax", x.ptr, 5000, i.ptr, stream)  # a workspace of the smallest size
+    capi.sync()
+    assert lib.hipStreamBeginCapture(stream, 1) == 0
+    run(outs[1], stream)
+    assert lib.hipStreamEndCapture(stream, ctypes.byref(graph)) == 0
+    assert lib.hipGraphInstantiate(ctypes.byref(ex), graph, None, None, 0) == 0
+    ref = np.empty((H, D))
+    for h in range(H):
+        kh, vh = k[:, h // (H // KVH)].astype(np.float64), v[:, h // (H // KVH)].astype(np.float64)
+        s = kh @ q[h].astype(np.float64) / np.sqrt(D)
+        p = np.exp(s - s.max())
+        ref[h] = p / p.sum() @ vh
+    for _ in range(3):
+        capi.call("vvh_memcpy_h2d", outs[1].ptr, np.zeros((H, D), np.float16).ctypes.data, H * D * 2)
+        assert lib.hipGraphLaunch(ex, stream) == 0
+        capi.sync()
+        for o in outs:
+            got = o.to_array(np.float16, (H, D)).astype(np.float64)
+            assert np.linalg.norm(got - ref) <= 2.0 ** -10 * np.linalg.norm(ref)
+    assert not np.array_equal(*(o.to_array(np.float16, (H, D)) for o in outs))  # the two plans round apart
+    assert lib.hipGraphExecDestroy(ex) == 0 and lib.hipGraphDestroy(graph) == 0
+    assert lib.hipStreamDestroy(stream) == 0
