@@ -323,7 +323,11 @@ VVH_API int vvh_plan_create(const vvh_q8_problem* problems, size_t count, int ac
                             int out_dtype, vvh_plan* plan);
 VVH_API int vvh_plan_run(vvh_plan plan, void* stream);
 VVH_API int vvh_plan_destroy(vvh_plan plan);
-/* Number of kernel launches one vvh_plan_run makes. */
+/* Number of linear launches one vvh_plan_run makes: 1 for a plan that runs as
+ * one, else one per problem.  The split of fp32 activations before a GEMM and
+ * the reduction after one of split k are not counted, and a plan made with the
+ * automatic choice runs problem by problem while vvh_set_kernel_override forces
+ * a family, as one of fp32 activations on the GEMM does without a workspace. */
 VVH_API int vvh_plan_launches(vvh_plan plan, int* launches);
 /* Gives every problem of a plan the input stage in_op (VVH_IN_*, with
  * in_w / in_eps as for vvh_linear_q8_dev_in): e.g. q/k/v reading the
@@ -383,8 +387,8 @@ VVH_API int vvh_plan_set_glu(vvh_plan plan, size_t index);
 /* vvh_plan_run with the position of activation row 0 for a RoPE epilogue. */
 VVH_API int vvh_plan_run_pos(vvh_plan plan, size_t pos, void* stream);
 /* Kernel family of a single-launch plan (VVH_KERNEL_DOT, VVH_KERNEL_STREAM
- * or VVH_KERNEL_SKINNY), or VVH_KERNEL_AUTO for a plan run as one launch per
- * problem. */
+ * or VVH_KERNEL_SKINNY), or VVH_KERNEL_AUTO for a plan run as one launch of
+ * another family or as one per problem. */
 VVH_API int vvh_plan_kernel(vvh_plan plan, int* kernel);
 
 /* ---- quantizer and data movement ----------------------------------------- */

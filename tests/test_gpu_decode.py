@@ -92,8 +92,8 @@ def test_decode_late_position(gpu, oracle, fused, P):
     """One step at a late position of a filled KV cache, Qwen2.5-0.5B shapes:
     511 as bench.py times it (512 keys: the MFMA decode attention with one
     8-wave block per kv head, 8 chunks of 64 keys) and 700 (11 chunks: the
-    span split over several blocks per kv head, merged in the same launch by
-    the last block to arrive), which the short steps above never reach.  The
+    span split over several blocks per kv head, merged by a second launch),
+    which the short steps above never reach.  The
     cache rows the step reads are copied back from the device, so the CPU
     forward attends to the same context."""
     cfg, max_ctx = qd.QWEN25_05B, 1024

@@ -174,11 +174,10 @@ def test_graph_survives_workspace_growth(gpu, oracle):
 
 
 def test_graph_split_attention(gpu, oracle):
-    """Split decode attention (blocks merged in the same launch through
-    per-kv-head arrival counters) captured into a graph and replayed, with
-    eager split calls on the same stream between the replays: every replay
-    matches the eager outputs bit for bit, so the counters are back at zero
-    after every call, captured or not."""
+    """Split decode attention (partials in the stream's workspace, merged by a
+    second launch) captured into a graph and replayed, with eager split calls
+    on the same stream, and so in the same workspace, between the replays:
+    every replay matches the eager outputs bit for bit."""
     hip = _hip()
     V = ctypes.c_void_p
     hip.hipStreamCreate.argtypes = [ctypes.POINTER(V)]

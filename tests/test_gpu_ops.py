@@ -126,7 +126,7 @@ def test_embedding(gpu, d):
 # n_q = 1 rows with head_dim % 8 == 0, head_dim <= 128 and <= 16 query heads
 # per kv head take a decode kernel: fp16 with head_dim 64 or 128 the
 # matrix-core one (one block of 4 waves up to 256 keys, of 8 waves up to 512,
-# split blocks merged in the same launch beyond: one key, a one-key tail,
+# split blocks merged by a second launch beyond: one key, a one-key tail,
 # 16 heads per kv head, spans of several chunks per wave), everything else
 # the lane kernel (one chunk, two chunks with one key in the second, many
 # chunks, a span beyond the general kernel's limit, blocks of several
@@ -187,8 +187,8 @@ def test_kv_append(gpu, nbytes, off):
 
 def test_attention_split_calls_in_a_row(gpu, oracle):
     """Split decode calls back to back on one stream, with different block
-    counts: each merges its own partials (the per-kv-head arrival counters
-    are back at zero after every call), the outputs match the oracle."""
+    counts: each merges its own partials from the workspace they share, the
+    outputs match the oracle."""
     H, KVH, D = 14, 2, 64
     T = 9000
     rng = np.random.default_rng(11)

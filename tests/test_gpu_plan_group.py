@@ -2,8 +2,8 @@
 on the GEMM (q/k/v, gate and up of a prompt; fp16, and fp32 split into fp16
 halves once), and fp32 decode problems.  Against 64-bit sums, at group sizes
 2-4, column counts that are no multiple of a tile or of 8, row counts at the
-edges of the tiles and of the dispatch, k split or not; and in a captured graph
-replayed between eager runs.
+edges of the tiles and of the dispatch, k split or not.  (Captured and
+replayed: test_gpu_capture_first.py.)
 
 Tolerance per element: one rounding to the output type, the fp32 sums (no
 product passes through more than K / 8 additions of partial sums of at most

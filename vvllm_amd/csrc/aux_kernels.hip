@@ -90,7 +90,7 @@ __global__ __launch_bounds__(256) void k_convert(DT* __restrict__ d, const ST* _
 }
 
 // The same, 8 elements a thread in 16-byte accesses, for 32-byte aligned rows; the
-// block after the whole chunks takes the remainder.
+// thread after the whole chunks takes the remainder.
 template <typename DT, typename ST>
 __global__ __launch_bounds__(256) void k_convert_vec(DT* __restrict__ d, const ST* __restrict__ s, int64_t n)
 {

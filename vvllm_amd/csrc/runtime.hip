@@ -336,12 +336,14 @@ int gemm3_norder(int64_t M, int64_t N, int64_t act_row_halfs, int64_t krange_cod
 // M=512, 10.3 -> 8.0 us), or where the activations are fp32 (their second set
 // of accumulators leaves one 128-row block per CU: 128 x 128 against 64 x 128,
 // M=300 N=17920 K=1536 64.4 -> 55.0 us, M=700 N=K=1536 32.4 -> 24.2, M=1000
-// N=4864 K=896 46 -> 38); else 128 x 192 when it takes fewer rounds of blocks
-// over the CUs than 128 x 128 by a margin that pays for its longer tiles, and at
-// most two, which its two blocks per CU make one (M=2048 N=4864 K=896: 27.6 us,
-// 128 x 128 26.6); else 128 x 128, whose longer ring is ahead from there (128 x
-// 192 against it, M=2048 K=1536: N=8960 68.8 -> 66.8 us, N=17920 132.1 -> 128.0;
-// M=1500 N=12000 K=512 40.0 -> 34.3).
+// N=4864 K=896 46 -> 38; it costs the largest calls, whose sums were not folded
+// before, M=2048 K=1536: N=17920 277 -> 332); else 128 x 192 when it takes fewer rounds
+// of blocks, counted one per CU, than 128 x 128 by a margin that pays for its
+// longer tiles, and at most two rounds; else 128 x 128.  Two blocks share a CU in
+// both, so the count is only a guide: forced, us, 128 x 192 / 128 x 128, and the
+// rule's choice: M=640 N=8960 K=1536 22.3 / 22.4 (192), M=2048 N=4864 K=896 24.2 / 23.2
+// (192), M=1000 15.4 / 14.9 (128), 2 x 4864 columns at M=512 15.6 / 14.5 (192), at M=700 22.8
+// / 16.0 (128), M=2048 N=8960 K=1536 59.3 / 62.5 (128), M=300 N=17920 32.1 / 23.4 (128).
 template <typename Tiles>
 int gemm3_layout(const Tiles& tiles_of, int splits, int split_layout, bool act_f32)
 {
