@@ -474,14 +474,14 @@ def test_fused_step_qwen25_05b_shapes(gpu, head):
     fused_vs_unfused(qd.QWEN25_05B, head, 2, 8)
 
 
-@pytest.mark.parametrize("P", [255, 256, 511, 600])
+@pytest.mark.parametrize("P", [255, 256, 511, 600, 1100])
 def test_fused_step_late_positions(gpu, P):
     """One step at a late position of a filled KV cache, Qwen2.5-0.5B shapes:
     spans of 256 and 512 keys take the attention parts merged in the o
     projection (4 and 8 parts), 257 the 8-part form with a short last chunk,
-    601 vvh_attention (the span over several blocks); the logits equal the
-    unfused step's bit for bit."""
-    cfg, max_ctx = qd.QWEN25_05B, 1024
+    601 vvh_attention (one block) and 1101 too (the span over several blocks);
+    the logits equal the unfused step's bit for bit."""
+    cfg, max_ctx = qd.QWEN25_05B, 1152
     models = [qd.Model(cfg, act=F16, lm_head="int8", max_ctx=max_ctx, seed=13, fused=f) for f in (False, True)]
     try:
         print(f"[case] fused step late position {P}", flush=True)

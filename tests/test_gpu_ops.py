@@ -125,7 +125,8 @@ def test_embedding(gpu, d):
 
 # n_q = 1 rows with head_dim % 8 == 0, head_dim <= 128 and <= 16 query heads
 # per kv head take a decode kernel: fp16 with head_dim 64 or 128 the
-# matrix-core one (one block of 4 waves up to 256 keys, of 8 waves up to 512,
+# matrix-core one (one block of 4 waves up to 256 keys, of 8 waves up to 512, at
+# head_dim 64 up to 1024,
 # split blocks merged by a second launch beyond: one key, a one-key tail,
 # 16 heads per kv head, spans of several chunks per wave), everything else
 # the lane kernel (one chunk, two chunks with one key in the second, many

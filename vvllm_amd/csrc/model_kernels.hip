@@ -1145,7 +1145,13 @@ static int64_t attn_per_block(int64_t len, int64_t KVH, int64_t D)
 
 // The matrix-core kernel takes spans of up to 8 chunks of 64 keys in one
 // block per kv head, one chunk per wave (4 waves up to 4 chunks, else 8), with
-// no cross-block merge.  Longer spans of up to kDecParts chunks take one-wave
+// no cross-block merge, and at head_dim 64 up to 16, two chunks per wave: the
+// merge's launch costs a program that issues the step itself about 3 us of host
+// time (two layers of 14 / 2 heads of 64 at position 800, 47 us against 53 with a
+// merge; the attention alone, graph replay, 520 / 700 / 1000 keys 6.2 / 6.5 / 7.7 us
+// against 6.7 / 6.8 / 6.3).  At head_dim 128 the second chunk costs more (12 / 2 heads,
+// 700 / 1000 keys 10.5 / 13.6 against 7.5 / 7.1), as does a third (14 / 2 of 64, 1500 keys
+// 10.2 against 6.9).  Longer spans of up to kDecParts chunks take one-wave
 // blocks of a chunk each (k_attention_parts) while they fit one round over the
 // CUs (256): 14 / 2 heads of 64, 1023 keys, 6.3 us against 6.6 in 4-wave blocks
 // and 7.8 with those merged by the last to arrive; 12 / 2 heads of 128, 700 keys
@@ -1166,6 +1172,9 @@ AttnDecodePlan attention_decode_plan(const void* q, int64_t len, int64_t H, int6
         if (chunks <= 8) {
             p.waves = chunks <= 4 ? 4 : 8;
             p.per_block = p.waves * kDecChunk;
+        } else if (D == 64 && chunks <= 16 && KVH <= 128) {
+            p.waves = 8;
+            p.per_block = 16 * kDecChunk;
         } else if (!coarse && chunks <= kDecParts && chunks * KVH <= 256) {
             p.waves = 1;
             p.per_block = kDecChunk;

@@ -170,19 +170,20 @@ int workspace_for(void* stream, std::size_t bytes, float** out, bool relaxed = f
 // it is large enough.
 bool workspace_try(void* stream, std::size_t bytes, float** ws, bool captured = false)
 {
+    if (captured) {
+        std::lock_guard<std::mutex> lock(g_wsmu);
+        const auto it = g_ws.find(stream);
+        if (it != g_ws.end() && it->second.bytes >= bytes) {
+            *ws = static_cast<float*>(it->second.p);
+            return true;
+        }
+    }
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(static_cast<hipStream_t>(stream), &st) != hipSuccess) {
         (void)hipGetLastError();
         return false;
     }
-    if (st != hipStreamCaptureStatusNone) {
-        if (!captured) return false;
-        std::lock_guard<std::mutex> lock(g_wsmu);
-        const auto it = g_ws.find(stream);
-        if (it == g_ws.end() || it->second.bytes < bytes) return false;
-        *ws = static_cast<float*>(it->second.p);
-        return true;
-    }
+    if (st != hipStreamCaptureStatusNone) return false;
     return workspace_for(stream, bytes, ws, true) == VVH_OK;
 }
 
@@ -838,14 +839,14 @@ int run_group(const std::vector<LinArgs>& args, int group, int act, int outd, vo
     if (sp > 1 && !mul_ok((uint64_t)M * (uint64_t)n, (uint64_t)sp * 4, &plane)) return VVH_OK;
     float* ws = nullptr;
     const uint64_t bytes = xs + rs + plane;
-    if (bytes > 0 && !workspace_try(stream, bytes, &ws)) {
+    if (bytes > 0 && !workspace_try(stream, bytes, &ws, f32)) {
         auto alone = [&](const LinArgs& a) {
             int l = 4;
             return choose_kernel((std::size_t)a.M, (std::size_t)a.N, (std::size_t)a.K, act, true) == K_GEMM &&
                    gemm_splits(a.M, a.N, stages, &l) > 1;
         };
-        if (!((f32 || std::any_of(args.begin(), args.end(), alone)) && workspace_try(stream, bytes, &ws, true))) {
-            if (f32) return VVH_OK;
+        if (f32) return VVH_OK;
+        if (!(std::any_of(args.begin(), args.end(), alone) && workspace_try(stream, bytes, &ws, true))) {
             sp = 1;
             kst = stages;
         }
@@ -2240,8 +2241,9 @@ VVH_API int vvh_attention_parts(float* parts, size_t parts_floats, size_t* npart
                     "<= 16 and 16-byte aligned q, k, v and parts");
     const AttnDecodePlan p = attention_decode_plan(q, (int64_t)len0, (int64_t)num_heads, (int64_t)num_kv_heads,
                                                    (int64_t)head_dim, dtype, false);
-    if (!p.mfma || p.nb != 1)
-        return fail(VVH_ERR_UNSUPPORTED, "a span of %zu positions is not one block per kv head (at most 512)", len0);
+    if (!p.mfma || p.nb != 1 || (p.waves == 8 && len0 > 512))
+        return fail(VVH_ERR_UNSUPPORTED, "a span of %zu positions is not one block of single chunks per kv head (at most 512)",
+                    len0);
     const std::size_t need = (std::size_t)p.waves * num_heads * (head_dim + 4);
     if (parts_floats < need)
         return fail(VVH_ERR_INVALID_ARG, "parts holds %zu floats, %zu needed", parts_floats, need);
