@@ -393,6 +393,7 @@ struct DensePlan {
 };
 bool dense_mfma_ok(const void* x, const void* w, int wdtype, int64_t M, int64_t N, int64_t K, int dtype);
 DensePlan dense_plan(int64_t M, int64_t N, int64_t K, int dtype, int64_t cus);
+bool dense_split_pays(int64_t M, int64_t N, int64_t K, int dtype);
 bool dense_unsplit_pays(const DensePlan& p, int64_t M, int64_t N, int64_t K, int dtype, int64_t cus);
 int64_t dense_ws_floats(const DensePlan& p, int64_t M, int64_t N);
 int launch_dense_mfma(const DensePlan& p, void* out, const void* x, const void* w, const float* bias, const void* res,

@@ -353,6 +353,20 @@ DensePlan dense_plan(int64_t M, int64_t N, int64_t K, int dtype, int64_t cus)
     return p;
 }
 
+// Whether a call that would split k is worth the reduction's launch, whose host
+// time a program that issues its calls one by one pays too: two launches take it
+// 9.3 to 10.6 us.  Not where the vector form is done before (issued in a row, us,
+// vector / split: fp16 8 / 10 x 1536 x 1536 8.1 / 10.2 against 9.4 / 11.4, 10 x 256 x 1536
+// 9.4 against 11.1, 7 x 3000 x 2048 9.1 against 10.7; fp32 16 x 512 x 512 8.0 against 9.3,
+// 12 x 896 x 896 8.0 against 9.3, 10 x 1536 x 1536 9.5 against 11.0): its time fitted to
+// these, passes of 4 rows over the weights and the products of a row and a value.
+bool dense_split_pays(int64_t M, int64_t N, int64_t K, int dtype)
+{
+    const double pass = 0.8 + 0.45 * std::max(0.0, (double)(N - 2000) / 1000.0), mk = (double)M * (double)K;
+    const double us = (double)((M + 3) / 4) * pass + (dtype == VVH_F32 ? 2.4 + 2.7e-4 * mk : 3.5 + 2.1e-4 * mk);
+    return us > 9.6;
+}
+
 // Whether a call that would split k and has no workspace for the planes takes a
 // tile's whole k in one block, or the vector form: its passes over the weights
 // (2.5 us and 0.42 ns per row and value, on 2200 weight rows and more in

@@ -2272,9 +2272,12 @@ VVH_API int vvh_dense(void* out, const void* x, const void* dev_weight, int wdty
         // one block takes all of a tile's k
         float* ws = nullptr;
         const int64_t wsf = dense_ws_floats(p, (int64_t)M, (int64_t)N);
-        const bool lacks = wsf > 0 && !workspace_try(stream, (std::size_t)wsf * 4, &ws);
-        if (lacks) p.splits = 1;
-        if (!lacks || dense_unsplit_pays(p, (int64_t)M, (int64_t)N, (int64_t)K, dtype, cus))
+        bool mfma = wsf == 0 || dense_split_pays((int64_t)M, (int64_t)N, (int64_t)K, dtype);
+        if (mfma && wsf > 0 && !workspace_try(stream, (std::size_t)wsf * 4, &ws)) {
+            p.splits = 1;
+            mfma = dense_unsplit_pays(p, (int64_t)M, (int64_t)N, (int64_t)K, dtype, cus);
+        }
+        if (mfma)
             return ret_launch(launch_dense_mfma(p, out, x, dev_weight, dev_bias, residual, (int64_t)M, (int64_t)N,
                                                 (int64_t)K, dtype, ws, stream),
                               "dense launch");
