@@ -295,8 +295,9 @@ VVH_API int vvh_linear_q8_dev_in(void* out, const void* inp, const int8_t* dev_w
 
 /* ---- grouped launch ------------------------------------------------------ */
 /* A plan is a fixed list of independent linear_q8 problems of one
- * (act_dtype, out_dtype) pair, resolved once (kernel choice, tile
- * decomposition, device-resident descriptor table) and launched with
+ * (act_dtype, out_dtype) pair, resolved once (kernel choice, descriptor
+ * table, for the decode path the tile decomposition too; a GEMM's tiles and
+ * splits are chosen at each run, for its workspace) and launched with
  * vvh_plan_run as a single kernel when every problem takes the decode path
  * (M <= 16), or when its problems read the same activations and take the
  * GEMM (not from fp16 to fp32), or are fp32 of few rows (a GEMM of fp32
