@@ -32,7 +32,9 @@ def reference(x, w, b, r):
 
 
 CASES = [(5, 64, 8), (9, 64, 8), (6, 70, 2052 * 4), (31, 63, 64), (32, 65, 72), (33, 130, 896), (64, 896, 4864), (65, 200, 2056), (128, 128, 32),
-         (129, 1000, 1000), (5, 512, 512), (7, 1100, 896), (10, 1024, 1024), (300, 9728, 136), (512, 8200, 896), (7, 40, 4864), (100, 33, 8960)]
+         (129, 1000, 1000), (5, 512, 512), (7, 1100, 896), (10, 1024, 1024), (300, 9728, 136), (512, 8200, 896), (7, 40, 4864), (100, 33, 8960),
+         # both sides of the lines where a k split gives way to a wave per weight row (its longest chain, K / 64 + 6, is shorter here)
+         (9, 130, 1968), (9, 130, 1984), (8, 100, 2672), (8, 100, 2688), (16, 70, 856), (16, 70, 872), (12, 2100, 640), (5, 4000, 1536)]
 
 
 @pytest.mark.parametrize("d", [F32, F16])
